@@ -156,24 +156,59 @@ __global__ __launch_bounds__(BLOCK) void k_cdff_tiles(const VehDesc* __restrict_
         tile_sum[blockIdx.x] = (double)tot;
 }
 
-// One thread per vehicle: sequential prefix over the vehicle's tile totals.
+// One workgroup per vehicle: sequential prefix over the vehicle's tile totals (the association of the float
+// modes).  The additions are one dependent chain, so one thread does them; the others stage
+// the totals in LDS and write the prefixes out, so that the chain waits for LDS reads issued ahead
+// of it and not for one memory round trip per tile.  8600 tiles (2048^2 cells, 8e6 + 8e5 weights): FP64 692 us
+// with every load and store in the chain, 124 us staged.
 template <class T>
-__global__ void k_cdff_top(const VehDesc* __restrict__ descs, int m, const double* __restrict__ tile_sum,
-                           double* __restrict__ tile_pre)
+__global__ __launch_bounds__(BLOCK) void k_cdff_top(const VehDesc* __restrict__ descs,
+                                                    const double* __restrict__ tile_sum, double* __restrict__ tile_pre)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= m)
-        return;
-    const VehDesc& d = descs[v];
+    constexpr int CHUNK = 2048;  // totals staged at once
+    constexpr int STEP = 16;     // totals read ahead of the chain
+    __shared__ double s_x[CHUNK];
+    const VehDesc& d = descs[blockIdx.x];
     if (d.cdf_mode != CdfFloatMode<T>::mode)
         return;
     const int t0 = d.u0[SP_J] / SCAN_Q;
     const int nt = d.nu[SP_J] / SCAN_Q;
     T run = (T)0;
-    for (int t = 0; t < nt; ++t)
+    for (int c = 0; c < nt; c += CHUNK)
     {
-        tile_pre[t0 + t] = (double)run;
-        run = run + (T)tile_sum[t0 + t];
+        const int len = min(CHUNK, nt - c);
+        __syncthreads();
+        for (int i = threadIdx.x; i < CHUNK; i += BLOCK)
+            s_x[i] = i < len ? tile_sum[t0 + c + i] : 0.0;
+        __syncthreads();
+        if (threadIdx.x == 0)
+        {
+            double x[STEP];
+#pragma unroll
+            for (int k = 0; k < STEP; ++k)
+                x[k] = s_x[k];
+            for (int i = 0; i < len; i += STEP)  // past len: zeros, whose prefixes are not written out
+            {
+                double next[STEP];
+                const int n0 = min(i + STEP, CHUNK - STEP);
+#pragma unroll
+                for (int k = 0; k < STEP; ++k)
+                    next[k] = s_x[n0 + k];
+#pragma unroll
+                for (int k = 0; k < STEP; ++k)
+                {
+                    const T before = run;
+                    run = run + (T)x[k];
+                    s_x[i + k] = (double)before;
+                }
+#pragma unroll
+                for (int k = 0; k < STEP; ++k)
+                    x[k] = next[k];
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < len; i += BLOCK)
+            tile_pre[t0 + c + i] = s_x[i];
     }
 }
 
@@ -235,31 +270,64 @@ __global__ __launch_bounds__(BLOCK) void k_cdff_apply(const VehDesc* __restrict_
         env[ENV_STRIDE * (size_t)blockIdx.x] = (double)tmax;
 }
 
-// One thread per vehicle: the envelope across tiles, the total and the new particle weight.
-__global__ void k_cdff_env(const VehDesc* __restrict__ descs, int m, double* __restrict__ env,
-                           DevScalars* __restrict__ scs)
+// One workgroup per vehicle: the envelope across tiles, the total and the new particle weight.  The
+// running maximum is exact in any order, so each thread takes a contiguous run of tiles and a block scan
+// joins them (a tile maximum that is not above 0, NaN among them, leaves the envelope unchanged).
+// 8600 tiles: 20 us, against 1628 us for one thread walking the tiles.
+constexpr int ENV_BLOCK = 1024;
+
+__global__ __launch_bounds__(ENV_BLOCK) void k_cdff_env(const VehDesc* __restrict__ descs, double* __restrict__ env,
+                                                        DevScalars* __restrict__ scs)
 {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= m)
-        return;
+    __shared__ double s_m[ENV_BLOCK / WAVE];
+    const int v = blockIdx.x;
     const VehDesc& d = descs[v];
     if (d.cdf_mode == CDF_EXACT)
         return;
     const int t0 = d.u0[SP_J] / SCAN_Q;
     const int nt = d.nu[SP_J] / SCAN_Q;
-    double run = 0.0;
-    for (int t = 0; t < nt; ++t)
+    const int per = (nt + ENV_BLOCK - 1) / ENV_BLOCK;
+    const int b0 = min(nt, (int)threadIdx.x * per), b1 = min(nt, b0 + per);
+    double mx = 0.0;
+#pragma unroll 4
+    for (int t = b0; t < b1; ++t)
     {
         const double tm = env[ENV_STRIDE * (size_t)(t0 + t)];
-        env[ENV_STRIDE * (size_t)(t0 + t) + 1] = run;
-        run = tm > run ? tm : run;
-        env[ENV_STRIDE * (size_t)(t0 + t)] = run;
+        mx = tm > mx ? tm : mx;
     }
-    DevScalars* sc = scs + v;
-    sc->ftotal = run;
-    const float jm = (float)run;
-    sc->joint_max = jm;
-    sc->new_weight = jm / (float)d.N;
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+    const double wmax = wave_inclusive_max_val(mx);
+    double run = shfl_up1(wmax);
+    if (lane == 0)
+        run = 0.0;
+    if (lane == WAVE - 1)
+        s_m[wid] = wmax;
+    __syncthreads();
+    double total = 0.0;
+#pragma unroll
+    for (int w = 0; w < ENV_BLOCK / WAVE; ++w)
+    {
+        const double x = s_m[w];
+        if (w < wid)
+            run = x > run ? x : run;
+        total = x > total ? x : total;
+    }
+    for (int t = b0; t < b1; ++t)
+    {
+        double* e = env + ENV_STRIDE * (size_t)(t0 + t);
+        const double tm = e[0];
+        e[1] = run;
+        run = tm > run ? tm : run;
+        e[0] = run;
+    }
+    if (threadIdx.x == 0)
+    {
+        DevScalars* sc = scs + v;
+        sc->ftotal = total;
+        const float jm = (float)total;
+        sc->joint_max = jm;
+        sc->new_weight = jm / (float)d.N;
+    }
 }
 
 // Ancestor search over the float modes' envelope (doubles): the draw, the coarse index entry of a
@@ -799,12 +867,11 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
     double* tsum = reinterpret_cast<double*>(E->scan_tile_sum);
     double* tpre = reinterpret_cast<double*>(E->exp_tile_sum);
     double* env = reinterpret_cast<double*>(E->cdf_tile_incl);
-    const int vb = div_up(E->m, 64);
     auto float_mode = [&](auto tag) {
         using T = decltype(tag);
         launch_begin(E, K_CDF_WRITE);
         hipLaunchKernelGGL(k_cdff_tiles<T>, dim3(jtiles), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_J), tsum);
-        hipLaunchKernelGGL(k_cdff_top<T>, dim3(vb), dim3(64), 0, E->stream, E->d_desc, E->m, tsum, tpre);
+        hipLaunchKernelGGL(k_cdff_top<T>, dim3(E->m), dim3(BLOCK), 0, E->stream, E->d_desc, tsum, tpre);
         hipLaunchKernelGGL(k_cdff_apply<T>, dim3(jtiles), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_J), tpre,
                            env);
         launch_end(E, K_CDF_WRITE);
@@ -816,7 +883,7 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
     if (modes & (1 << CDF_FP32C))
         float_mode(f32c(0));
     if (modes & ~(1 << CDF_EXACT))
-        hipLaunchKernelGGL(k_cdff_env, dim3(vb), dim3(64), 0, E->stream, E->d_desc, E->m, env, E->scalars);
+        hipLaunchKernelGGL(k_cdff_env, dim3(E->m), dim3(ENV_BLOCK), 0, E->stream, E->d_desc, env, E->scalars);
 
     const int mt = E->tiles(SP_P, RS_TILE / UNIT);
     const bool wide = E->tune.merge_slice == 0 ? mt <= RS_WIDE_MAX_TILES : E->tune.merge_slice == 2;

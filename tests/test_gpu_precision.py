@@ -7,7 +7,7 @@ import pytest
 
 from dogm_ctypes import DOGM, Batch
 from oracle_ctypes import OracleDOGM
-from parity_util import (assert_grid_equal, assert_int_equal, assert_particles_equal, assert_state_equal,
+from parity_util import (assert_bits_equal, assert_grid_equal, assert_int_equal, assert_particles_equal, assert_state_equal,
                          small_params, small_scene)
 
 pytestmark = pytest.mark.gpu
@@ -137,3 +137,28 @@ def test_batch_mixes_draw_modes():
                 assert_particles_equal(f"frame {f} vehicle {k}", batch.get_particles(ids[k]), g.get_particles())
                 assert_int_equal(f"frame {f} vehicle {k} ancestors", batch.get_resampled_indices(ids[k]),
                                  g.get_resampled_indices())
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fp32", "fp32c"])
+@pytest.mark.parametrize("joint", [1, 1024, 2048 * 1024, 2048 * 1024 + 1])
+def test_float_modes_tile_prefix_edges(mode, joint):
+    """The tile prefix and envelope at one tile, at exactly the 2048 tile totals staged at once and past them."""
+    b = min(joint - 1, 1000)
+    n = joint - b
+    p = small_params(gs=16, res=0.5, n=n, b=b)
+    sc = small_scene(gs=16, res=0.5)
+    rng = np.random.default_rng(joint)
+    w = (10.0 ** (-9.0 * rng.random(n))).astype(np.float32)
+    w[:: 7] = 0.0
+    with DOGM(p, seed=SEED) as gpu:
+        orc = OracleDOGM(p, seed=SEED)
+        for o in (gpu, orc):
+            o.set_cdf_mode(mode)
+            o.update_measurement_grid(sc.measurement(0))
+            o.set_weight_array(w)
+            if b:
+                o.set_birth_particles(weight=np.full(b, 1e-4, np.float32))
+            o.resampling()
+        assert_int_equal(f"{mode} {joint}", gpu.get_resampled_indices(), orc.get_resampled_indices())
+        assert_bits_equal(f"{mode} {joint} weight", gpu.get_particles()["weight"], orc.get_particles()["weight"])
+        orc.close()
