@@ -168,13 +168,18 @@ __device__ __forceinline__ void stream_store(dogm_measurement_cell* p, dogm_meas
 // Predicted weight of a particle (dogm/src/kernel/predict.cu:34-43): persistence probability times
 // the prior weight, 0 once the predicted position o leaves the grid.  predict and the gathering sort
 // pass (uniform weights) both form it here, so the two give the same bits.
-__device__ __forceinline__ float predicted_weight(const VehDesc& d, float w_in, const float4& o)
+__device__ __forceinline__ bool outside_grid(const VehDesc& d, const float4& o)
 {
     const float zero = 0.0f;
     const float top = (float)(d.gs - 1);
+    return (o.x > top || o.x < zero) || (o.y > top || o.y < zero);
+}
+
+__device__ __forceinline__ float predicted_weight(const VehDesc& d, float w_in, const float4& o)
+{
     float w = d.ps * w_in;
-    if ((o.x > top || o.x < zero) || (o.y > top || o.y < zero))
-        w = zero;
+    if (outside_grid(d, o))
+        w = 0.0f;
     return w;
 }
 
@@ -341,18 +346,30 @@ __device__ __forceinline__ void wave_count(unsigned* s_h, unsigned d, bool valid
     }
 }
 
-// Sort values: the particle index (< 2^31) with its association flag in bit 31.
+// Cell indices and particle indices are below 2^28 (grid sides up to 16383, MAX_SPACE_LEN), so the words
+// that travel with a particle carry its flags in their top bits: the association (bit 31) and, for
+// vehicles with per-cell weights, that the predicted position left the grid (bit 30).  Inside a full step
+// predict leaves (cell | flags), the sort's values are (particle | flags), and the sorted cell indices
+// keep the out-of-grid flag until the moments.
+constexpr unsigned WORD_ASSOC = 0x80000000u;
+constexpr unsigned WORD_OUT = 0x40000000u;
+constexpr unsigned WORD_FLAGS = WORD_ASSOC | WORD_OUT;
+
+__device__ __forceinline__ int word_index(int w)
+{
+    return (int)((unsigned)w & ~WORD_FLAGS);
+}
+__device__ __forceinline__ bool word_out(int w)
+{
+    return ((unsigned)w & WORD_OUT) != 0u;
+}
+__device__ __forceinline__ uint8_t word_assoc(int w)
+{
+    return (uint8_t)((unsigned)w >> 31);
+}
 __device__ __forceinline__ int sort_value(int p, uint8_t assoc)
 {
-    return (int)((unsigned)p | (assoc ? 0x80000000u : 0u));
-}
-__device__ __forceinline__ int sort_value_index(int v)
-{
-    return (int)((unsigned)v & 0x7fffffffu);
-}
-__device__ __forceinline__ uint8_t sort_value_assoc(int v)
-{
-    return (uint8_t)((unsigned)v >> 31);
+    return (int)((unsigned)p | (assoc ? WORD_ASSOC : 0u));
 }
 
 // Radix-sort tiles: SORT_ITEMS keys per thread, SORT_Q units per tile (the engine sizes the
@@ -435,9 +452,10 @@ void k_segreduce(Op op, const VehDesc* __restrict__ descs,
     const VehDesc& d = descs[tr.v];
     const int n = d.N;
     const int tbase = tr.base;
-    if (tbase >= n)
+    if (tbase >= n || d.wcell)
     {
-        // Padding tile past the vehicle's particles: no segment, no carry.
+        // Padding tile past the vehicle's particles, or a vehicle with per-cell weights: no segment, no
+        // carry.
         if (threadIdx.x == 0)
             carry.flags[tile] = 0;
         return;

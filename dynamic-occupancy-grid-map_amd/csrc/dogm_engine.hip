@@ -22,7 +22,7 @@ const char* const kKernelNames[K_COUNT] = {
     "seg_moments_fix", "cdf_write",      "exp_tiles",       "rs_merge",        "fill",            "pack_grid",
     "unpack_grid",    "build_tables",    "extract_mark",    "extract_scan",    "extract_compact",
     "extract_gather", "ego_particles",   "ego_field",       "pack_state",      "unpack_state",
-    "materialize",
+    "materialize",    "cell_bounds",
 };
 
 // ---- timing ------------------------------------------------------------------------------------
@@ -541,6 +541,9 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         uint32_t e = v->epoch;
         d.init = (stages & ST_INIT) && v->init_pending ? 1 : 0;
         d.wuni = v->w_uniform || d.init ? 1 : 0;  // initialisation sets every weight to 1 / N
+        // In a full update from uniform weights every in-grid particle carries the same predicted weight
+        // and every other one 0, so the per-cell sums need counts only.
+        d.wcell = d.wuni && (stages & ST_ALL) == ST_ALL ? 1 : 0;
         d.rs_gather = v->rs_pending && !d.init && full_predict ? 1 : 0;
         d.rs_defer = (stages & ST_RESAMPLE) ? 1 : 0;
         d.ep_init = e;
@@ -603,6 +606,9 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         d.nz = v->nz;
         d.nz_valid = v->nz_valid ? 1 : 0;
     }
+    E->any_wcell = E->any_general = false;
+    for (int i = 0; i < m; ++i)
+        (E->h_desc[i].wcell ? E->any_wcell : E->any_general) = true;
     // Table offsets per vehicle (units); the prefixes are those the tables were built from.
     {
         long long off[SP_COUNT] = {};
@@ -696,6 +702,7 @@ int engine_run(Engine* E, Vehicle* const* veh, int m, int stages)
     std::memcpy(&occ_bits, &E->ext.min_occ, 4);
     std::memcpy(&vel_bits, &E->ext.min_vel, 4);
     const uint64_t sig[3] = {(uint64_t)stages | ((uint64_t)any_init << 16) | ((uint64_t)modes << 17) |
+                                 ((uint64_t)E->any_wcell << 21) | ((uint64_t)E->any_general << 22) |
                                  ((uint64_t)(stages & ST_EXTRACT ? E->ext.what : 0) << 24) |
                                  ((uint64_t)(stages & ST_EXTRACT ? E->ext.source : 0) << 32),
                              (stages & ST_EXTRACT) ? ((uint64_t)occ_bits << 32 | vel_bits) : 0,

@@ -114,6 +114,7 @@ struct VehDesc
     float dt;
     int init;                // first measurement: particles are initialised in this step
     int wuni;                // every weight predict reads equals weight[0] (resampled or initialised)
+    int wcell;               // full step from uniform weights: a cell's particles share one weight (cell_weights)
     int rs_gather;           // part[0] is a deferred resampled set: predict reads it through ancestors
     int rs_defer;            // the resampling writes ancestors and weight[0] only (a deferred set)
     int move;                // pending particle shift (fused into predict)
@@ -229,6 +230,7 @@ enum KernelId
     K_PACK_STATE,
     K_UNPACK_STATE,
     K_MATERIALIZE,
+    K_CELL_BOUNDS,
     K_COUNT
 };
 
@@ -468,6 +470,9 @@ struct Engine
         long long sort_tiles_cap;
     } own{};
     bool bound = false;
+
+    // Vehicles of the current step that run with / without per-cell weights (VehDesc::wcell).
+    bool any_wcell = false, any_general = true;
 
     std::string last_error;
 

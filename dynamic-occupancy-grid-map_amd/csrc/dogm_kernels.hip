@@ -1,6 +1,6 @@
 // Stage kernels of the DOGM particle-filter update on gfx950.
 //
-// Layout in HBM, per vehicle: particles structure-of-arrays (float4 state, int cell index, float
+// Layout in HBM, per vehicle: particles structure-of-arrays (position, velocity, int cell index, float
 // weight, uint8 association), grid cells structure-of-arrays (one array per field), measurement
 // cells as given by the caller (16-byte AoS).  Every per-cell sum is an exact 128-bit fixed-point
 // segmented reduction over the cell-sorted particles (dogm_device.h).  Step kernels find their
@@ -221,7 +221,22 @@ __device__ __forceinline__ int clamp_cell(float x, int gs)
 // upsweep.  With aos (the sort's gathering pass follows in the same step) the new state goes to the
 // vehicle's CDF buffer, free until the resampling, as 16-byte (x, y, vx, vy) records, so that the
 // gather reads one 16-byte record per particle at random instead of two 8-byte ones from two arrays;
-// nothing else reads the positions or velocities in between.
+// nothing else reads the positions or velocities in between.  The cell indices then carry the particles'
+// flags (WORD_FLAGS), so the sort's first pass reads one word per particle and no association byte.
+// Border cells: the cells whose coordinate predict clamps to, so the only ones that can hold out-of-grid
+// particles (weight 0) beside in-grid ones.  For vehicles with per-cell weights their out-of-grid particles
+// are counted in m_raw (as ints), which such vehicles do not use otherwise: zeroed beside predict, counted
+// by k_cell_bounds, read by the occupancy update.
+__device__ __forceinline__ bool border_cell(int c, int gs)
+{
+    const int y = c / gs, x = c - y * gs;
+    return x == 0 || y == 0 || x == gs - 1 || y == gs - 1;
+}
+__device__ __forceinline__ int* border_out(const VehDesc& d)
+{
+    return reinterpret_cast<int*>(d.m_raw);
+}
+
 // start = end = -1 for the cells of work-table group `group` (THREADS x 4 cells), four cells per
 // thread with 16-byte stores.  With valid occupancy bits only groups of four containing a cell that
 // had particles are written (the others still hold -1, and rewriting -1 is harmless).
@@ -234,6 +249,15 @@ __device__ __forceinline__ void reset_bounds_cells(const VehDesc* __restrict__ d
     const int c = tr.base + 4 * threadIdx.x;
     if (c >= d.C)
         return;
+    if (d.wcell)
+    {
+        const int last = min(c + 3, d.C - 1);
+        const int y = c / d.gs, x = c - y * d.gs;
+        // a border cell among the four (a group that wraps into the next row holds one)
+        if (y == 0 || x == 0 || x + 3 >= d.gs - 1 || last >= d.C - d.gs)
+            for (int k = c; k <= last; ++k)
+                border_out(d)[k] = 0;
+    }
     if (d.nz_valid && ((d.nz[c >> 6] >> (c & 63)) & 0xfull) == 0)
         return;
     if (c + 4 <= d.C)
@@ -300,22 +324,24 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
         if (valid)
         {
             float2 ps, vs;
+            uint8_t assoc = 0;
             if (d.rs_gather)
             {
-                // A deferred resampled set (see merge_write): the state of the particle's ancestor
-                // (part[pph ^ 1] below N, the birth set above), and its association flag written here
-                // for the sort.
+                // A deferred resampled set (see merge_write): the state and association of the
+                // particle's ancestor (part[pph ^ 1] below N, the birth set above).
                 const int a = d.ancestors[i];
                 const bool from_p = a < n;
                 const int o = from_p ? a : a - n;
                 ps = (from_p ? Q.pos : Bq.pos)[o];
                 vs = (from_p ? Q.vel : Bq.vel)[o];
-                P.assoc[i] = (from_p ? Q.assoc : Bq.assoc)[o];
+                assoc = (from_p ? Q.assoc : Bq.assoc)[o];
             }
             else
             {
                 ps = P.pos[i];
                 vs = P.vel[i];
+                if (aos)
+                    assoc = P.assoc[i];
             }
             float4 s = make_float4(ps.x, ps.y, vs.x, vs.y);
             // The gathering pass forms the weight (always so for a deferred set: the host reads one
@@ -350,9 +376,12 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
             o.w = svy + nvy;
             const float w = predicted_weight(d, w_in, o);
             cell = clamp_cell(o.x, gs) + gs * clamp_cell(o.y, gs);
+            int word = cell;
             if (aos)
             {
                 stream_store(reinterpret_cast<float4*>(d.cdf) + i, o);
+                word = (int)((unsigned)cell | (assoc ? WORD_ASSOC : 0u) |
+                             (d.wcell && outside_grid(d, o) ? WORD_OUT : 0u));
             }
             else
             {
@@ -361,7 +390,7 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
             }
             if (!keep_w)
                 P.weight[i] = w;
-            stream_store(&P.idx[i], cell);
+            stream_store(&P.idx[i], word);
         }
         for (int ps = 0; ps < passes; ++ps)
             wave_count(s_h[ps], ((unsigned)cell >> (ps * RADIX_BITS)) & (RADIX - 1), valid);
@@ -428,13 +457,13 @@ __global__ __launch_bounds__(BLOCK) void k_sort_gather(const VehDesc* __restrict
     const DevParticles dst = d.part[pph ^ 1];
     const int* skeys = d.sort_keys[fin];
     const int sv = d.sort_vals[fin][k];
-    const int o = sort_value_index(sv);
+    const int o = word_index(sv);
     const int key = skeys[k];
     const float w = src.weight[o];
     dst.pos[k] = src.pos[o];
     dst.vel[k] = src.vel[o];
     dst.weight[k] = w;
-    dst.assoc[k] = sort_value_assoc(sv);
+    dst.assoc[k] = word_assoc(sv);
     dst.idx[k] = key;
     d.weight_array[k] = w;
     if (k == 0 || skeys[k - 1] != key)
@@ -509,9 +538,17 @@ struct OccOp
 // Cells whose particles cross reduction tiles get their weight sum here from the reduction's tile
 // partials (the first tile's tail, whole middle tiles, the last tile's head), as the fix-up pass
 // would, and m_raw is written for them.
+//
+// Vehicles with per-cell weights (VehDesc::wcell): every in-grid particle of a cell has the weight
+// w = persistence * prior and the out-of-grid ones (border cells only) weight 0, so the exact sums over a
+// cell's particles are its counts times one fixed-point value (integer products: the same 128-bit sums, wrap
+// included, as adding the particles one by one), and everything the persistent update derives from them
+// is formed here, one thread per cell.  cellrec then holds the two posterior weights of the cell's particles
+// (in-grid, out-of-grid) and rho_p for the moments.  No per-particle reduction is left: the two segmented
+// reductions and their fix-up took @SEG@.
 // One cell; returns its born mass rho_b.
 __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int zero_empty, const SegCarry& carry,
-                                                  int occ_tile)
+                                                  int occ_tile, int pph)
 {
     const int gs = d.gs;
     const float* free_src = d.free[0];
@@ -528,7 +565,16 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
         if ((c & 63) == 0)
             d.nz[c >> 6] = now;
     }
-    if (occupied)
+    float w_in = 0.0f;  // per-cell weights: the in-grid particles' predicted weight, and the counts
+    int n_in = 0, n_out = 0;
+    if (occupied && d.wcell)
+    {
+        w_in = d.ps * d.part[pph ^ 1].weight[0];
+        n_out = border_cell(c, gs) ? border_out(d)[c] : 0;
+        n_in = d.end[c] - d.start[c] + 1 - n_out;
+        m_occ_pred = fx_to_f32(fx_from_f32(w_in) * n_in);
+    }
+    else if (occupied)
     {
         const int OT = occ_tile;  // particles per reduction tile
         m_occ_pred = d.m_raw[c];
@@ -579,7 +625,7 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
     const dogm_measurement_cell mc = d.meas_in ? d.meas_in[c] : d.meas[c];
     if (d.meas_in)
         stream_store(&d.meas[c], mc);
-    if ((zero_empty & 1) && occupied)
+    if ((zero_empty & 1) && occupied && !d.wcell)
         stream_store(&d.cellin[c], make_float2(mc.likelihood, m_raw_c));
     const float pB = d.pB;
     const float m_free_pred = fminf(d.alpha * fprev, one - m_occ_pred);
@@ -592,6 +638,24 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
         (m_free_pred * meas_unknown + unknown_pred * mc.free_mass + m_free_pred * mc.free_mass) / (one - K);
     const float rho_b = (occ_up * pB * (one - m_occ_pred)) / (m_occ_pred + pB * (one - m_occ_pred));
     const float rho_p = occ_up - rho_b;
+    if (occupied && d.wcell)
+    {
+        // mass_update.cu:51-59 (weights of overfull cells), update_persistent_particles.cu:16-87.
+        const bool over = m_raw_c > one;
+        const float wi = over ? w_in / m_raw_c : w_in;
+        const float wo = over ? 0.0f / m_raw_c : 0.0f;
+        const float lwi = mc.likelihood * wi, lwo = mc.likelihood * wo;
+        fx_t sum = fx_from_f32(lwi) * n_in;
+        if (n_out)
+            sum += fx_from_f32(lwo) * n_out;
+        const float acc = fx_to_f32(sum);
+        const float mu_A = acc > 0.0f ? rho_p / acc : 0.0f;
+        const float mu_UA = m_occ_pred > 0.0f ? rho_p / m_occ_pred : 0.0f;
+        const float a = mc.p_A * mu_A, b = (one - mc.p_A) * mu_UA;
+        d.f[GF_MU_A][c] = mu_A;
+        d.f[GF_MU_UA][c] = mu_UA;
+        d.cellrec[c] = make_float4(a * lwi + b * wi, a * lwo + b * wo, rho_p, 0.0f);
+    }
     stream_store(&d.born[c], rho_b);
     stream_store(&d.f[GF_PERS][c], rho_p);
     stream_store(&d.f[GF_NEW_BORN][c], rho_b);
@@ -610,7 +674,7 @@ __global__ __launch_bounds__(BLOCK) void k_mass_update(const VehDesc* __restrict
                                                        const uint32_t* __restrict__ tab, int zero_empty,
                                                        SegCarry carry, int occ_tile, fx_t* __restrict__ born_sums,
                                                        int units, const uint32_t* __restrict__ tab_e,
-                                                       fx_t* __restrict__ exp_sums)
+                                                       fx_t* __restrict__ exp_sums, int pph)
 {
     if ((int)blockIdx.x >= units)
     {
@@ -622,13 +686,93 @@ __global__ __launch_bounds__(BLOCK) void k_mass_update(const VehDesc* __restrict
     const int c = tr.base + threadIdx.x;
     float rho_b = 0.0f;
     if (c < d.C)
-        rho_b = mass_update_cell(d, c, zero_empty, carry, occ_tile);
+        rho_b = mass_update_cell(d, c, zero_empty, carry, occ_tile, pph);
     if (born_sums)
     {
         fx_t total;
         block_exclusive_scan_fx(c < d.C ? fx_from_f32(rho_b) : (fx_t)0, &total);
         if (threadIdx.x == 0)
             born_sums[blockIdx.x] = total;
+    }
+}
+
+// Vehicles with per-cell weights: first / last occurrence of every cell in the sorted particles (dogm.cu:262-281)
+// and the out-of-grid particles of the border cells.  Bound by the read of the cell words (4 N) and the
+// scattered 4-byte bounds; BOUNDS_ITEMS consecutive words per thread in 16-byte loads.
+constexpr int BOUNDS_ITEMS = 4;
+constexpr int BOUNDS_Q = BLOCK * BOUNDS_ITEMS / UNIT;
+
+__global__ __launch_bounds__(BLOCK) void k_cell_bounds(const VehDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ tab, int pph)
+{
+    const TileRef tr = tile_ref(tab, BOUNDS_Q, blockIdx.x);
+    const VehDesc& d = descs[tr.v];
+    const int n = d.N;
+    if (!d.wcell || tr.base >= n)
+        return;
+    const int* words = d.part[pph].idx;
+    const int p0 = tr.base + threadIdx.x * BOUNDS_ITEMS;
+    const int cnt = max(0, min(BOUNDS_ITEMS, n - p0));
+    const int lane = threadIdx.x & (WAVE - 1);
+    int w[BOUNDS_ITEMS];
+    load_run<BOUNDS_ITEMS>(words, p0, cnt, w, -1);
+    bool any_out = false;
+#pragma unroll
+    for (int i = 0; i < BOUNDS_ITEMS; ++i)
+        any_out |= i < cnt && word_out(w[i]);
+    int key[BOUNDS_ITEMS];
+#pragma unroll
+    for (int i = 0; i < BOUNDS_ITEMS; ++i)
+        key[i] = i < cnt ? word_index(w[i]) : -1;
+    int kprev = __shfl_up(key[BOUNDS_ITEMS - 1], 1, WAVE);
+    int knext = __shfl_down(key[0], 1, WAVE);
+    if (lane == 0)
+        kprev = p0 > 0 && p0 <= n ? word_index(words[p0 - 1]) : -1;
+    if (lane == WAVE - 1)
+        knext = p0 + BOUNDS_ITEMS < n ? word_index(words[p0 + BOUNDS_ITEMS]) : -1;
+#pragma unroll
+    for (int i = 0; i < BOUNDS_ITEMS; ++i)
+    {
+        if (i >= cnt)
+            break;
+        if (key[i] != (i == 0 ? kprev : key[i - 1]))
+            d.start[key[i]] = p0 + i;
+        if (key[i] != (i == BOUNDS_ITEMS - 1 ? knext : key[i + 1]))
+            d.end[key[i]] = p0 + i;
+    }
+    if (__ballot(any_out) == 0)
+        return;
+    // Out-of-grid particles: one atomic per run of equal cells in a thread, or one per wave inside a
+    // long run (a far ego jump puts whole sides of the grid into a few cells).
+    int* out = border_out(d);
+    const int first = __shfl(key[0], 0, WAVE);
+    bool one_cell = true;
+    int mine = 0;
+#pragma unroll
+    for (int i = 0; i < BOUNDS_ITEMS; ++i)
+    {
+        one_cell &= i >= cnt || key[i] == first;
+        mine += i < cnt && word_out(w[i]) ? 1 : 0;
+    }
+    if (__ballot(!one_cell) == 0)
+    {
+#pragma unroll
+        for (int s = WAVE / 2; s > 0; s >>= 1)
+            mine += __shfl_xor(mine, s, WAVE);
+        if (lane == 0 && mine)
+            atomicAdd(&out[first], mine);
+        return;
+    }
+    int run = 0;
+#pragma unroll
+    for (int i = 0; i < BOUNDS_ITEMS; ++i)
+    {
+        run += i < cnt && word_out(w[i]) ? 1 : 0;
+        const bool last = i == BOUNDS_ITEMS - 1 || key[i + 1] != key[i];
+        if (i < cnt && last && run)
+            atomicAdd(&out[key[i]], run);
+        if (last)
+            run = 0;
     }
 }
 
@@ -654,16 +798,23 @@ __global__ __launch_bounds__(BLOCK) void k_normalize(const VehDesc* __restrict__
 void run_occupancy(Engine* E, int pph, int zero_empty, bool defer_normalize, bool bounds, bool born_sums,
                    bool exp_sums)
 {
-    if (E->tune.seg_items == 4)
+    if (E->any_wcell)
+    {
+        launch_begin(E, K_CELL_BOUNDS);
+        hipLaunchKernelGGL(k_cell_bounds, dim3(E->tiles(SP_P, BOUNDS_Q)), dim3(BLOCK), 0, E->stream, E->d_desc,
+                           E->tab(SP_P), pph);
+        launch_end(E, K_CELL_BOUNDS);
+    }
+    if (E->any_general && E->tune.seg_items == 4)
         launch_segreduce(E, K_SEG_OCC, K_SEG_OCC_FIX, OccOp<4>{pph, bounds ? 1 : 0}, false);
-    else
+    else if (E->any_general)
         launch_segreduce(E, K_SEG_OCC, K_SEG_OCC_FIX, OccOp<8>{pph, bounds ? 1 : 0}, false);
     launch_begin(E, K_MASS_UPDATE);
     const int units = E->tiles(SP_C, 1);
     const int etiles = exp_sums ? E->tiles(SP_E, SCAN_Q) : 0;
     hipLaunchKernelGGL(k_mass_update, dim3(units + etiles), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_C),
                        zero_empty, E->seg, BLOCK * E->tune.seg_items, born_sums ? born_unit_sums(E) : (fx_t*)nullptr,
-                       units, E->tab(SP_E), E->exp_tile_sum);
+                       units, E->tab(SP_E), E->exp_tile_sum, pph);
     launch_end(E, K_MASS_UPDATE);
     if (defer_normalize)
         return;
@@ -781,6 +932,8 @@ __global__ __launch_bounds__(BLOCK) void k_post_weights(const VehDesc* __restric
 
 void run_persistent(Engine* E, int pph, bool fused_normalize, bool empty_done, bool defer_post)
 {
+    if (!E->any_general)
+        return;  // full steps only: the occupancy update did it all
     if (E->tune.seg_items == 4)
         launch_segreduce(E, K_SEG_PERS, K_SEG_PERS_FIX, PersOp<4>{pph, fused_normalize ? 1 : 0, defer_post ? 1 : 0});
     else
@@ -1065,15 +1218,20 @@ __device__ __forceinline__ int dpp_i(int x)
 
 // carry.flags[unit], and per unit MOM_CH doubles in carry.head_partial (piece of the chunk's first
 // cell when that cell started in an earlier chunk) and carry.tail_partial (piece of its last cell).
-template <int WAVES_PER_WG>
-__global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per_eu(7))) void k_moments(const VehDesc* __restrict__ descs,
-                                                                const uint32_t* __restrict__ tab, int pph, int post,
-                                                                SegCarry carry)
+// CELLS: the vehicles with per-cell weights (their records hold the posterior weights, so no prior or
+// likelihood weights are read: 16 N instead of 24 N, and eight waves per SIMD without spills); else the
+// others.
+template <int WAVES_PER_WG, bool CELLS>
+__global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per_eu(CELLS ? 6 : 7)))
+void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab, int pph, int post,
+               SegCarry carry)
 {
     const int lane = threadIdx.x & (WAVE - 1);
     const int unit = xcd_tile(blockIdx.x, gridDim.x) * WAVES_PER_WG + (int)threadIdx.x / WAVE;
     const TileRef tr = tile_ref(tab, 1, unit);
     const VehDesc& d = descs[tr.v];
+    if (CELLS != (d.wcell != 0))
+        return;
     const int n = d.N;
     const int base = tr.base;
     if (base >= n)
@@ -1084,15 +1242,18 @@ __global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per
     }
     const int p0 = base + lane * MOM_ITEMS;
     const int cnt = max(0, min(MOM_ITEMS, n - p0));
-    const int* keys = d.part[pph].idx;
-    int key[MOM_ITEMS];
-    load_run<MOM_ITEMS>(keys, p0, cnt, key, -1);
+    const int* words = d.part[pph].idx;
+    int word[MOM_ITEMS], key[MOM_ITEMS];
+    load_run<MOM_ITEMS>(words, p0, cnt, word, -1);
+#pragma unroll
+    for (int i = 0; i < MOM_ITEMS; ++i)
+        key[i] = i < cnt ? word_index(word[i]) : -1;
     int kprev = __shfl_up(key[MOM_ITEMS - 1], 1, WAVE);
     int knext = __shfl_down(key[0], 1, WAVE);
     if (lane == 0)
-        kprev = base > 0 ? keys[base - 1] : -1;
+        kprev = base > 0 ? word_index(words[base - 1]) : -1;
     if (lane == WAVE - 1)
-        knext = p0 + MOM_ITEMS < n ? keys[p0 + MOM_ITEMS] : -1;
+        knext = p0 + MOM_ITEMS < n ? word_index(words[p0 + MOM_ITEMS]) : -1;
     bool head[MOM_ITEMS], end[MOM_ITEMS], started[MOM_ITEMS];
     bool lh = false;
 #pragma unroll
@@ -1110,24 +1271,46 @@ __global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per
     // carry them), loaded before any store so that they travel with the other loads instead of
     // waiting behind the weight_array stores.
     float rho[MOM_ITEMS];
-    float4 cf[MOM_ITEMS];
-#pragma unroll
-    for (int i = 0; i < MOM_ITEMS; ++i)
-    {
-        cf[i] = post && i < cnt ? d.cellrec[key[i]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        rho[i] = post ? cf[i].z : (end[i] ? d.f[GF_PERS][key[i]] : 0.0f);
-    }
     float w[MOM_ITEMS];
-    load_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
-    if (post)
+    if constexpr (CELLS)
     {
-        float wp[MOM_ITEMS];
-        load_run<MOM_ITEMS>(d.part[pph].weight, p0, cnt, wp);
+        // The cell record holds the posterior weights themselves (mass_update_cell).
 #pragma unroll
         for (int i = 0; i < MOM_ITEMS; ++i)
+        {
+            float in = 0.0f, out = 0.0f;
+            rho[i] = 0.0f;
             if (i < cnt)
-                w[i] = cf[i].x * w[i] + cf[i].y * wp[i];  // (p_A mu_A) w + ((1 - p_A) mu_UA) w_prior
+            {
+                const float4 cf = d.cellrec[key[i]];
+                in = cf.x;
+                out = cf.y;
+                rho[i] = cf.z;
+            }
+            w[i] = word_out(word[i]) ? out : in;
+        }
         store_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
+    }
+    else
+    {
+        float4 cf[MOM_ITEMS];
+#pragma unroll
+        for (int i = 0; i < MOM_ITEMS; ++i)
+        {
+            cf[i] = post && i < cnt ? d.cellrec[key[i]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            rho[i] = post ? cf[i].z : (end[i] ? d.f[GF_PERS][key[i]] : 0.0f);
+        }
+        load_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
+        if (post)
+        {
+            float wp[MOM_ITEMS];
+            load_run<MOM_ITEMS>(d.part[pph].weight, p0, cnt, wp);
+#pragma unroll
+            for (int i = 0; i < MOM_ITEMS; ++i)
+                if (i < cnt)
+                    w[i] = cf[i].x * w[i] + cf[i].y * wp[i];  // (p_A mu_A) w + ((1 - p_A) mu_UA) w_prior
+            store_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
+        }
     }
     float vx[MOM_ITEMS], vy[MOM_ITEMS];
     {
@@ -1262,7 +1445,7 @@ __global__ __launch_bounds__(BLOCK) void k_moments_fix(const VehDesc* __restrict
         s[c] = (float)(acc[c] + headp[(size_t)j * MOM_CH + c]);
     const TileRef tr = tile_ref(tab, 1, u);
     const VehDesc& d = descs[tr.v];
-    const int key = d.part[pph].idx[tr.base + MOM_CHUNK - 1];
+    const int key = word_index(d.part[pph].idx[tr.base + MOM_CHUNK - 1]);
     mom_finalize(d, key, d.f[GF_PERS][key], s);
 }
 
@@ -1273,9 +1456,14 @@ void run_moments(Engine* E, int pph, bool fused_post, bool empty_done)
     const int units = (int)E->units[SP_P];
     if (units > 0)
     {
+        const dim3 grid(units / MOM_WAVES_PER_WG), block(MOM_WAVES_PER_WG * WAVE);
         launch_begin(E, K_SEG_MOM);
-        hipLaunchKernelGGL(k_moments<MOM_WAVES_PER_WG>, dim3(units / MOM_WAVES_PER_WG), dim3(MOM_WAVES_PER_WG * WAVE),
-                           0, E->stream, E->d_desc, E->tab(SP_P), pph, fused_post ? 1 : 0, E->seg);
+        if (E->any_wcell)
+            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, true>), grid, block, 0, E->stream, E->d_desc,
+                               E->tab(SP_P), pph, 1, E->seg);
+        if (E->any_general)
+            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, false>), grid, block, 0, E->stream, E->d_desc,
+                               E->tab(SP_P), pph, fused_post ? 1 : 0, E->seg);
         launch_end(E, K_SEG_MOM);
         launch_begin(E, K_SEG_MOM_FIX);
         hipLaunchKernelGGL(k_moments_fix, dim3(div_up(units, BLOCK)), dim3(BLOCK), 0, E->stream, E->d_desc,

@@ -537,7 +537,7 @@ __device__ __forceinline__ void merge_write(const VehDesc& d, const DevScalars* 
         const uint8_t* as = from_p ? P.assoc : Bp.assoc;
         out.pos[k] = ps[o];
         out.vel[k] = vs[o];
-        out.idx[k] = ix[o];
+        out.idx[k] = word_index(ix[o]);
         out.assoc[k] = as[o];
         out.weight[k] = nw;
     }
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(BLOCK) void k_materialize(DevParticles dst, DevPart
     const DevParticles& s = from_p ? src : birth;
     dst.pos[k] = s.pos[o];
     dst.vel[k] = s.vel[o];
-    dst.idx[k] = s.idx[o];
+    dst.idx[k] = word_index(s.idx[o]);
     dst.assoc[k] = s.assoc[o];
     if (k > 0)
         dst.weight[k] = dst.weight[0];

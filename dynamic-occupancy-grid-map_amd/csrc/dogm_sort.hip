@@ -83,6 +83,30 @@ __device__ __forceinline__ const int* sort_keys_in(const VehDesc& d, int pph, in
     return ps == 0 ? d.part[pph].idx : d.sort_keys[(ps - 1) & 1];
 }
 
+// Key and value of element p of a pass.  Pass 0 (no values yet) takes the identity values with the
+// particles' flags: from the words predict left in the same step (packed), else from the association bytes.
+__device__ __forceinline__ void load_key(const VehDesc& d, int pph, const int* __restrict__ keys_in,
+                                         const int* __restrict__ vals_in, int p, bool valid, bool packed, int& key,
+                                         int& val)
+{
+    const int k = valid ? keys_in[p] : 0;
+    if (vals_in)
+    {
+        key = k;
+        val = valid ? vals_in[p] : 0;
+    }
+    else if (packed)
+    {
+        key = word_index(k);
+        val = (int)((unsigned)p | ((unsigned)k & WORD_FLAGS));
+    }
+    else
+    {
+        key = k;
+        val = valid ? sort_value(p, d.part[pph].assoc[p]) : 0;
+    }
+}
+
 // ---- reduce-then-scan form: per pass an upsweep of tile digit counts, a scan per (vehicle, digit)
 //      over the vehicle's tiles, and the ranking and scatter -----------------------------------
 
@@ -195,13 +219,14 @@ __global__ __launch_bounds__(BLOCK) void k_sort_scan(const VehDesc* __restrict__
 }
 
 // Stable ranking and scatter of one tile.  Pass 0 ranks the particles' cell indices with identity
-// values carrying the particle's association flag in bit 31 (read here in particle order, so the
-// gather needs no random byte load); later passes read the previous pass's output.
+// values carrying the particle's flags (read here in particle order, so the gather needs no random byte
+// load); later passes read the previous pass's output.
 // GATHER (last pass only): instead of the sorted keys and the permutation, write the particles in
 // sorted order into part[pph ^ 1] (cell index, state, weight, association) and, with GATHER_WA, the
 // weight copy into weight_array; the cell bounds are then recorded by the next segmented reduction.
 // With GATHER_AOS the state is read from the 16-byte records predict left in the CDF buffer, and
-// for vehicles with uniform weights the predicted weight is formed here (predicted_weight).
+// for vehicles with uniform weights the predicted weight is formed here (predicted_weight), or not at all where
+// the occupancy update forms the weights per cell (VehDesc::wcell).
 template <bool GATHER>
 __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ tab, int pph, int ps, int tiles,
@@ -222,6 +247,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
     if (tbase >= n)
         return;
     const int shift = ps * RADIX_BITS;
+    const bool packed = (gflags & GATHER_AOS) != 0;
     if (ps == passes - 1 && tbase == 0)
     {
         // The digit scans of every pass have run: clear this vehicle's histograms for the next sort.
@@ -248,8 +274,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
     {
         const int p = tbase + (wid * SORT_ITEMS + j) * WAVE + lane;
         const bool valid = p < n;
-        key[j] = valid ? keys_in[p] : 0;
-        val[j] = valid ? (vals_in ? vals_in[p] : sort_value(p, dv.part[pph].assoc[p])) : 0;
+        load_key(dv, pph, keys_in, vals_in, p, valid, packed, key[j], val[j]);
         const unsigned d = ((unsigned)key[j] >> shift) & (RADIX - 1);
         const uint64_t peers = match_digit(d, __ballot(valid));
         unsigned r = 0;
@@ -342,13 +367,17 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
         {
             const DevParticles src = dv.part[pph];
             const DevParticles dst = dv.part[pph ^ 1];
-            const int o = sort_value_index(vv[b]);
+            const int o = word_index(vv[b]);
+            dst.assoc[g] = word_assoc(vv[b]);
+            dst.idx[g] = (int)((unsigned)kk[b] | ((unsigned)vv[b] & WORD_OUT));
             float w;
             if (gflags & GATHER_AOS)
             {
                 const float4 st = reinterpret_cast<const float4*>(dv.cdf)[o];
                 dst.pos[g] = make_float2(st.x, st.y);
                 dst.vel[g] = make_float2(st.z, st.w);
+                if (dv.wcell)
+                    continue;  // the occupancy update forms the weights per cell
                 w = dv.wuni ? predicted_weight(dv, w_prior, st) : src.weight[o];
             }
             else
@@ -358,8 +387,6 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
                 dst.vel[g] = src.vel[o];
             }
             dst.weight[g] = w;
-            dst.assoc[g] = sort_value_assoc(vv[b]);
-            dst.idx[g] = kk[b];
             if (gflags & GATHER_WA)
                 dv.weight_array[g] = w;
         }
@@ -427,14 +454,14 @@ __device__ __forceinline__ unsigned lb_read(const unsigned* w)
 // position (w*ITEMS + j)*64 + l), each wave ranks its 64 keys of one item with ballot-matched peer
 // masks against per-wave digit counters in LDS, and waves are combined in order.  The scatter is
 // staged through LDS in digit-sorted order so that equal digits leave the tile as contiguous runs.
-// Pass 0 ranks the particles' cell indices with identity values carrying the particle's association
-// flag in bit 31 (read here in particle order, so the gather needs no random byte load); later
-// passes read the previous pass's output.
+// Pass 0 ranks the particles' cell indices with identity values carrying the particle's flags (read here
+// in particle order, so the gather needs no random byte load); later passes read the previous pass's output.
 // GATHER (last pass only): instead of the sorted keys and the permutation, write the particles in
 // sorted order into part[pph ^ 1] (cell index, state, weight, association) and, with GATHER_WA, the
 // weight copy into weight_array; the cell bounds are then recorded by the next segmented reduction.
 // With GATHER_AOS the state is read from the 16-byte records predict left in the CDF buffer, and
-// for vehicles with uniform weights the predicted weight is formed here (predicted_weight).
+// for vehicles with uniform weights the predicted weight is formed here (predicted_weight), or not at all where
+// the occupancy update forms the weights per cell (VehDesc::wcell).
 template <bool GATHER>
 __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restrict__ descs,
                                                          const uint32_t* __restrict__ tab, int pph, int ps, int passes,
@@ -463,6 +490,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
     if (tbase >= n)
         return;  // padding past the vehicle's particles: no later tile of the vehicle looks back here
     const int shift = ps * RADIX_BITS;
+    const bool packed = (gflags & GATHER_AOS) != 0;
     const int* keys_in = sort_keys_in(dv, pph, ps);
     const int* vals_in = ps == 0 ? nullptr : dv.sort_vals[(ps - 1) & 1];
     int* keys_out = dv.sort_keys[ps & 1];
@@ -479,8 +507,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
     {
         const int p = tbase + (wid * SORT_ITEMS + j) * WAVE + lane;
         const bool valid = p < n;
-        key[j] = valid ? keys_in[p] : 0;
-        val[j] = valid ? (vals_in ? vals_in[p] : sort_value(p, dv.part[pph].assoc[p])) : 0;
+        load_key(dv, pph, keys_in, vals_in, p, valid, packed, key[j], val[j]);
         const unsigned d = ((unsigned)key[j] >> shift) & (RADIX - 1);
         const uint64_t peers = match_digit(d, __ballot(valid));
         unsigned r = 0;
@@ -655,13 +682,17 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
         {
             const DevParticles src = dv.part[pph];
             const DevParticles dst = dv.part[pph ^ 1];
-            const int o = sort_value_index(vv[b]);
+            const int o = word_index(vv[b]);
+            dst.assoc[g] = word_assoc(vv[b]);
+            dst.idx[g] = (int)((unsigned)kk[b] | ((unsigned)vv[b] & WORD_OUT));
             float w;
             if (gflags & GATHER_AOS)
             {
                 const float4 st = reinterpret_cast<const float4*>(dv.cdf)[o];
                 dst.pos[g] = make_float2(st.x, st.y);
                 dst.vel[g] = make_float2(st.z, st.w);
+                if (dv.wcell)
+                    continue;  // the occupancy update forms the weights per cell
                 w = dv.wuni ? predicted_weight(dv, w_prior, st) : src.weight[o];
             }
             else
@@ -671,8 +702,6 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
                 dst.vel[g] = src.vel[o];
             }
             dst.weight[g] = w;
-            dst.assoc[g] = sort_value_assoc(vv[b]);
-            dst.idx[g] = kk[b];
             if (gflags & GATHER_WA)
                 dv.weight_array[g] = w;
         }
@@ -730,7 +759,7 @@ void run_sort(Engine* E, int pph, bool hist_done, bool gather, bool write_wa)
             else
                 hipLaunchKernelGGL(k_sort_onesweep<false>, dim3(tiles), dim3(BLOCK), 0, E->stream, E->d_desc,
                                    E->tab(SP_P), pph, ps, passes, E->sort_ghist, E->sort_status, E->sort_tickets,
-                                   epoch, E->lookback_spin, E->d_err, 0);
+                                   epoch, E->lookback_spin, E->d_err, gflags);
             launch_end(E, g ? K_SORT_GATHER : K_SORT_DOWNSWEEP);
             continue;
         }
@@ -752,7 +781,7 @@ void run_sort(Engine* E, int pph, bool hist_done, bool gather, bool write_wa)
                                pph, ps, tiles, E->sort_status, passes, E->sort_ghist, gflags);
         else
             hipLaunchKernelGGL(k_sort_downsweep<false>, dim3(tiles), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, ps, tiles, E->sort_status, passes, E->sort_ghist, 0);
+                               E->tab(SP_P), pph, ps, tiles, E->sort_status, passes, E->sort_ghist, gflags);
         launch_end(E, g ? K_SORT_GATHER : K_SORT_DOWNSWEEP);
     }
     E->ghist_clean = true;  // the last pass cleared the histograms
