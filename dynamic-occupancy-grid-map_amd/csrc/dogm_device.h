@@ -47,6 +47,26 @@ __device__ __forceinline__ fx_t wave_inclusive_scan_fx(fx_t x)
     return x;
 }
 
+// The same scan of 64-bit integers.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint64_t dpp_u64(uint64_t x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROW_MASK, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, ROW_MASK, 0xf, false);
+    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+
+__device__ __forceinline__ uint64_t wave_inclusive_scan_u64(uint64_t x)
+{
+    x += dpp_u64<0x111, 0xf>(x);
+    x += dpp_u64<0x112, 0xf>(x);
+    x += dpp_u64<0x114, 0xf>(x);
+    x += dpp_u64<0x118, 0xf>(x);
+    x += dpp_u64<0x142, 0xa>(x);
+    x += dpp_u64<0x143, 0xc>(x);
+    return x;
+}
+
 // DPP moves and the same wave scan for f32 / f64 values (float CDF modes).  The association is
 // fixed by the six DPP steps: value + shifted value, rows of 16 first, then the row totals.
 template <int CTRL, int ROW_MASK>
@@ -739,6 +759,35 @@ struct SrcExp
     }
 };
 
+// Tile `tile` of the exponentials: the tile total into tile_sum[tile], summed in units of 2^-48 (64-bit adds
+// instead of 128-bit conversions and adds).
+__device__ __forceinline__ void exp_tile_body(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab,
+                                              int tile, fx_t* __restrict__ tile_sum)
+{
+    __shared__ uint64_t s_w[BLOCK / WAVE];
+    const TileRef tr = tile_ref(tab, SCAN_Q, tile);
+    const VehDesc& d = descs[tr.v];
+    if (!SrcExp{}.active(d))
+        return;  // uniform over the workgroup
+    const int p0 = tr.base + threadIdx.x * SCAN_ITEMS;
+    const int n = d.N + 1;
+    uint64_t s = 0;
+    if (p0 < n)
+    {
+        float v[SCAN_ITEMS];
+        SrcExp{}.load4(d, p0, SCAN_ITEMS, v);
+#pragma unroll
+        for (int i = 0; i < SCAN_ITEMS; ++i)
+            s += p0 + i < n ? exp_units(v[i]) : 0;
+    }
+    const uint64_t incl = wave_inclusive_scan_u64(s);
+    if ((threadIdx.x & (WAVE - 1)) == WAVE - 1)
+        s_w[threadIdx.x / WAVE] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        tile_sum[tile] = fx_from_exp_units(s_w[0] + s_w[1] + s_w[2] + s_w[3]);
+}
+
 // Tile `tile` of a space: the tile total into tile_sum[tile] (and the segment ends, see above).
 template <class Src>
 __device__ __forceinline__ void scan_tile_body(const Src& src, const VehDesc* __restrict__ descs,
@@ -776,20 +825,19 @@ __global__ __launch_bounds__(BLOCK) void k_scan_tiles(Src src, const VehDesc* __
     scan_tile_body(src, descs, tab, blockIdx.x, tile_sum, seg_end);
 }
 
-// The tiles of two independent spaces in one launch: workgroups [0, tiles_a) take space A, the rest
-// space B (one launch instead of two; alternating the spaces measured no faster).
-template <class SrcA, class SrcB>
-__global__ __launch_bounds__(BLOCK) void k_scan_tiles_pair(SrcA a, const uint32_t* __restrict__ tab_a, int tiles_a,
-                                                           fx_t* __restrict__ sum_a, fx_t* __restrict__ seg_end_a,
-                                                           SrcB b, const uint32_t* __restrict__ tab_b, int tiles_b,
-                                                           fx_t* __restrict__ sum_b,
-                                                           const VehDesc* __restrict__ descs)
+// The tiles of a space and of the exponentials in one launch: workgroups [0, tiles_a) take space A, the
+// rest the exponentials (one launch instead of two; alternating them measured no faster).
+template <class SrcA>
+__global__ __launch_bounds__(BLOCK) void k_scan_tiles_exp(SrcA a, const uint32_t* __restrict__ tab_a, int tiles_a,
+                                                          fx_t* __restrict__ sum_a, fx_t* __restrict__ seg_end_a,
+                                                          const uint32_t* __restrict__ tab_e,
+                                                          fx_t* __restrict__ sum_e,
+                                                          const VehDesc* __restrict__ descs)
 {
-    (void)tiles_b;
     if ((int)blockIdx.x < tiles_a)
         scan_tile_body(a, descs, tab_a, blockIdx.x, sum_a, seg_end_a);
     else
-        scan_tile_body(b, descs, tab_b, blockIdx.x - tiles_a, sum_b, (fx_t*)nullptr);
+        exp_tile_body(descs, tab_e, blockIdx.x - tiles_a, sum_e);
 }
 
 enum ScanMode

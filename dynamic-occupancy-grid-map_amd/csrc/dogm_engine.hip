@@ -545,7 +545,6 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         // and every other one 0, so the per-cell sums need counts only.
         d.wcell = d.wuni && (stages & ST_ALL) == ST_ALL ? 1 : 0;
         d.rs_gather = v->rs_pending && !d.init && full_predict ? 1 : 0;
-        d.rs_defer = (stages & ST_RESAMPLE) ? 1 : 0;
         d.ep_init = e;
         e += d.init ? 1u : 0u;
         d.ep_pred = e;
@@ -831,7 +830,7 @@ int engine_run(Engine* E, Vehicle* const* veh, int m, int stages)
         else
             v->w_uniform = d.wuni != 0;
         // A resampling leaves a deferred set (merge_write); a prediction that read one consumed it.
-        if (d.rs_defer)
+        if (stages & ST_RESAMPLE)
             v->rs_pending = true;
         else if (d.rs_gather)
             v->rs_pending = false;

@@ -116,7 +116,6 @@ struct VehDesc
     int wuni;                // every weight predict reads equals weight[0] (resampled or initialised)
     int wcell;               // full step from uniform weights: a cell's particles share one weight (cell_weights)
     int rs_gather;           // part[0] is a deferred resampled set: predict reads it through ancestors
-    int rs_defer;            // the resampling writes ancestors and weight[0] only (a deferred set)
     int move;                // pending particle shift (fused into predict)
     float mx, my;
     int shifted;             // pending grid shift (fused into the occupancy update)

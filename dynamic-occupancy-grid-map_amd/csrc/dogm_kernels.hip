@@ -679,7 +679,7 @@ __global__ __launch_bounds__(BLOCK) void k_mass_update(const VehDesc* __restrict
 {
     if ((int)blockIdx.x >= units)
     {
-        scan_tile_body(SrcExp{}, descs, tab_e, (int)blockIdx.x - units, exp_sums, (fx_t*)nullptr);
+        exp_tile_body(descs, tab_e, (int)blockIdx.x - units, exp_sums);
         return;
     }
     const TileRef tr = tile_ref(tab, 1, blockIdx.x);

@@ -494,6 +494,24 @@ DOGM_HD void resample_exponentials4(uint64_t seed, uint32_t instance, uint32_t e
     e[3] = -log_f32(uniform01_oc(r.w));
 }
 
+// An exponential (log_f32 of a 24-bit uniform, negated) in units of 2^-48: exact, because all 2^24 of them are
+// multiples of 2^-48 below 17 (0 for u = 1), so up to 1024 of them sum in 64 bits and the fixed-point value
+// is the sum times 2^40.
+constexpr int EXP_FRAC = 48;
+
+DOGM_HD uint64_t exp_units(float e)
+{
+    const uint32_t b = f32_bits(e);
+    const int E = (int)((b >> 23) & 0xffu);
+    const uint64_t m = (uint64_t)((b & 0x007fffffu) | 0x00800000u);
+    return E == 0 ? 0 : m << ((E - 150 + EXP_FRAC) & 63);
+}
+
+DOGM_HD fx_t fx_from_exp_units(uint64_t s)
+{
+    return (fx_t)((ufx_t)s << (FX_FRAC - EXP_FRAC));
+}
+
 DOGM_HD float resample_exponential(uint64_t seed, uint32_t instance, uint32_t epoch, uint32_t k)
 {
     float e[4];

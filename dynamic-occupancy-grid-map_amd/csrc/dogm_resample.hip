@@ -9,11 +9,12 @@
 // 3. Merge: a workgroup owns 1024 consecutive (hence sorted) draws.  Its ancestors lie between the
 //    CDF segments holding its first and last draw; those are found by a two-level k-ary search over
 //    the coarse index (two dependent loads instead of a 22-level binary search), the CDF entries of
-//    those segments are rebuilt in LDS from the weights (one wave per segment: exact wave scan +
-//    the index entry before the segment), and every draw finds its ancestor there (the reference's
-//    lower_bound).  The reference's resamplingKernel gather is deferred: only the ancestors (and the
-//    new weight) are written, the next full step's prediction reads each state through its
-//    ancestor, and anything else that reads the particles first has k_materialize copy them.
+//    those segments are rebuilt from the weights as 31-bit keys relative to the window (one wave per
+//    segment), and every draw finds its ancestor among the keys (the reference's lower_bound); the few
+//    draws whose key does not decide are resolved exactly.  The reference's resamplingKernel gather is
+//    deferred: only the ancestors (and the new weight) are written, the next full step's prediction
+//    reads each state through its ancestor, and anything else that reads the particles first has
+//    k_materialize copy them.
 // No atomics on global memory and no global sort: the result is a pure function of the inputs.
 // Every vehicle of a step resamples from its own CDF with its own draws.
 #include "dogm_device.h"
@@ -23,13 +24,11 @@ namespace dogm_hip
 
 constexpr int RS_ITEMS = 4;
 constexpr int RS_TILE = BLOCK * RS_ITEMS;  // draws per workgroup
-// CDF entries staged in LDS per window: 8 segments (2048 entries) for launches of up to
-// RS_WIDE_MAX_TILES workgroups (fewer windows per workgroup shortens the critical path), 4 segments
-// for larger launches (half the LDS, more workgroups per CU).  The float modes stage whole tiles
-// (RS_FLOAT_SLICE_TILES per window).
+// CDF entries staged in LDS per window: 8 segments (2048 entries, the built-in choice: 1024 draws mostly need one
+// window) or 4 (the other choice of the tuning, 1% slower per step of 32 x 2e6 particles).  The float
+// modes stage whole tiles (RS_FLOAT_SLICE_TILES per window).
 constexpr int RS_WINDOW_NARROW = 4;
 constexpr int RS_WINDOW_WIDE = 8;
-constexpr int RS_WIDE_MAX_TILES = 4096;
 constexpr int RS_FLOAT_SLICE_TILES = 2;
 // Doubles per scan tile in the float modes' index (the envelope at the tile end and before it),
 // spaced like the exact mode's segment ends so that vehicles of both kinds in one step keep
@@ -62,14 +61,41 @@ struct SrcJointPos
     }
 };
 
-// E for the four consecutive draws k = p0 .. p0 + 3 of one thread (p0 is a multiple of 4).
-__device__ __forceinline__ void exp4(const VehDesc& d, int p0, int n, fx_t* e)
+// The spacings' exact prefixes S_k of the thread's four consecutive draws k = base + 4 threadIdx.x .. + 3, each
+// handed to put(i, S_k) (multinomial draws; all threads of the workgroup call it).  Inside the workgroup's 1024
+// draws the exponentials are summed in 64-bit units of 2^-48; the tile's prefix joins in 128 bits.
+template <class Put>
+__device__ __forceinline__ void spacing_prefixes(const VehDesc& d, int base, int n,
+                                                 const fx_t* __restrict__ exp_tile_pre, const Put& put)
 {
-    float f[4];
-    resample_exponentials4(d.seed, d.inst, d.ep_rs, (uint32_t)(p0 >> 2), f);
+    __shared__ uint64_t s_w[BLOCK / WAVE];
+    const int q0 = base + threadIdx.x * RS_ITEMS;
+    float f[RS_ITEMS];
+    resample_exponentials4(d.seed, d.inst, d.ep_rs, (uint32_t)(q0 >> 2), f);
+    uint64_t e[RS_ITEMS];
+    uint64_t sum = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        e[i] = p0 + i < n ? fx_from_f32_nonneg(f[i]) : (fx_t)0;  // -log(u) >= 0 (or -0)
+    for (int i = 0; i < RS_ITEMS; ++i)
+    {
+        e[i] = q0 + i < n ? exp_units(f[i]) : 0;
+        sum += e[i];
+    }
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+    const uint64_t incl = wave_inclusive_scan_u64(sum);
+    if (lane == WAVE - 1)
+        s_w[wid] = incl;
+    __syncthreads();
+    uint64_t run = incl - sum;
+#pragma unroll
+    for (int w = 0; w < BLOCK / WAVE - 1; ++w)
+        run += w < wid ? s_w[w] : 0;
+    const fx_t pre = exp_tile_pre[d.u0[SP_E] / SCAN_Q + base / RS_TILE];
+#pragma unroll
+    for (int i = 0; i < RS_ITEMS; ++i)
+    {
+        run += e[i];
+        put(i, pre + fx_from_exp_units(run));
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -352,49 +378,15 @@ struct CdfFloatTr
     }
 };
 
-// A chunk of CDF entries staged in LDS.  Exact entries (128-bit) are kept as separate high and low
-// 64-bit words: the lower-bound search compares the high words (8-byte LDS reads, half the bytes
-// and bank traffic of 16-byte ones) and reads a low word only where the high words tie.  Entry i
-// sits at slot i + i / 32: the rebuild writes four consecutive entries per thread, and without the
-// skew the lanes of a wave would hit the same banks eight at a time (entries 32 words apart).
-__device__ __forceinline__ int cdf_slot(int i)
-{
-    return i + (i >> 5);
-}
-
-template <class V, int LEN>
+// Envelope entries staged in LDS (float modes).  Entry i sits at slot i + i / 32.
+template <int LEN>
 struct CdfStage
 {
-    V v[LEN + LEN / 32];
-    __device__ void put(int i, const V& x) { v[cdf_slot(i)] = x; }
-    __device__ V get(int i) const { return v[cdf_slot(i)]; }
-    __device__ bool less(int i, const V& r) const { return v[cdf_slot(i)] < r; }
-};
-
-template <int LEN>
-struct CdfStage<fx_t, LEN>
-{
-    int64_t hi[LEN + LEN / 32];
-    uint64_t lo[LEN + LEN / 32];
-    __device__ void put(int i, const fx_t& x)
-    {
-        const int s = cdf_slot(i);
-        hi[s] = (int64_t)(x >> 64);
-        lo[s] = (uint64_t)x;
-    }
-    __device__ fx_t get(int i) const
-    {
-        const int s = cdf_slot(i);
-        return (fx_t)(((ufx_t)(uint64_t)hi[s] << 64) | (ufx_t)lo[s]);
-    }
-    // Both words are read at once (one LDS round trip per probe) and compared without a branch.
-    __device__ bool less(int i, const fx_t& r) const
-    {
-        const int s = cdf_slot(i);
-        const int64_t h = hi[s], rh = (int64_t)(r >> 64);
-        const uint64_t l = lo[s];
-        return (h < rh) | ((h == rh) & (l < (uint64_t)r));
-    }
+    double v[LEN + LEN / 32];
+    __device__ static int slot(int i) { return i + (i >> 5); }
+    __device__ void put(int i, double x) { v[slot(i)] = x; }
+    __device__ double get(int i) const { return v[slot(i)]; }
+    __device__ bool less(int i, double r) const { return v[slot(i)] < r; }
 };
 
 // Index of the first of n non-decreasing values value(0 .. n-1) that is >= r (n - 1 if none): a
@@ -424,16 +416,12 @@ __device__ int find_first_not_below(const Get& value, int n, V r, int* s_cnt)
     return t;
 }
 
-// The workgroup's draws r_k, k = base + threadIdx.x + i * BLOCK (item i of a thread is strided, so
-// at every item a wave searches 64 consecutive draws, whose lower bounds are neighbouring CDF
-// entries: the probes of a wave read neighbouring LDS words, and the ancestors come out
-// wave-contiguous for the gather), and s_rb = {first draw, last draw}.  Multinomial draws: the
-// spacings' prefix runs over four consecutive draws per thread (one Philox call each); the draws
-// are then moved to their strided owners through the staging buffer.
-template <class V, class Draw, class Stage>
+// The workgroup's draws r_k, k = base + threadIdx.x + i * BLOCK, in the float modes (item i of a thread is
+// strided, so at every item a wave searches 64 consecutive draws), and s_rb = {first draw, last draw}.
+template <class Draw, class Stage>
 __device__ __forceinline__ void merge_draws(const VehDesc& d, const DevScalars* sc, int base, int n,
                                             const fx_t* __restrict__ exp_tile_pre, const Draw& draw, Stage& stage,
-                                            V (&r)[RS_ITEMS], V* s_rb)
+                                            double (&r)[RS_ITEMS], double* s_rb)
 {
     const int last = min(base + RS_TILE, n) - 1;
     const Spacing sp = sc->spacing;
@@ -446,18 +434,8 @@ __device__ __forceinline__ void merge_draws(const VehDesc& d, const DevScalars* 
     }
     else
     {
-        const int q0 = base + threadIdx.x * RS_ITEMS;
-        fx_t e[4];
-        exp4(d, q0, n, e);
-        fx_t tot;
-        fx_t run = block_exclusive_scan_fx(e[0] + e[1] + e[2] + e[3], &tot) +
-                   exp_tile_pre[d.u0[SP_E] / SCAN_Q + base / RS_TILE];
-#pragma unroll
-        for (int i = 0; i < RS_ITEMS; ++i)
-        {
-            run += e[i];
-            stage.put(threadIdx.x * RS_ITEMS + i, draw(run, sp));
-        }
+        spacing_prefixes(d, base, n, exp_tile_pre,
+                         [&](int i, fx_t s_k) { stage.put(threadIdx.x * RS_ITEMS + i, draw(s_k, sp)); });
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < RS_ITEMS; ++i)
@@ -503,44 +481,22 @@ __device__ __forceinline__ int merge_next_draw(int base, int n, const int (&anc)
     return kmin;
 }
 
-// The resampled particles k = base + threadIdx.x + i * BLOCK: ancestor index, state copied from the
-// ancestor (posterior particle or new-born one) and the uniform new weight.  A draw without an
-// ancestor (above the CDF total by rounding) takes the last joint entry.  A deferred set
-// (d.rs_defer) gets the ancestors and weight[0] only: the next prediction reads the states through
-// the ancestors, and every other reader first writes the set out (k_materialize).
+// The resampled particles k = base + threadIdx.x + i * BLOCK, left by reference: the ancestor index (a draw
+// without an ancestor, above the CDF total by rounding, takes the last joint entry) and the uniform new weight in
+// weight[0].  The next full step's prediction reads the states through the ancestors, and every other reader first
+// writes the set out (k_materialize).
 __device__ __forceinline__ void merge_write(const VehDesc& d, const DevScalars* sc, int pph, int base, int n, int J,
                                             const int (&anc)[RS_ITEMS])
 {
-    const float nw = sc->new_weight;
-    const DevParticles P = d.part[pph];
-    const DevParticles Bp = d.birth;
-    const DevParticles out = d.part[pph ^ 1];
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
     {
         const int k = base + i * BLOCK + (int)threadIdx.x;
-        if (k >= n)
-            break;
-        const int a = anc[i] < 0 ? J - 1 : min(anc[i], J - 1);
-        d.ancestors[k] = a;
-        if (d.rs_defer)
-        {
-            if (k == 0)
-                out.weight[0] = nw;
-            continue;
-        }
-        const bool from_p = a < n;
-        const int o = from_p ? a : a - n;
-        const float2* ps = from_p ? P.pos : Bp.pos;
-        const float2* vs = from_p ? P.vel : Bp.vel;
-        const int* ix = from_p ? P.idx : Bp.idx;
-        const uint8_t* as = from_p ? P.assoc : Bp.assoc;
-        out.pos[k] = ps[o];
-        out.vel[k] = vs[o];
-        out.idx[k] = word_index(ix[o]);
-        out.assoc[k] = as[o];
-        out.weight[k] = nw;
+        if (k < n)
+            d.ancestors[k] = anc[i] < 0 ? J - 1 : min(anc[i], J - 1);
     }
+    if (base == 0 && threadIdx.x == 0)
+        d.part[pph ^ 1].weight[0] = sc->new_weight;
 }
 
 // Index of the first of n non-decreasing values value(0 .. n-1) that is >= r (n - 1 if none), for
@@ -568,29 +524,85 @@ __device__ __forceinline__ void wave_find2(const Get& value, int n, V r0, V r1, 
     *c1 = min(b1 + n1, n - 1);
 }
 
-// Exact-CDF merge.  The workgroup's ancestors lie in the CDF segments [s_lo, s_hi] holding its first
-// and last draw; they are staged WSEG segments at a time.  Each wave rebuilds whole segments: the 64
-// lanes' four joint weights in fixed point, a 64-lane exact scan, and the index entry before the
-// segment as its start (integer adds, so the entries equal those of any other association).  A
-// draw is resolved in the first window whose last entry is >= its value (the CDF is non-decreasing,
-// so its lower bound is there), by a branch-free binary search over the window padded to a power
-// of two; windows no remaining draw lands in are skipped with one coarse-index search.  Every wave
-// runs the coarse-index searches itself (the same answer in each), so the only barriers are those of
-// the draws' prefix and two per window plus one between windows.
-// Seven waves per SIMD for the 4-segment window; the 8-segment form is bounded by its LDS.
+// The CDF in raw fixed-point units (value * 2^88) as a double; exact below 2^53 raw units.
+__device__ __forceinline__ double fx_raw_f64(fx_t v)
+{
+    return fx_to_f64(v) * 0x1p88;
+}
+
+// Four joint weights in raw fixed-point units: fx_from_f32_nonneg as doubles (a 24-bit significand truncated to an
+// integer), for weights below 2^39.
+__device__ __forceinline__ void raw_weights(const float (&f)[SCAN_ITEMS], double (&v)[SCAN_ITEMS])
+{
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i)
+        v[i] = trunc((double)f[i] * 0x1p88);
+}
+
+// First joint entry whose exact CDF value is >= r, by one wave: the coarse index gives the segment, the
+// segment's entries are rebuilt exactly (the 64 lanes' four weights in fixed point, a 64-lane exact scan and the
+// index entry before the segment) and those below r counted.
+__device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const fx_t* __restrict__ si, int S, int J, fx_t r)
+{
+    const int lane = threadIdx.x & (WAVE - 1);
+    int s, unused;
+    wave_find2<fx_t>([si](int k) { return si[k]; }, S, r, r, &s, &unused);
+    const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
+    const int cnt = max(0, min(SCAN_ITEMS, J - q0));
+    float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (cnt > 0)
+        SrcJointPos{}.load4(d, q0, cnt, f);
+    fx_t v[SCAN_ITEMS];
+    fx_t sum = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i)
+    {
+        v[i] = i < cnt ? fx_from_f32_nonneg(f[i]) : (fx_t)0;  // cdf_weight: sign bit clear
+        sum += v[i];
+    }
+    fx_t run = wave_inclusive_scan_fx(sum) - sum + (s > 0 ? si[s - 1] : (fx_t)0);
+    int below = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i)
+    {
+        run += v[i];
+        below += __popcll(__ballot(i < cnt && run < r));
+    }
+    return s * CDF_SEG + below;
+}
+
+// Exact-CDF merge.  The workgroup's ancestors lie in the CDF segments [s_lo, s_hi] holding its first and
+// last draw; they are staged WSEG segments at a time (a window).  The answer is the exact lower bound in the 128-bit
+// CDF, but nearly every comparison is decided by far fewer bits: a window stages one 31-bit key per entry,
+// key(x) = floor((x - B0) 2^(30 - m)) with B0 the CDF before the window, W its exact total and m = msb(W), and
+// the draws are compared by the same key.
+//   - Weights, draws and their differences from B0 are formed in f64 in raw units (integers).  The rebuild's sums (a
+//     wave scan of one segment from its exact index entry) are off by less than 2^-48 W, a draw's
+//     difference by less than that (B0 is subtracted in two doubles), so both keys are within 1 of the exact ones
+//     and two keys at least 2 apart decide.  With W below 2^31 every value is an integer below 2^31 and the
+//     keys are exact.
+//   - A draw within 1 of an entry's key (about 3e-6 of them: a window holds at most 2048 of 2^30 keys, and draws
+//     fall in proportion to the CDF) is resolved by wave_exact_ancestor.
+//   - A window whose sums could leave the fixed-point range (a weight of 2^27 or more, or a wrapped CDF), or
+//     whose total is below 2^-66 of the CDF before it, sends all remaining draws there.
+// Draws are sorted, so the resolved ones are a prefix: the next window starts at the segment of the first draw left.
+// Bound by the vector ALU (Philox and logarithms of the draws, searches).  Before, windows held 128-bit
+// entries (four 128-bit conversions and adds per lane and segment, 128-bit scans and two-word probes).
+// 2e6 draws: 31.9 -> 22.1 us alone (3e5: 19.1 -> 15.2), 32 x 2e6 per step 3.4% off the whole step.
 template <int WSEG>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WSEG <= RS_WINDOW_NARROW ? 7 : 4)))
-void k_rs_merge_exact(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab, int pph,
-                      const fx_t* __restrict__ exp_tile_pre, const fx_t* __restrict__ seg_incl,
-                      const DevScalars* __restrict__ scs)
+__global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restrict__ descs,
+                                                          const uint32_t* __restrict__ tab, int pph,
+                                                          const fx_t* __restrict__ exp_tile_pre,
+                                                          const fx_t* __restrict__ seg_incl,
+                                                          const DevScalars* __restrict__ scs)
 {
     constexpr int WLEN = WSEG * CDF_SEG;
     constexpr int NWAVE = BLOCK / WAVE;
-    static_assert(WLEN >= RS_TILE, "the window also stages the workgroup's draws");
-    __shared__ CdfStage<fx_t, WLEN> s_cdf;
-    __shared__ fx_t s_rb[2];
-    __shared__ int s_wmin[NWAVE];
-    __shared__ fx_t s_wr[NWAVE];
+    constexpr uint32_t PAD = 0xffffffffu;  // above every draw's key
+    static_assert((WLEN & (WLEN - 1)) == 0, "the search halves the window");
+    __shared__ double s_r[RS_TILE];  // the draws in raw units
+    __shared__ __attribute__((aligned(16))) uint32_t s_key[WLEN];
+    __shared__ int s_big[NWAVE], s_done[NWAVE];
 
     const TileRef tr = tile_ref(tab, RS_TILE / UNIT, blockIdx.x);
     const VehDesc& d = descs[tr.v];
@@ -600,114 +612,159 @@ void k_rs_merge_exact(const VehDesc* __restrict__ descs, const uint32_t* __restr
         return;
     const DevScalars* sc = scs + tr.v;
     const int J = n + d.B;
-    fx_t r[RS_ITEMS];
-    merge_draws<fx_t>(d, sc, base, n, exp_tile_pre,
-                      [](fx_t s_k, const Spacing& sp) { return spacing_draw_nonneg(s_k, sp); }, s_cdf, r, s_rb);
+    const int cnt_draws = min(RS_TILE, n - base);
+    const int wid = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const Spacing sp = sc->spacing;
+    // fx(total * u_k) as a double: the product truncated to an integer number of raw units.
+    const auto raw_draw = [&sp](fx_t s_k) { return trunc(sp.total * spacing_fraction(s_k, sp) * 0x1p88); };
+    const auto draw_fx = [](double raw) { return fx_from_f64_nonneg(raw * 0x1p-88); };
+    if (d.draw_mode == DRAW_SYSTEMATIC)
+    {
+        const uint32_t u = systematic_u32(d.seed, d.inst, d.ep_rs);
+#pragma unroll
+        for (int i = 0; i < RS_ITEMS; ++i)
+            s_r[threadIdx.x + i * BLOCK] = raw_draw(systematic_s(base + (int)threadIdx.x + i * BLOCK, u));
+    }
+    else
+    {
+        spacing_prefixes(d, base, n, exp_tile_pre,
+                         [&](int i, fx_t s_k) { s_r[threadIdx.x * RS_ITEMS + i] = raw_draw(s_k); });
+    }
+    __syncthreads();
+    // Item i of a thread is draw base + threadIdx.x + i * BLOCK, so at every item a wave searches 64 consecutive draws,
+    // whose probes read neighbouring keys, and the ancestors come out wave-contiguous.
+    double r[RS_ITEMS];
+    int anc[RS_ITEMS];
+#pragma unroll
+    for (int i = 0; i < RS_ITEMS; ++i)
+    {
+        r[i] = s_r[threadIdx.x + i * BLOCK];
+        anc[i] = threadIdx.x + i * BLOCK < cnt_draws ? -1 : 0;
+    }
     const int S = (J + CDF_SEG - 1) / CDF_SEG;  // segments holding entries
     const fx_t* si = seg_incl + (size_t)(d.u0[SP_J] / SCAN_Q) * CDF_SEGS_PER_TILE;
     const auto seg_end = [si](int s) { return si[s]; };
     int s_lo, s_hi;
-    wave_find2<fx_t>(seg_end, S, s_rb[0], s_rb[1], &s_lo, &s_hi);
-    const int wid = threadIdx.x / WAVE;
-    const int lane = threadIdx.x & (WAVE - 1);
-    int anc[RS_ITEMS];
-#pragma unroll
-    for (int i = 0; i < RS_ITEMS; ++i)
-        anc[i] = -1;
-    for (int s0 = s_lo; s0 <= s_hi;)
+    wave_find2<fx_t>(seg_end, S, draw_fx(s_r[0]), draw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
+    for (int s0 = s_lo;;)
     {
         const int s1 = min(s0 + WSEG, s_hi + 1);  // window: segments [s0, s1)
         const int c0 = s0 * CDF_SEG;
         const int clen = min(J, s1 * CDF_SEG) - c0;
-        __syncthreads();  // the previous window's searches (and the draws' staging) are done
-        for (int s = s0 + wid; s < s1; s += NWAVE)
+        const fx_t B0 = s0 > 0 ? si[s0 - 1] : (fx_t)0;
+        const fx_t W = si[s1 - 1] - B0;
+        const int m = W > 0 ? 127 - clz128((ufx_t)W) : 0;
+        const int mb = B0 > 0 ? 127 - clz128((ufx_t)B0) : 0;
+        // Two doubles hold B0 exactly up to 107 bits, and to 2^-40 W while m >= mb - 66.
+        const bool odd = B0 < 0 || W < 0 || (mb > 106 && m < mb - 66);
+        const double g = ldexp(1.0, 30 - m);
+        const uint32_t margin = m <= 30 ? 0u : 1u;
+        const double b_hi = odd ? 0.0 : fx_raw_f64(B0);
+        const double b_lo = odd ? 0.0 : fx_raw_f64(B0 - draw_fx(b_hi));
+        bool big = odd;
+#pragma unroll
+        for (int q = 0; q < WSEG / NWAVE; ++q)
         {
-            const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
-            const int cnt = max(0, min(SCAN_ITEMS, J - q0));
-            float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (cnt > 0)
-                SrcJointPos{}.load4(d, q0, cnt, f);
-            fx_t v[SCAN_ITEMS];
-            fx_t sum = 0;
-#pragma unroll
-            for (int i = 0; i < SCAN_ITEMS; ++i)
+            const int s = s0 + q * NWAVE + wid;
+            uint32_t key[SCAN_ITEMS] = {PAD, PAD, PAD, PAD};
+            if (s < s1)
             {
-                v[i] = i < cnt ? fx_from_f32_nonneg(f[i]) : (fx_t)0;  // cdf_weight: sign bit clear
-                sum += v[i];
-            }
-            fx_t run = wave_inclusive_scan_fx(sum) - sum + (s > 0 ? si[s - 1] : (fx_t)0);
-            const int at = (s - s0) * CDF_SEG + lane * SCAN_ITEMS;
+                const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
+                const int cnt = max(0, min(SCAN_ITEMS, J - q0));
+                float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (cnt > 0)
+                    SrcJointPos{}.load4(d, q0, cnt, f);
+                double v[SCAN_ITEMS];
+                raw_weights(f, v);
+                double sum = v[0];
 #pragma unroll
-            for (int i = 0; i < SCAN_ITEMS; ++i)
-            {
-                run += v[i];
-                if (i < cnt)
-                    s_cdf.put(at + i, run);
+                for (int i = 1; i < SCAN_ITEMS; ++i)
+                    sum += v[i];
+                big |= fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])) >= 0x1p27f;
+                const fx_t before = s > s0 ? si[s - 1] - B0 : (fx_t)0;
+                double run = wave_inclusive_scan_val(sum) - sum + fx_raw_f64(before);
+#pragma unroll
+                for (int i = 0; i < SCAN_ITEMS; ++i)
+                {
+                    run += v[i];
+                    if (i < cnt)
+                        key[i] = (uint32_t)(run * g);
+                }
             }
+            *reinterpret_cast<uint4*>(&s_key[(q * NWAVE + wid) * CDF_SEG + lane * SCAN_ITEMS]) =
+                make_uint4(key[0], key[1], key[2], key[3]);
         }
+        const bool any_big = __ballot(big) != 0;
+        if (lane == 0)
+            s_big[wid] = any_big;
         __syncthreads();
-        const fx_t cmax = s_cdf.get(clen - 1);
-        const int span = clen > 1 ? 1 << (32 - __clz(clen - 1)) : 1;  // power of two >= clen, <= WLEN
+        bool exact = false;
+#pragma unroll
+        for (int w = 0; w < NWAVE; ++w)
+            exact |= s_big[w] != 0;
+        // Keys below rk - margin are below the draw, keys from rk + 2 margin on are not.  The thread's searches go
+        // step by step together (four LDS reads in flight).
+        uint32_t rk[RS_ITEMS], rs[RS_ITEMS];
+        int lo[RS_ITEMS];
 #pragma unroll
         for (int i = 0; i < RS_ITEMS; ++i)
         {
-            if (anc[i] < 0 && base + (int)threadIdx.x + i * BLOCK < n && !(cmax < r[i]))
+            rk[i] = (uint32_t)fmin(fmax(((r[i] - b_hi) - b_lo) * g, 0.0), 2415919104.0);
+            rs[i] = rk[i] > margin ? rk[i] - margin : 0u;
+            lo[i] = 0;
+        }
+#pragma unroll
+        for (int step = WLEN / 2; step > 0; step >>= 1)
+        {
+#pragma unroll
+            for (int i = 0; i < RS_ITEMS; ++i)
+                lo[i] += s_key[lo[i] + step - 1] < rs[i] ? step : 0;
+        }
+        int left = 0;  // bit i: draw i is to be resolved exactly
+#pragma unroll
+        for (int i = 0; i < RS_ITEMS; ++i)
+        {
+            const uint32_t at = s_key[lo[i]];
+            if (anc[i] < 0)
             {
-                // lo counts the entries < r[i]: after the probe at lo + step - 1 the count lies in
-                // [lo, lo + step).  Entries at clen and beyond count as +infinity; probing the last
-                // entry (>= r[i]) in their place gives the same answer without a branch.
-                int lo = 0;
-                for (int step = span >> 1; step > 0; step >>= 1)
-                {
-                    const int j = min(lo + step, clen) - 1;
-                    if (s_cdf.less(j, r[i]))
-                        lo += step;
-                }
-                anc[i] = c0 + lo;
+                if (exact)
+                    left |= 1 << i;
+                else if (at >= rs[i] && at < rk[i] + 2u * margin)
+                    left |= 1 << i;
+                else if (at >= rs[i] && lo[i] < clen)
+                    anc[i] = c0 + lo[i];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < RS_ITEMS; ++i)
+        {
+            uint64_t todo = __ballot((left >> i) & 1);
+            while (todo)
+            {
+                const int l = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const int a = wave_exact_ancestor(d, si, S, J, draw_fx(__shfl(r[i], l, WAVE)));
+                if (lane == l)
+                    anc[i] = a;
             }
         }
         if (s1 > s_hi)
             break;
-        // The smallest unresolved draw: each wave's minimum (draw indices are distinct, so one lane
-        // holds it) with its value, then the minimum over the waves.
-        int mine = n;
-        fx_t rmine = 0;
+        int done = 0;
 #pragma unroll
-        for (int i = RS_ITEMS - 1; i >= 0; --i)
-        {
-            const int k = base + (int)threadIdx.x + i * BLOCK;
-            if (anc[i] < 0 && k < n)
-            {
-                mine = k;
-                rmine = r[i];
-            }
-        }
-        int wmin = mine;
-#pragma unroll
-        for (int o = WAVE / 2; o > 0; o >>= 1)
-            wmin = min(wmin, __shfl_xor(wmin, o, WAVE));
-        if (wmin < n && mine == wmin)
-        {
-            s_wmin[wid] = wmin;
-            s_wr[wid] = rmine;
-        }
-        if (wmin >= n && lane == 0)
-            s_wmin[wid] = n;
-        __syncthreads();
-        int kmin = n, kw = 0;
+        for (int i = 0; i < RS_ITEMS; ++i)
+            done += __popcll(__ballot(anc[i] >= 0 && threadIdx.x + i * BLOCK < cnt_draws));
+        if (lane == 0)
+            s_done[wid] = done;
+        __syncthreads();  // also: every search of this window is done
+        done = 0;
 #pragma unroll
         for (int w = 0; w < NWAVE; ++w)
-        {
-            const int x = s_wmin[w];
-            if (x < kmin)
-            {
-                kmin = x;
-                kw = w;
-            }
-        }
-        if (kmin >= n)
+            done += s_done[w];
+        if (done >= cnt_draws)
             break;
-        const fx_t rmin = s_wr[kw];
+        const fx_t rmin = draw_fx(s_r[done]);
         const int next_last = min(s1 - 1 + WSEG, s_hi);
         if (!(si[next_last] < rmin))
         {
@@ -733,7 +790,7 @@ void k_rs_merge_float(const VehDesc* __restrict__ descs, const uint32_t* __restr
 {
     using Tr = CdfFloatTr;
     constexpr int SLICE = RS_FLOAT_SLICE_TILES * SCAN_TILE;
-    __shared__ CdfStage<double, SLICE> s_cdf;
+    __shared__ CdfStage<SLICE> s_cdf;
     __shared__ double s_rb[2];
     __shared__ int s_cnt[1];
     __shared__ int s_kmin;
@@ -747,7 +804,7 @@ void k_rs_merge_float(const VehDesc* __restrict__ descs, const uint32_t* __restr
     const DevScalars* sc = scs + tr.v;
     const int J = n + d.B;
     double r[RS_ITEMS];
-    merge_draws<double>(
+    merge_draws(
         d, sc, base, n, exp_tile_pre,
         [sc, &d](fx_t s_k, const Spacing& sp) { return Tr::draw(s_k, sp, sc, d.cdf_mode); }, s_cdf, r, s_rb);
     const int T = (J + SCAN_TILE - 1) / SCAN_TILE;
@@ -854,9 +911,9 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
     // index; the merge recomputes entries) and of the exponentials (multinomial draws) in one launch,
     // then both top-level scans in one launch.
     launch_begin(E, K_SCAN_TILES);
-    hipLaunchKernelGGL((k_scan_tiles_pair<SrcJointPos, SrcExp>), dim3(jtiles + etiles), dim3(BLOCK), 0, E->stream,
-                       SrcJointPos{}, E->tab(SP_J), jtiles, E->scan_tile_sum, E->cdf_tile_incl, SrcExp{}, E->tab(SP_E),
-                       etiles, E->exp_tile_sum, E->d_desc);
+    hipLaunchKernelGGL(k_scan_tiles_exp<SrcJointPos>, dim3(jtiles + etiles), dim3(BLOCK), 0, E->stream,
+                       SrcJointPos{}, E->tab(SP_J), jtiles, E->scan_tile_sum, E->cdf_tile_incl, E->tab(SP_E),
+                       E->exp_tile_sum, E->d_desc);
     launch_end(E, K_SCAN_TILES);
     launch_begin(E, K_SCAN_TOP);
     hipLaunchKernelGGL(k_scan_top_resample, dim3(E->m), dim3(BLOCK), 0, E->stream, E->d_desc, E->scan_tile_sum,
@@ -886,7 +943,7 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
         hipLaunchKernelGGL(k_cdff_env, dim3(E->m), dim3(ENV_BLOCK), 0, E->stream, E->d_desc, env, E->scalars);
 
     const int mt = E->tiles(SP_P, RS_TILE / UNIT);
-    const bool wide = E->tune.merge_slice == 0 ? mt <= RS_WIDE_MAX_TILES : E->tune.merge_slice == 2;
+    const bool wide = E->tune.merge_slice != 1;
     launch_begin(E, K_RS_MERGE);
     if (exact)
     {

@@ -61,6 +61,7 @@ def lib():
             "oracle_fx_from_f32_nonneg_mismatches": (C.c_int, [C.c_void_p, C.c_int]),
             "oracle_fx_from_f64_nonneg_mismatches": (C.c_int, [C.c_void_p, C.c_int]),
             "oracle_exponential_sign_violations": (C.c_int, []),
+            "oracle_exponential_unit_violations": (C.c_int, []),
             "oracle_fx_from_f64": (None, [C.c_double, C.POINTER(C.c_int64), C.POINTER(C.c_uint64)]),
             "oracle_fx_to_f32": (f, [C.c_int64, C.c_uint64]),
             "oracle_fx_to_f64": (C.c_double, [C.c_int64, C.c_uint64]),
@@ -343,6 +344,10 @@ def fx_from_f64_nonneg_mismatches(bits) -> int:
 
 def exponential_sign_violations() -> int:
     return lib().oracle_exponential_sign_violations()
+
+
+def exponential_unit_violations() -> int:
+    return lib().oracle_exponential_unit_violations()
 
 
 def fx_from_f64(v: float) -> int:

@@ -1420,6 +1420,18 @@ int oracle_exponential_sign_violations(void)
     }
     return bad;
 }
+// Of the same exponentials, those whose value in units of 2^-48 is not their fixed-point value, or too large for a
+// sum of 1024 in 64 bits.
+int oracle_exponential_unit_violations(void)
+{
+    int bad = 0;
+    for (uint32_t q = 0; q < (1u << 24); ++q)
+    {
+        const float e = -log_f32(uniform01_oc(q << 8));
+        bad += fx_from_exp_units(exp_units(e)) != fx_from_f32_nonneg(e) || exp_units(e) >= (1ull << 54);
+    }
+    return bad;
+}
 void oracle_fx_from_f64(double v, int64_t* hi, uint64_t* lo)
 {
     const fx_t r = fx_from_f64(v);

@@ -174,6 +174,11 @@ def test_resampling_exponentials_have_a_clear_sign():
     assert oc.exponential_sign_violations() == 0
 
 
+def test_resampling_exponentials_are_whole_units():
+    """All 2^24 exponentials are whole multiples of 2^-48 and equal their fixed-point value when converted as such."""
+    assert oc.exponential_unit_violations() == 0
+
+
 def test_fx_from_f32_exact():
     rng = np.random.default_rng(4)
     vals = [0.0, -0.0, 1.0, -1.0, 0.5, 1e-30, 2.0**-88, 2.0**-89, 3 * 2.0**-90, 2.0**38, -(2.0**38) * 1.5,
