@@ -135,6 +135,26 @@ __device__ __forceinline__ T wave_inclusive_max_val(T x)
     return x;
 }
 
+// Exclusive scan of one fx value per thread over NT threads (whole waves; `wid` is the wave's index in the group,
+// s_wave[NT / WAVE] the group's own LDS); returns the exclusive prefix and writes the total.  Every thread of
+// the workgroup calls it.
+template <int NT>
+__device__ __forceinline__ fx_t group_exclusive_scan_fx(fx_t v, fx_t* total, int wid, fx_t* s_wave)
+{
+    const int lane = threadIdx.x & (WAVE - 1);
+    const fx_t incl = wave_inclusive_scan_fx(v);
+    if (lane == WAVE - 1)
+        s_wave[wid] = incl;
+    __syncthreads();
+    // The waves' totals are scanned by every wave (one lane each), so no thread adds up to NT / WAVE of them.
+    const fx_t w = lane < NT / WAVE ? s_wave[lane] : (fx_t)0;
+    const fx_t wi = wave_inclusive_scan_fx(w);
+    const fx_t carry = wid > 0 ? shfl_fx(wi, wid - 1) : (fx_t)0;
+    *total = shfl_fx(wi, NT / WAVE - 1);
+    __syncthreads();
+    return carry + incl - v;
+}
+
 // Exclusive block scan of one fx value per thread (BLOCK threads); returns the exclusive prefix
 // and writes the block total.
 __device__ __forceinline__ fx_t block_exclusive_scan_fx(fx_t v, fx_t* total)
@@ -743,8 +763,8 @@ constexpr int SCAN_Q = SCAN_TILE / UNIT;  // units per scan tile
 //   __device__ int len(const VehDesc& d) const;                       // elements of the vehicle
 //   __device__ void load4(const VehDesc& d, int p0, int cnt, float (&v)[4]) const;
 // A CDF segment is one wave's share of a scan tile.  With seg_end set, the tile-local inclusive end
-// of every segment is written at seg_end[CDF_SEGS_PER_TILE * tile + segment] (k_scan_top turns
-// these into the vehicle's inclusive segment ends: the resampling CDF index).
+// of every segment is written at seg_end[CDF_SEGS_PER_TILE * tile + segment]; with the tile's prefix added (the
+// merge does that as it reads them) these are the vehicle's inclusive segment ends: the resampling CDF index.
 static_assert(CDF_SEG == WAVE * SCAN_ITEMS && CDF_SEGS_PER_TILE * CDF_SEG == SCAN_TILE, "CDF segments are waves");
 
 // The N + 1 exponentials as a scan source (tile totals only); systematic draws need none.
@@ -844,8 +864,6 @@ enum ScanMode
 {
     SCAN_ORDERS_N = 0,  // first-frame placement: scale = N / total
     SCAN_ORDERS_B = 1,  // birth placement: scale = B / total
-    SCAN_RESAMPLE = 2,  // resampling: joint_max and new weight
-    SCAN_EXP = 3,       // exponential spacings: total into exp_total
 };
 
 // Vehicle filters of the exact scans.
@@ -853,18 +871,13 @@ enum ScanOnly
 {
     ONLY_ALL = 0,
     ONLY_INIT = 1,       // vehicles initialising their particles in this step
-    ONLY_CDF_EXACT = 2,  // vehicles resampling with the exact CDF
 };
 
 __device__ __forceinline__ bool scan_takes(const VehDesc& d, int only)
 {
-    return only == ONLY_ALL || (only == ONLY_INIT && d.init) || (only == ONLY_CDF_EXACT && d.cdf_mode == CDF_EXACT);
+    return only == ONLY_ALL || (only == ONLY_INIT && d.init);
 }
 
-// One workgroup per vehicle: exclusive prefix of the vehicle's tile totals (each thread scans a
-// contiguous chunk), optionally the inclusive segment ends (tile_incl holds the tile-local ends
-// k_scan_tiles wrote; the tile's prefix is added in place), and the scalars derived from the
-// vehicle's total.  Vehicles the filter `only` excludes are skipped.
 // tile_sum holds `parts` partial sums per tile (consecutive), which are added first.
 __device__ __forceinline__ fx_t scan_tile_total(const fx_t* __restrict__ tile_sum, int t, int parts)
 {
@@ -876,102 +889,88 @@ __device__ __forceinline__ fx_t scan_tile_total(const fx_t* __restrict__ tile_su
     return s;
 }
 
-__device__ __forceinline__ void scan_top_body(const VehDesc* __restrict__ descs, int space,
-                                              const fx_t* __restrict__ tile_sum, fx_t* __restrict__ tile_pre,
-                                              fx_t* __restrict__ tile_incl, DevScalars* __restrict__ scs, int mode,
-                                              int only, int parts = 1)
+// Exclusive prefix of the ntiles tile totals from t0 on, by NT threads (thread `tid` of the group, s_wave its LDS);
+// tile_pre may be tile_sum.  Every thread of the workgroup takes part, in `rounds` rounds of
+// TOP_ITEMS consecutive tiles per thread (enough for the longest group).  Returns the total.
+constexpr int TOP_ITEMS = 4;
+
+template <int NT>
+__device__ __forceinline__ fx_t scan_tile_prefixes(const fx_t* tile_sum, fx_t* tile_pre, int t0, int ntiles, int parts,
+                                                   int tid, int rounds, fx_t* s_wave)
 {
-    const VehDesc& d = descs[blockIdx.x];
-    if (!scan_takes(d, only))
-        return;  // uniform over the workgroup
-    DevScalars* sc = scs + blockIdx.x;
-    const int t0 = d.u0[space] / SCAN_Q;
-    const int ntiles = d.nu[space] / SCAN_Q;
-    const int per = (ntiles + BLOCK - 1) / BLOCK;
-    const int b0 = t0 + min(ntiles, (int)threadIdx.x * per);
-    const int b1 = t0 + min(ntiles, (int)threadIdx.x * per + per);
-    // Chunks of four independent loads (a loop-carried load per tile would wait for each).
-    fx_t s = 0;
-    for (int tc = b0; tc < b1; tc += 4)
+    fx_t carry = 0;
+    for (int r = 0; r < rounds; ++r)
     {
-        fx_t x[4];
+        const int b = (r * NT + tid) * TOP_ITEMS;
+        fx_t x[TOP_ITEMS];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            x[k] = tc + k < b1 ? scan_tile_total(tile_sum, tc + k, parts) : (fx_t)0;
+        for (int k = 0; k < TOP_ITEMS; ++k)  // independent loads
+            x[k] = b + k < ntiles ? scan_tile_total(tile_sum, t0 + b + k, parts) : (fx_t)0;
+        fx_t s = 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < TOP_ITEMS; ++k)
             s += x[k];
-    }
-    fx_t carry;
-    fx_t run = block_exclusive_scan_fx(s, &carry);
-    for (int tc = b0; tc < b1; tc += 4)
-    {
-        fx_t x[4];
+        fx_t total;
+        fx_t run = carry + group_exclusive_scan_fx<NT>(s, &total, tid / WAVE, s_wave);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            x[k] = tc + k < b1 ? scan_tile_total(tile_sum, tc + k, parts) : (fx_t)0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < TOP_ITEMS; ++k)
         {
-            if (tc + k < b1)
-            {
-                if (tile_pre)
-                    tile_pre[tc + k] = run;
-                if (tile_incl)
-                {
-                    fx_t* se = tile_incl + (size_t)CDF_SEGS_PER_TILE * (tc + k);
-#pragma unroll
-                    for (int q = 0; q < CDF_SEGS_PER_TILE; ++q)
-                        se[q] += run;
-                }
-            }
+            if (b + k < ntiles)
+                tile_pre[t0 + b + k] = run;
             run += x[k];
         }
+        carry += total;
     }
+    return carry;
+}
+
+__device__ __forceinline__ int top_rounds(int ntiles, int nt)
+{
+    return (ntiles + nt * TOP_ITEMS - 1) / (nt * TOP_ITEMS);
+}
+
+// Particle orders of vehicle v (one workgroup of NT threads): the tile prefixes and the order scale of a scan over
+// the cells' masses.  Vehicles the filter `only` excludes are skipped.
+template <int NT>
+__device__ __forceinline__ void scan_top_orders(const VehDesc* __restrict__ descs, int v,
+                                                const fx_t* __restrict__ tile_sum, fx_t* __restrict__ tile_pre,
+                                                DevScalars* __restrict__ scs, int mode, int only, int parts)
+{
+    __shared__ fx_t s_wave[NT / WAVE];
+    const VehDesc& d = descs[v];
+    if (!scan_takes(d, only))
+        return;  // uniform over the workgroup
+    const int ntiles = d.nu[SP_C] / SCAN_Q;
+    const fx_t total = scan_tile_prefixes<NT>(tile_sum, tile_pre, d.u0[SP_C] / SCAN_Q, ntiles, parts, threadIdx.x,
+                                              top_rounds(ntiles, NT), s_wave);
     if (threadIdx.x == 0)
     {
-        if (mode == SCAN_EXP)
-        {
-            // Systematic draws do not use the exponentials: S_N = N * 2^32 (dogm_numerics.h).
-            const fx_t s_n = d.draw_mode == DRAW_SYSTEMATIC ? systematic_s(d.N, 0u) : carry;
-            sc->exp_total = s_n;
-            sc->spacing = spacing_setup(s_n, sc->total);
-            return;
-        }
-        sc->total = carry;
-        if (mode == SCAN_ORDERS_N || mode == SCAN_ORDERS_B)
-        {
-            const int v = mode == SCAN_ORDERS_N ? d.N : d.B;
-            sc->scale = carry != 0 ? order_scale(carry, v) : 0.0;
-        }
-        else
-        {
-            const float jm = fx_to_f32(carry);
-            sc->joint_max = jm;
-            sc->new_weight = jm / (float)d.N;
-        }
+        const int n = mode == SCAN_ORDERS_N ? d.N : d.B;
+        scs[v].total = total;
+        scs[v].scale = total != 0 ? order_scale(total, n) : 0.0;
     }
 }
 
+constexpr int TOP_BLOCK = 1024;
+
 template <int Unused = 0>
-__global__ __launch_bounds__(BLOCK) void k_scan_top(const VehDesc* __restrict__ descs, int space,
-                                                    const fx_t* __restrict__ tile_sum, fx_t* __restrict__ tile_pre,
-                                                    fx_t* __restrict__ tile_incl, DevScalars* __restrict__ scs,
-                                                    int mode, int only, int parts = 1)
+__global__ __launch_bounds__(TOP_BLOCK) void k_scan_top(const VehDesc* __restrict__ descs,
+                                                        const fx_t* __restrict__ tile_sum, fx_t* __restrict__ tile_pre,
+                                                        DevScalars* __restrict__ scs, int mode, int only, int parts)
 {
-    scan_top_body(descs, space, tile_sum, tile_pre, tile_incl, scs, mode, only, parts);
+    scan_top_orders<TOP_BLOCK>(descs, blockIdx.x, tile_sum, tile_pre, scs, mode, only, parts);
 }
 
 // Sink interface:
 //   __device__ void apply4(const VehDesc& d, const DevScalars* sc, int p0, int cnt,
 //                          const fx_t (&prefix)[4], const fx_t (&own)[4]) const;
 template <class Src, class Sink>
-__global__ __launch_bounds__(BLOCK) void k_scan_apply(Src src, Sink sink, const VehDesc* __restrict__ descs,
-                                                      const uint32_t* __restrict__ tab,
-                                                      const fx_t* __restrict__ tile_pre,
-                                                      const DevScalars* __restrict__ scs)
+__device__ __forceinline__ void scan_apply_body(const Src& src, const Sink& sink, const VehDesc* __restrict__ descs,
+                                                const uint32_t* __restrict__ tab, int tile,
+                                                const fx_t* __restrict__ tile_pre,
+                                                const DevScalars* __restrict__ scs)
 {
-    const TileRef tr = tile_ref(tab, SCAN_Q, blockIdx.x);
+    const TileRef tr = tile_ref(tab, SCAN_Q, tile);
     const VehDesc& d = descs[tr.v];
     if (!src.active(d))
         return;
@@ -992,7 +991,7 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(Src src, Sink sink, const 
         s += v[i];
     }
     fx_t total;
-    fx_t run = block_exclusive_scan_fx(s, &total) + tile_pre[blockIdx.x];
+    fx_t run = block_exclusive_scan_fx(s, &total) + tile_pre[tile];
     fx_t pre[SCAN_ITEMS];
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i)
@@ -1004,30 +1003,40 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(Src src, Sink sink, const 
         sink.apply4(d, scs + tr.v, p0, cnt, pre, v);
 }
 
-// unit_sums: the sources' exact sums per 256-element unit were left there by an earlier kernel of the
-// step (SCAN_Q per tile), so the tile pass is skipped.
 template <class Src, class Sink>
-inline void run_exact_scan(Engine* E, int space, const Src& src, const Sink& sink, int mode, int kid_apply,
-                           int only, fx_t* tile_incl = nullptr, const fx_t* unit_sums = nullptr)
+__global__ __launch_bounds__(BLOCK) void k_scan_apply(Src src, Sink sink, const VehDesc* __restrict__ descs,
+                                                      const uint32_t* __restrict__ tab,
+                                                      const fx_t* __restrict__ tile_pre,
+                                                      const DevScalars* __restrict__ scs)
 {
-    const int tiles = E->tiles(space, SCAN_Q);
+    scan_apply_body(src, sink, descs, tab, blockIdx.x, tile_pre, scs);
+}
+
+// Exact scan over the cells: tile totals, their prefixes and the order scale, the sink.  unit_sums: the sources' exact
+// sums per 256-cell unit were left there by an earlier kernel of the step (SCAN_Q per tile), so the tile
+// pass is skipped.
+template <class Src, class Sink>
+inline void run_exact_scan(Engine* E, const Src& src, const Sink& sink, int mode, int kid_apply, int only,
+                           const fx_t* unit_sums = nullptr)
+{
+    const int tiles = E->tiles(SP_C, SCAN_Q);
     if (tiles <= 0)
         return;
     if (!unit_sums)
     {
         launch_begin(E, K_SCAN_TILES);
-        hipLaunchKernelGGL(k_scan_tiles<Src>, dim3(tiles), dim3(BLOCK), 0, E->stream, src, E->d_desc, E->tab(space),
-                           E->scan_tile_sum, tile_incl);
+        hipLaunchKernelGGL(k_scan_tiles<Src>, dim3(tiles), dim3(BLOCK), 0, E->stream, src, E->d_desc, E->tab(SP_C),
+                           E->scan_tile_sum, (fx_t*)nullptr);
         launch_end(E, K_SCAN_TILES);
     }
     launch_begin(E, K_SCAN_TOP);
-    hipLaunchKernelGGL(k_scan_top<0>, dim3(E->m), dim3(BLOCK), 0, E->stream, E->d_desc, space,
-                       unit_sums ? unit_sums : E->scan_tile_sum, E->scan_tile_pre, tile_incl, E->scalars, mode, only,
+    hipLaunchKernelGGL(k_scan_top<0>, dim3(E->m), dim3(TOP_BLOCK), 0, E->stream, E->d_desc,
+                       unit_sums ? unit_sums : E->scan_tile_sum, E->scan_tile_pre, E->scalars, mode, only,
                        unit_sums ? SCAN_Q : 1);
     launch_end(E, K_SCAN_TOP);
     launch_begin(E, kid_apply);
     hipLaunchKernelGGL((k_scan_apply<Src, Sink>), dim3(tiles), dim3(BLOCK), 0, E->stream, src, sink, E->d_desc,
-                       E->tab(space), E->scan_tile_pre, E->scalars);
+                       E->tab(SP_C), E->scan_tile_pre, E->scalars);
     launch_end(E, kid_apply);
 }
 

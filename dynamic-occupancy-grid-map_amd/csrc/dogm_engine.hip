@@ -761,15 +761,23 @@ int engine_run(Engine* E, Vehicle* const* veh, int m, int stages)
             StageRange r("updatePersistentParticles");
             run_persistent(E, pph, occ_pers, (zero_empty & 1) != 0, pers_mom);
         }
+        // Births and moments do not depend on each other; a full step runs the moments first, with the births'
+        // single-workgroup scan beside them.
+        const bool moments_first = (stages & ST_ALL) == ST_ALL;
+        if ((stages & ST_MOMENTS) && moments_first)
+        {
+            StageRange r("statisticalMoments");
+            run_moments(E, pph, pers_mom, (zero_empty & 2) != 0, true);
+        }
         if (stages & ST_BIRTH)
         {
             StageRange r("initializeNewParticles");
-            run_births(E, occ_birth);
+            run_births(E, occ_birth, moments_first, pph);
         }
-        if (stages & ST_MOMENTS)
+        if ((stages & ST_MOMENTS) && !moments_first)
         {
             StageRange r("statisticalMoments");
-            run_moments(E, pph, pers_mom, (zero_empty & 2) != 0);
+            run_moments(E, pph, pers_mom, (zero_empty & 2) != 0, false);
         }
     }
     if (stages & ST_RESAMPLE)

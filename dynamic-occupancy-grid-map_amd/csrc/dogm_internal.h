@@ -163,14 +163,12 @@ struct VehDesc
 // Scalars produced and consumed on the device within one step, one per vehicle.
 struct DevScalars
 {
-    fx_t total;        // last exact scan total (particle orders or resampling CDF)
-    fx_t exp_total;    // resampling: sum of the N + 1 exponentials
-    dogm_num::Spacing spacing;  // resampling: draw mapping derived from exp_total and total
+    fx_t total;        // exact total of the cells' masses (particle orders)
+    fx_t cdf_total;    // resampling: exact CDF total
+    dogm_num::Spacing spacing;  // resampling: draw mapping derived from the totals of exponentials and CDF
     double scale;      // particle-order scale v / total
     double ftotal;     // resampling, float CDF modes: the CDF total (envelope maximum)
-    float joint_max;   // resampling: f32 of the CDF total
-    float new_weight;  // resampling: joint_max / N
-    int pad[2];
+    float new_weight;  // resampling: f32 of the CDF total over N
 };
 
 // Per-tile carry of the exact segmented reductions.
@@ -414,8 +412,8 @@ struct Engine
     fx_t* scan_tile_sum = nullptr;
     fx_t* scan_tile_pre = nullptr;
     fx_t* exp_tile_sum = nullptr;  // resampling: the exponentials' tile totals (scanned beside the CDF's)
-    // Resampling CDF index: exact mode, the inclusive end of every CDF segment (CDF_SEGS_PER_TILE
-    // per scan tile); float modes, two doubles per scan tile (envelope at the end and before it).
+    // Resampling CDF index: exact mode, the tile-local inclusive end of every CDF segment (CDF_SEGS_PER_TILE
+    // per scan tile; scan_tile_sum holds the tiles' prefixes); float modes, two doubles per scan tile (envelope at the end and before it).
     fx_t* cdf_tile_incl = nullptr;
     long long seg_tiles_cap = 0;
     SegCarry seg{};
@@ -593,12 +591,16 @@ void run_assignment(Engine* E, int pph, bool hist_done, bool defer_bounds, bool 
 void run_occupancy(Engine* E, int pph, int zero_empty, bool defer_normalize, bool bounds, bool born_sums,
                    bool exp_sums);  // free[0] -> free[1]
 void run_persistent(Engine* E, int pph, bool fused_normalize, bool empty_done, bool defer_post);
-void run_births(Engine* E, bool born_sums);
+// moments_first (full steps, after run_moments with births_top): the birth orders' top-level scan has run, and
+// the launch of the birth cells also sums the moments of cells crossing chunks.
+void run_births(Engine* E, bool born_sums, bool moments_first, int pph);
 // Unit sums of the born masses between the occupancy update and the births of a step: the CDF index
 // buffer (SCAN_Q units per scan tile fit its CDF_SEGS_PER_TILE entries per tile), unused until the
 // resampling.
 inline fx_t* born_unit_sums(Engine* E) { return E->cdf_tile_incl; }
-void run_moments(Engine* E, int pph, bool fused_post, bool empty_done);
+// births_top: the top-level scan of the birth orders (over the occupancy update's unit sums) runs in workgroups of
+// the moments' launch, and cells crossing chunks are left to the births' launch.
+void run_moments(Engine* E, int pph, bool fused_post, bool empty_done, bool births_top);
 // modes: bit m set when a vehicle of the step resamples with CDF mode m (dogm_num::CdfMode).
 void run_resampling(Engine* E, int pph, int modes, bool exp_done);  // reads pph, writes pph ^ 1
 // Flags of the gathering sort pass.

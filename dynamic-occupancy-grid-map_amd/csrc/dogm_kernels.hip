@@ -1105,20 +1105,6 @@ __global__ __launch_bounds__(BLOCK) void k_birth_particles(const VehDesc* __rest
     d.birth.assoc[k] = assoc ? 1 : 0;
 }
 
-void run_births(Engine* E, bool born_sums)
-{
-    // With B = 0 the cell pass still runs (every cell gets n_j = 0 and w_A = w_UA = 0) and the
-    // stage still consumes its RNG epoch, so the stream of later stages does not depend on B.
-    run_exact_scan(E, SP_C, SrcBorn{0}, SinkBirth{}, SCAN_ORDERS_B, K_BIRTH_CELLS, ONLY_ALL, nullptr,
-                   born_sums ? born_unit_sums(E) : nullptr);
-    const int blocks = E->tiles(SP_B, 1);
-    if (blocks <= 0)
-        return;
-    launch_begin(E, K_BIRTH_PARTICLES);
-    hipLaunchKernelGGL(k_birth_particles, dim3(blocks), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_B));
-    launch_end(E, K_BIRTH_PARTICLES);
-}
-
 // ---------------------------------------------------------------------------------------------
 // First-measurement initialisation (dogm/src/dogm.cu:217-241, init_new_particles.cu:76-124),
 // for the vehicles of the step whose descriptor has `init` set.
@@ -1158,7 +1144,7 @@ void run_init_particles(Engine* E)
     launch_begin(E, K_COPY_MASSES);
     hipLaunchKernelGGL(k_copy_masses, dim3(E->tiles(SP_C, 1)), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_C));
     launch_end(E, K_COPY_MASSES);
-    run_exact_scan(E, SP_C, SrcBorn{1}, SinkOrders{}, SCAN_ORDERS_N, K_INIT_CELLS, ONLY_INIT);
+    run_exact_scan(E, SrcBorn{1}, SinkOrders{}, SCAN_ORDERS_N, K_INIT_CELLS, ONLY_INIT);
     launch_begin(E, K_INIT_PARTICLES);
     hipLaunchKernelGGL(k_init_particles, dim3(E->tiles(SP_P, 1)), dim3(BLOCK), 0, E->stream, E->d_desc,
                        E->tab(SP_P));
@@ -1219,6 +1205,16 @@ __device__ __forceinline__ int dpp_i(int x)
 
 // carry.flags[unit], and per unit MOM_CH doubles in carry.head_partial (piece of the chunk's first
 // cell when that cell started in an earlier chunk) and carry.tail_partial (piece of its last cell).
+// The first `top` workgroups (full steps) scan the birth orders, one vehicle each: single-workgroup latency (12 us at
+// 1200 x 1200 cells) beside the particle work instead of in a launch of its own.
+struct BirthTop
+{
+    int m;                  // vehicles
+    const fx_t* unit_sums;  // born masses per cell unit
+    fx_t* tile_pre;
+    DevScalars* scalars;
+};
+
 // CELLS: the vehicles with per-cell weights (their records hold the posterior weights, so no prior or
 // likelihood weights are read: 16 N instead of 24 N); else the others.  Bound by the latency of the cell
 // records and of the f64 scans: 19.5 us at 2e6 particles with six waves per SIMD and no spills, 20.6 with seven
@@ -1226,10 +1222,18 @@ __device__ __forceinline__ int dpp_i(int x)
 template <int WAVES_PER_WG, bool CELLS>
 __global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per_eu(CELLS ? 6 : 7)))
 void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab, int pph, int post,
-               SegCarry carry)
+               SegCarry carry, int top, BirthTop births)
 {
+    if ((int)blockIdx.x < top)
+    {
+        if ((int)blockIdx.x < births.m)
+            scan_top_orders<WAVES_PER_WG * WAVE>(descs, blockIdx.x, births.unit_sums, births.tile_pre, births.scalars,
+                                                 SCAN_ORDERS_B, ONLY_ALL, SCAN_Q);
+        return;
+    }
     const int lane = threadIdx.x & (WAVE - 1);
-    const int unit = xcd_tile(blockIdx.x, gridDim.x) * WAVES_PER_WG + (int)threadIdx.x / WAVE;
+    const int unit =
+        xcd_tile((int)blockIdx.x - top, (int)gridDim.x - top) * WAVES_PER_WG + (int)threadIdx.x / WAVE;
     const TileRef tr = tile_ref(tab, 1, unit);
     const VehDesc& d = descs[tr.v];
     if (CELLS != (d.wcell != 0))
@@ -1416,12 +1420,10 @@ void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ t
     }
 }
 
-// Cells crossing chunks: one thread per chunk whose last cell starts in it and continues.
-__global__ __launch_bounds__(BLOCK) void k_moments_fix(const VehDesc* __restrict__ descs,
-                                                       const uint32_t* __restrict__ tab, int units, int pph,
-                                                       SegCarry carry)
+// Cells crossing chunks: one thread per chunk u whose last cell starts in it and continues.
+__device__ __forceinline__ void moments_fix_chunk(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab,
+                                                  int u, int units, int pph, const SegCarry& carry)
 {
-    const int u = blockIdx.x * BLOCK + threadIdx.x;
     if (u >= units)
         return;
     const uint8_t fl = carry.flags[u];
@@ -1451,26 +1453,43 @@ __global__ __launch_bounds__(BLOCK) void k_moments_fix(const VehDesc* __restrict
     mom_finalize(d, key, d.f[GF_PERS][key], s);
 }
 
-constexpr int MOM_WAVES_PER_WG = 4;
+__global__ __launch_bounds__(BLOCK) void k_moments_fix(const VehDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ tab, int units, int pph,
+                                                       SegCarry carry)
+{
+    moments_fix_chunk(descs, tab, blockIdx.x * BLOCK + threadIdx.x, units, pph, carry);
+}
 
-void run_moments(Engine* E, int pph, bool fused_post, bool empty_done)
+constexpr int MOM_WAVES_PER_WG = 4;
+static_assert(MOM_WAVES_PER_WG * WAVE == BLOCK, "the births' scan shares the moments' launch");
+
+void run_moments(Engine* E, int pph, bool fused_post, bool empty_done, bool births_top)
 {
     const int units = (int)E->units[SP_P];
     if (units > 0)
     {
-        const dim3 grid(units / MOM_WAVES_PER_WG), block(MOM_WAVES_PER_WG * WAVE);
+        // The scan's workgroups come first (they are the longest), padded to whole rounds of the 8 XCDs.
+        int top = births_top ? div_up(E->m, 8) * 8 : 0;
+        const BirthTop bt{E->m, born_unit_sums(E), E->scan_tile_pre, E->scalars};
+        const dim3 block(MOM_WAVES_PER_WG * WAVE);
         launch_begin(E, K_SEG_MOM);
         if (E->any_wcell)
-            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, true>), grid, block, 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, 1, E->seg);
+        {
+            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, true>), dim3(top + units / MOM_WAVES_PER_WG), block, 0,
+                               E->stream, E->d_desc, E->tab(SP_P), pph, 1, E->seg, top, bt);
+            top = 0;
+        }
         if (E->any_general)
-            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, false>), grid, block, 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, fused_post ? 1 : 0, E->seg);
+            hipLaunchKernelGGL((k_moments<MOM_WAVES_PER_WG, false>), dim3(top + units / MOM_WAVES_PER_WG), block, 0,
+                               E->stream, E->d_desc, E->tab(SP_P), pph, fused_post ? 1 : 0, E->seg, top, bt);
         launch_end(E, K_SEG_MOM);
-        launch_begin(E, K_SEG_MOM_FIX);
-        hipLaunchKernelGGL(k_moments_fix, dim3(div_up(units, BLOCK)), dim3(BLOCK), 0, E->stream, E->d_desc,
-                           E->tab(SP_P), units, pph, E->seg);
-        launch_end(E, K_SEG_MOM_FIX);
+        if (!births_top)
+        {
+            launch_begin(E, K_SEG_MOM_FIX);
+            hipLaunchKernelGGL(k_moments_fix, dim3(div_up(units, BLOCK)), dim3(BLOCK), 0, E->stream, E->d_desc,
+                               E->tab(SP_P), units, pph, E->seg);
+            launch_end(E, K_SEG_MOM_FIX);
+        }
     }
     if (empty_done)
         return;
@@ -1478,6 +1497,46 @@ void run_moments(Engine* E, int pph, bool fused_post, bool empty_done)
     hipLaunchKernelGGL(k_empty_cells, dim3(E->tiles(SP_C, 1)), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_C),
                        (int)GF_MEAN_X, (int)GF_COVAR);
     launch_end(E, K_EMPTY_CELLS);
+}
+
+// The birth cells of a full step, and in the workgroups after the `tiles` cell tiles the moments of cells crossing
+// chunks (both wait for the moments' launch only; as a launch of its own the latter took 4 to 5 us).
+__global__ __launch_bounds__(BLOCK) void k_birth_cells(const VehDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ tab_c, int tiles,
+                                                       const fx_t* __restrict__ tile_pre,
+                                                       const DevScalars* __restrict__ scs,
+                                                       const uint32_t* __restrict__ tab_p, int units, int pph,
+                                                       SegCarry carry)
+{
+    if ((int)blockIdx.x < tiles)
+        scan_apply_body(SrcBorn{0}, SinkBirth{}, descs, tab_c, blockIdx.x, tile_pre, scs);
+    else
+        moments_fix_chunk(descs, tab_p, ((int)blockIdx.x - tiles) * BLOCK + (int)threadIdx.x, units, pph, carry);
+}
+
+void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
+{
+    // With B = 0 the cell pass still runs (every cell gets n_j = 0 and w_A = w_UA = 0) and the
+    // stage still consumes its RNG epoch, so the stream of later stages does not depend on B.
+    if (moments_first)
+    {
+        const int tiles = E->tiles(SP_C, SCAN_Q), units = (int)E->units[SP_P];
+        launch_begin(E, K_BIRTH_CELLS);
+        hipLaunchKernelGGL(k_birth_cells, dim3(tiles + div_up(units, BLOCK)), dim3(BLOCK), 0, E->stream, E->d_desc,
+                           E->tab(SP_C), tiles, E->scan_tile_pre, E->scalars, E->tab(SP_P), units, pph, E->seg);
+        launch_end(E, K_BIRTH_CELLS);
+    }
+    else
+    {
+        run_exact_scan(E, SrcBorn{0}, SinkBirth{}, SCAN_ORDERS_B, K_BIRTH_CELLS, ONLY_ALL,
+                       born_sums ? born_unit_sums(E) : nullptr);
+    }
+    const int blocks = E->tiles(SP_B, 1);
+    if (blocks <= 0)
+        return;
+    launch_begin(E, K_BIRTH_PARTICLES);
+    hipLaunchKernelGGL(k_birth_particles, dim3(blocks), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_B));
+    launch_end(E, K_BIRTH_PARTICLES);
 }
 
 // ---------------------------------------------------------------------------------------------

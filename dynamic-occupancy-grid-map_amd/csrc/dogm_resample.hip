@@ -34,6 +34,9 @@ constexpr int RS_FLOAT_SLICE_TILES = 2;
 // spaced like the exact mode's segment ends so that vehicles of both kinds in one step keep
 // disjoint index ranges.
 constexpr int ENV_STRIDE = 2 * CDF_SEGS_PER_TILE;
+// Doubles per scan tile in the float modes' tile totals, which lie in scan_tile_sum beside the exact
+// vehicles' fixed-point prefixes.
+constexpr int FSUM_STRIDE = sizeof(fx_t) / sizeof(double);
 
 static_assert(RS_TILE == SCAN_TILE, "draw tiles and CDF tiles share the exact-scan tile size");
 
@@ -179,7 +182,7 @@ __global__ __launch_bounds__(BLOCK) void k_cdff_tiles(const VehDesc* __restrict_
     T carry, ex, tot;
     tile_float_scan<T>(d, p0, cnt, loc, &carry, &ex, &tot);
     if (threadIdx.x == 0)
-        tile_sum[blockIdx.x] = (double)tot;
+        tile_sum[FSUM_STRIDE * (size_t)blockIdx.x] = (double)tot;
 }
 
 // One workgroup per vehicle: sequential prefix over the vehicle's tile totals (the association of the float
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(BLOCK) void k_cdff_top(const VehDesc* __restrict__ 
         const int len = min(CHUNK, nt - c);
         __syncthreads();
         for (int i = threadIdx.x; i < CHUNK; i += BLOCK)
-            s_x[i] = i < len ? tile_sum[t0 + c + i] : 0.0;
+            s_x[i] = i < len ? tile_sum[FSUM_STRIDE * (size_t)(t0 + c + i)] : 0.0;
         __syncthreads();
         if (threadIdx.x == 0)
         {
@@ -351,7 +354,6 @@ __global__ __launch_bounds__(ENV_BLOCK) void k_cdff_env(const VehDesc* __restric
         DevScalars* sc = scs + v;
         sc->ftotal = total;
         const float jm = (float)total;
-        sc->joint_max = jm;
         sc->new_weight = jm / (float)d.N;
     }
 }
@@ -539,14 +541,42 @@ __device__ __forceinline__ void raw_weights(const float (&f)[SCAN_ITEMS], double
         v[i] = trunc((double)f[i] * 0x1p88);
 }
 
+// The CDF index of a vehicle: the inclusive CDF value at the end of segment s, from the tile-local ends of
+// the tile pass and the tiles' prefixes.
+struct SegEnds
+{
+    const fx_t* local;     // [segments]
+    const fx_t* tile_pre;  // [tiles]
+    fx_t total;
+    int tiles, segs;       // tiles and segments holding entries
+    __device__ fx_t operator()(int s) const { return local[s] + tile_pre[s / CDF_SEGS_PER_TILE]; }
+
+    // The first segments whose end is >= r0 and >= r1 (the last segment if none), by one wave without a barrier: a
+    // search over the tile ends (each the next tile's prefix), then the ends inside the two tiles.
+    __device__ void find2(fx_t r0, fx_t r1, int* s0, int* s1) const
+    {
+        const int lane = threadIdx.x & (WAVE - 1);
+        const auto tile_end = [this](int t) { return t + 1 < tiles ? tile_pre[t + 1] : total; };
+        int t0, t1;
+        wave_find2<fx_t>(tile_end, tiles, r0, r1, &t0, &t1);
+        // lanes 0 .. 3 hold the segment ends of tile t0, lanes 4 .. 7 those of t1
+        const bool second = lane >= CDF_SEGS_PER_TILE;
+        const int s = min((second ? t1 : t0) * CDF_SEGS_PER_TILE + (lane & (CDF_SEGS_PER_TILE - 1)), segs - 1);
+        const uint64_t below = __ballot((*this)(s) < (second ? r1 : r0));
+        *s0 = min(t0 * CDF_SEGS_PER_TILE + __popcll(below & 0xfull), segs - 1);
+        *s1 = min(t1 * CDF_SEGS_PER_TILE + __popcll(below & 0xf0ull), segs - 1);
+    }
+};
+static_assert(CDF_SEGS_PER_TILE == 4, "find2 tests a tile's segments with four lanes");
+
 // First joint entry whose exact CDF value is >= r, by one wave: the coarse index gives the segment, the
 // segment's entries are rebuilt exactly (the 64 lanes' four weights in fixed point, a 64-lane exact scan and the
 // index entry before the segment) and those below r counted.
-__device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const fx_t* __restrict__ si, int S, int J, fx_t r)
+__device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const SegEnds& seg_end, int J, fx_t r)
 {
     const int lane = threadIdx.x & (WAVE - 1);
     int s, unused;
-    wave_find2<fx_t>([si](int k) { return si[k]; }, S, r, r, &s, &unused);
+    seg_end.find2(r, r, &s, &unused);
     const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
     const int cnt = max(0, min(SCAN_ITEMS, J - q0));
     float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -560,7 +590,7 @@ __device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const fx_t*
         v[i] = i < cnt ? fx_from_f32_nonneg(f[i]) : (fx_t)0;  // cdf_weight: sign bit clear
         sum += v[i];
     }
-    fx_t run = wave_inclusive_scan_fx(sum) - sum + (s > 0 ? si[s - 1] : (fx_t)0);
+    fx_t run = wave_inclusive_scan_fx(sum) - sum + (s > 0 ? seg_end(s - 1) : (fx_t)0);
     int below = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; ++i)
@@ -593,7 +623,8 @@ template <int WSEG>
 __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ tab, int pph,
                                                           const fx_t* __restrict__ exp_tile_pre,
-                                                          const fx_t* __restrict__ seg_incl,
+                                                          const fx_t* __restrict__ seg_local,
+                                                          const fx_t* __restrict__ cdf_pre,
                                                           const DevScalars* __restrict__ scs)
 {
     constexpr int WLEN = WSEG * CDF_SEG;
@@ -601,7 +632,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     constexpr uint32_t PAD = 0xffffffffu;  // above every draw's key
     static_assert((WLEN & (WLEN - 1)) == 0, "the search halves the window");
     __shared__ double s_r[RS_TILE];  // the draws in raw units
-    __shared__ __attribute__((aligned(16))) uint32_t s_key[WLEN];
+    __shared__ __attribute__((aligned(16))) uint32_t s_key[WLEN];  // keys + margin
     __shared__ int s_big[NWAVE], s_done[NWAVE];
 
     const TileRef tr = tile_ref(tab, RS_TILE / UNIT, blockIdx.x);
@@ -634,26 +665,22 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     __syncthreads();
     // Item i of a thread is draw base + threadIdx.x + i * BLOCK, so at every item a wave searches 64 consecutive draws,
     // whose probes read neighbouring keys, and the ancestors come out wave-contiguous.
-    double r[RS_ITEMS];
     int anc[RS_ITEMS];
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
-    {
-        r[i] = s_r[threadIdx.x + i * BLOCK];
         anc[i] = threadIdx.x + i * BLOCK < cnt_draws ? -1 : 0;
-    }
-    const int S = (J + CDF_SEG - 1) / CDF_SEG;  // segments holding entries
-    const fx_t* si = seg_incl + (size_t)(d.u0[SP_J] / SCAN_Q) * CDF_SEGS_PER_TILE;
-    const auto seg_end = [si](int s) { return si[s]; };
+    const int t0 = d.u0[SP_J] / SCAN_Q;
+    const SegEnds seg_end{seg_local + (size_t)t0 * CDF_SEGS_PER_TILE, cdf_pre + t0, sc->cdf_total,
+                          (J + SCAN_TILE - 1) / SCAN_TILE, (J + CDF_SEG - 1) / CDF_SEG};
     int s_lo, s_hi;
-    wave_find2<fx_t>(seg_end, S, draw_fx(s_r[0]), draw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
+    seg_end.find2(draw_fx(s_r[0]), draw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
     for (int s0 = s_lo;;)
     {
         const int s1 = min(s0 + WSEG, s_hi + 1);  // window: segments [s0, s1)
         const int c0 = s0 * CDF_SEG;
         const int clen = min(J, s1 * CDF_SEG) - c0;
-        const fx_t B0 = s0 > 0 ? si[s0 - 1] : (fx_t)0;
-        const fx_t W = si[s1 - 1] - B0;
+        const fx_t B0 = s0 > 0 ? seg_end(s0 - 1) : (fx_t)0;
+        const fx_t W = seg_end(s1 - 1) - B0;
         const int m = W > 0 ? 127 - clz128((ufx_t)W) : 0;
         const int mb = B0 > 0 ? 127 - clz128((ufx_t)B0) : 0;
         // Two doubles hold B0 exactly up to 107 bits, and to 2^-40 W while m >= mb - 66.
@@ -682,14 +709,14 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
                 for (int i = 1; i < SCAN_ITEMS; ++i)
                     sum += v[i];
                 big |= fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])) >= 0x1p27f;
-                const fx_t before = s > s0 ? si[s - 1] - B0 : (fx_t)0;
+                const fx_t before = s > s0 ? seg_end(s - 1) - B0 : (fx_t)0;
                 double run = wave_inclusive_scan_val(sum) - sum + fx_raw_f64(before);
 #pragma unroll
                 for (int i = 0; i < SCAN_ITEMS; ++i)
                 {
                     run += v[i];
                     if (i < cnt)
-                        key[i] = (uint32_t)(run * g);
+                        key[i] = (uint32_t)(run * g) + margin;
                 }
             }
             *reinterpret_cast<uint4*>(&s_key[(q * NWAVE + wid) * CDF_SEG + lane * SCAN_ITEMS]) =
@@ -703,15 +730,14 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
 #pragma unroll
         for (int w = 0; w < NWAVE; ++w)
             exact |= s_big[w] != 0;
-        // Keys below rk - margin are below the draw, keys from rk + 2 margin on are not.  The thread's searches go
-        // step by step together (four LDS reads in flight).
-        uint32_t rk[RS_ITEMS], rs[RS_ITEMS];
+        // Keys below rk - margin (staged: below rk) are below the draw, keys from rk + 2 margin on are not.  The
+        // thread's searches go step by step together (four LDS reads in flight).
+        uint32_t rk[RS_ITEMS];
         int lo[RS_ITEMS];
 #pragma unroll
         for (int i = 0; i < RS_ITEMS; ++i)
         {
-            rk[i] = (uint32_t)fmin(fmax(((r[i] - b_hi) - b_lo) * g, 0.0), 2415919104.0);
-            rs[i] = rk[i] > margin ? rk[i] - margin : 0u;
+            rk[i] = (uint32_t)fmin(fmax(((s_r[threadIdx.x + i * BLOCK] - b_hi) - b_lo) * g, 0.0), 2415919104.0);
             lo[i] = 0;
         }
 #pragma unroll
@@ -719,7 +745,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
         {
 #pragma unroll
             for (int i = 0; i < RS_ITEMS; ++i)
-                lo[i] += s_key[lo[i] + step - 1] < rs[i] ? step : 0;
+                lo[i] += s_key[lo[i] + step - 1] < rk[i] ? step : 0;
         }
         int left = 0;  // bit i: draw i is to be resolved exactly
 #pragma unroll
@@ -730,9 +756,9 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             {
                 if (exact)
                     left |= 1 << i;
-                else if (at >= rs[i] && at < rk[i] + 2u * margin)
+                else if (at >= rk[i] && at < rk[i] + 3u * margin)
                     left |= 1 << i;
-                else if (at >= rs[i] && lo[i] < clen)
+                else if (at >= rk[i] && lo[i] < clen)
                     anc[i] = c0 + lo[i];
             }
         }
@@ -744,7 +770,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             {
                 const int l = __builtin_ctzll(todo);
                 todo &= todo - 1;
-                const int a = wave_exact_ancestor(d, si, S, J, draw_fx(__shfl(r[i], l, WAVE)));
+                const int a = wave_exact_ancestor(d, seg_end, J, draw_fx(s_r[wid * WAVE + l + i * BLOCK]));
                 if (lane == l)
                     anc[i] = a;
             }
@@ -766,14 +792,14 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             break;
         const fx_t rmin = draw_fx(s_r[done]);
         const int next_last = min(s1 - 1 + WSEG, s_hi);
-        if (!(si[next_last] < rmin))
+        if (!(seg_end(next_last) < rmin))
         {
             s0 = s1;
         }
         else
         {
             int c, unused;
-            wave_find2<fx_t>(seg_end, S, rmin, rmin, &c, &unused);
+            seg_end.find2(rmin, rmin, &c, &unused);
             s0 = max(s1, c);
         }
     }
@@ -857,9 +883,6 @@ void k_rs_merge_float(const VehDesc* __restrict__ descs, const uint32_t* __restr
     merge_write(d, sc, pph, base, n, J, anc);
 }
 
-// The resampling's two top-level scans in one launch, in their order (the spacings read the CDF
-// total): the joint CDF of exact-CDF vehicles (segment ends in place, no tile prefixes), then the
-// exponentials of every vehicle (tile prefixes into exp_pre).
 // Writes out a deferred resampled set (see merge_write): particle k of dst copied from its ancestor
 // (particle anc[k] of src below n, birth particle anc[k] - n above) with the new weight, which the
 // resampling left in dst.weight[0].
@@ -891,15 +914,44 @@ void run_materialize(Engine* E, const Vehicle* v)
     launch_end(E, K_MATERIALIZE);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_scan_top_resample(const VehDesc* __restrict__ descs,
-                                                             const fx_t* __restrict__ cdf_sum,
-                                                             fx_t* __restrict__ cdf_incl,
-                                                             const fx_t* __restrict__ exp_sum,
-                                                             fx_t* __restrict__ exp_pre, DevScalars* __restrict__ scs)
+// One workgroup per vehicle: half of its waves scan the joint CDF's tile totals (exact-CDF vehicles; prefixes in
+// place), the other half the exponentials' (prefixes into exp_pre), then one thread derives the draws'
+// mapping from both totals.  Bound by latency: a few dependent rounds of loads and 128-bit scans on one CU
+// per vehicle.  2148 + 1954 tiles (2e6 particles): 20 us with one 256-thread workgroup doing both in turn
+// and adding the prefixes into the four segment ends per tile, 8.4 us so.
+__global__ __launch_bounds__(TOP_BLOCK) void k_scan_top_resample(const VehDesc* __restrict__ descs,
+                                                                 fx_t* __restrict__ cdf_sum,
+                                                                 const fx_t* __restrict__ exp_sum,
+                                                                 fx_t* __restrict__ exp_pre,
+                                                                 DevScalars* __restrict__ scs)
 {
-    scan_top_body(descs, SP_J, cdf_sum, (fx_t*)nullptr, cdf_incl, scs, SCAN_RESAMPLE, ONLY_CDF_EXACT);
+    constexpr int HALF = TOP_BLOCK / 2;
+    __shared__ fx_t s_wave[2][HALF / WAVE];
+    __shared__ fx_t s_total[2];
+    const VehDesc& d = descs[blockIdx.x];
+    const int half = threadIdx.x / HALF, tid = threadIdx.x % HALF;
+    const int nj = d.cdf_mode == CDF_EXACT ? d.nu[SP_J] / SCAN_Q : 0;
+    const int ne = d.draw_mode == DRAW_MULTINOMIAL ? d.nu[SP_E] / SCAN_Q : 0;
+    const int rounds = max(top_rounds(nj, HALF), top_rounds(ne, HALF));
+    const fx_t total = scan_tile_prefixes<HALF>(half ? exp_sum : cdf_sum, half ? exp_pre : cdf_sum,
+                                                half ? d.u0[SP_E] / SCAN_Q : d.u0[SP_J] / SCAN_Q, half ? ne : nj, 1, tid,
+                                                rounds, s_wave[half]);
+    if (tid == 0)
+        s_total[half] = total;
     __syncthreads();
-    scan_top_body(descs, SP_E, exp_sum, exp_pre, (fx_t*)nullptr, scs, SCAN_EXP, ONLY_ALL);
+    if (threadIdx.x == 0)
+    {
+        DevScalars* sc = scs + blockIdx.x;
+        const fx_t cdf_total = s_total[0];
+        // Systematic draws do not use the exponentials: S_N = N * 2^32 (dogm_numerics.h).
+        sc->spacing = spacing_setup(ne ? s_total[1] : systematic_s(d.N, 0u), cdf_total);
+        sc->cdf_total = cdf_total;
+        if (nj)
+        {
+            const float jm = fx_to_f32(cdf_total);
+            sc->new_weight = jm / (float)d.N;
+        }
+    }
 }
 
 void run_resampling(Engine* E, int pph, int modes, bool exp_done)
@@ -916,11 +968,11 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
                        E->exp_tile_sum, E->d_desc);
     launch_end(E, K_SCAN_TILES);
     launch_begin(E, K_SCAN_TOP);
-    hipLaunchKernelGGL(k_scan_top_resample, dim3(E->m), dim3(BLOCK), 0, E->stream, E->d_desc, E->scan_tile_sum,
-                       E->cdf_tile_incl, E->exp_tile_sum, E->scan_tile_pre, E->scalars);
+    hipLaunchKernelGGL(k_scan_top_resample, dim3(E->m), dim3(TOP_BLOCK), 0, E->stream, E->d_desc, E->scan_tile_sum,
+                       E->exp_tile_sum, E->scan_tile_pre, E->scalars);
     launch_end(E, K_SCAN_TOP);
-    // Float modes: tile totals and prefixes as doubles in the two consumed total buffers (the
-    // exponentials' prefixes stay in scan_tile_pre for the merge).
+    // Float modes: tile totals as doubles in scan_tile_sum (each in its tile's own entry), prefixes in the consumed
+    // exponential totals (the exponentials' prefixes stay in scan_tile_pre for the merge).
     double* tsum = reinterpret_cast<double*>(E->scan_tile_sum);
     double* tpre = reinterpret_cast<double*>(E->exp_tile_sum);
     double* env = reinterpret_cast<double*>(E->cdf_tile_incl);
@@ -949,10 +1001,10 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
     {
         if (wide)
             hipLaunchKernelGGL(k_rs_merge_exact<RS_WINDOW_WIDE>, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scalars);
+                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars);
         else
             hipLaunchKernelGGL(k_rs_merge_exact<RS_WINDOW_NARROW>, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scalars);
+                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars);
     }
     if (modes & ~(1 << CDF_EXACT))
         hipLaunchKernelGGL(k_rs_merge_float, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_P), pph,
