@@ -180,6 +180,13 @@ __device__ __forceinline__ fx_t block_exclusive_scan_fx(fx_t v, fx_t* total)
     return carry + incl - v;
 }
 
+// The wave's index in the workgroup as a scalar: what is found from it (work-table entries, descriptors, their array
+// pointers) then stays in scalar registers and scalar loads instead of one copy per lane.
+__device__ __forceinline__ int wave_index()
+{
+    return __builtin_amdgcn_readfirstlane((int)threadIdx.x / WAVE);
+}
+
 // Stores of streaming outputs, which no later work of the same launch reads and which are far out of
 // the caches by the time the next stage reads them: vector stores with the nontemporal hint.
 template <class T>

@@ -158,6 +158,9 @@ struct VehDesc
     // whether they describe the grid in memory (see Vehicle::nz_valid).
     unsigned long long* nz;
     int nz_valid;
+    // Per 64 cells: one of them had birth slots at the last full update (so w_A or w_UA may be non-zero);
+    // describes the grid in memory while nz_valid holds.
+    uint8_t* bu;
 };
 
 // Scalars produced and consumed on the device within one step, one per vehicle.
@@ -169,7 +172,11 @@ struct DevScalars
     double scale;      // particle-order scale v / total
     double ftotal;     // resampling, float CDF modes: the CDF total (envelope maximum)
     float new_weight;  // resampling: f32 of the CDF total over N
+    int born_odd;      // a born mass of this step is negative, NaN or above BORN_MAX (k_mass_update)
 };
+
+// Born masses up to this sum to less than the fixed-point range over any grid (2^28 cells).
+constexpr float BORN_MAX = 1024.0f;
 
 // Per-tile carry of the exact segmented reductions.
 constexpr int SEG_TAIL_CONT = 1;  // tile's last segment continues into the next tile
@@ -296,6 +303,7 @@ struct Vehicle
     // those fields (stage-by-stage steps, eager shifts and rotations, grid-cell injection) clears
     // nz_valid, and the next full update rewrites every cell.
     unsigned long long* nz = nullptr;
+    uint8_t* bu = nullptr;  // 64-cell groups with birth slots at the last full update (see VehDesc::bu)
     bool nz_valid = false;
     size_t bytes = 0;                   // device bytes held
 

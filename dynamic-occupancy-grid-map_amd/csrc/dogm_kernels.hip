@@ -280,7 +280,8 @@ template <int PRED_BLOCK>
 __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab,
                                                    int pph, int passes, unsigned* __restrict__ ghist,
                                                    unsigned* __restrict__ tickets, unsigned* __restrict__ thist,
-                                                   int tiles, int aos, const uint32_t* __restrict__ tab_c)
+                                                   int tiles, int aos, const uint32_t* __restrict__ tab_c,
+                                                   DevScalars* __restrict__ scs)
 {
     constexpr int PRED_ITEMS = SORT_TILE / PRED_BLOCK;
     static_assert(PRED_ITEMS * PRED_BLOCK == SORT_TILE, "predict workgroups are the sort's tiles");
@@ -297,6 +298,8 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
     const TileRef tr = tile_ref(tab, SORT_Q, blockIdx.x);
     const VehDesc& d = descs[tr.v];
     const int n = d.N;
+    if (tr.base == 0 && threadIdx.x == 0)
+        scs[tr.v].born_odd = 0;  // until the occupancy update finds one
     if (tr.base >= n)
     {
         if (passes > 0 && thist)
@@ -427,10 +430,10 @@ void run_predict(Engine* E, int pph, bool hist, bool aos)
     launch_begin(E, K_PREDICT);
     if (pb == 256)
         hipLaunchKernelGGL(k_predict<256>, dim3(blocks + resets), dim3(256), 0, E->stream, E->d_desc, E->tab(SP_P),
-                           pph, passes, E->sort_ghist, E->sort_tickets, thist, blocks, aos ? 1 : 0, E->tab(SP_C));
+                           pph, passes, E->sort_ghist, E->sort_tickets, thist, blocks, aos ? 1 : 0, E->tab(SP_C), E->scalars);
     else
         hipLaunchKernelGGL(k_predict<512>, dim3(blocks + resets), dim3(512), 0, E->stream, E->d_desc, E->tab(SP_P),
-                           pph, passes, E->sort_ghist, E->sort_tickets, thist, blocks, aos ? 1 : 0, E->tab(SP_C));
+                           pph, passes, E->sort_ghist, E->sort_tickets, thist, blocks, aos ? 1 : 0, E->tab(SP_C), E->scalars);
     launch_end(E, K_PREDICT);
 }
 
@@ -675,7 +678,8 @@ __global__ __launch_bounds__(BLOCK) void k_mass_update(const VehDesc* __restrict
                                                        const uint32_t* __restrict__ tab, int zero_empty,
                                                        SegCarry carry, int occ_tile, fx_t* __restrict__ born_sums,
                                                        int units, const uint32_t* __restrict__ tab_e,
-                                                       fx_t* __restrict__ exp_sums, int pph)
+                                                       fx_t* __restrict__ exp_sums, int pph,
+                                                       DevScalars* __restrict__ scs)
 {
     if ((int)blockIdx.x >= units)
     {
@@ -688,6 +692,8 @@ __global__ __launch_bounds__(BLOCK) void k_mass_update(const VehDesc* __restrict
     float rho_b = 0.0f;
     if (c < d.C)
         rho_b = mass_update_cell(d, c, zero_empty, carry, occ_tile, pph);
+    if (!(rho_b >= 0.0f && rho_b <= BORN_MAX))
+        scs[tr.v].born_odd = 1;
     if (born_sums)
     {
         fx_t total;
@@ -815,7 +821,7 @@ void run_occupancy(Engine* E, int pph, int zero_empty, bool defer_normalize, boo
     const int etiles = exp_sums ? E->tiles(SP_E, SCAN_Q) : 0;
     hipLaunchKernelGGL(k_mass_update, dim3(units + etiles), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_C),
                        zero_empty, E->seg, BLOCK * E->tune.seg_items, born_sums ? born_unit_sums(E) : (fx_t*)nullptr,
-                       units, E->tab(SP_E), E->exp_tile_sum, pph);
+                       units, E->tab(SP_E), E->exp_tile_sum, pph, E->scalars);
     launch_end(E, K_MASS_UPDATE);
     if (defer_normalize)
         return;
@@ -1075,8 +1081,28 @@ __device__ int wave_slot_cells(const int* __restrict__ pend, int C, int k_first,
     }
     return jlo + upper_bound_i32(pend + jlo, r, k);
 }
+
+// What the birth cells of a full step leave for the birth particles, 64 consecutive slots (a block) per wave: the
+// cell that holds the block's first slot, and in birth.idx the cells of the slots whose cell starts inside the
+// block (with the association flag).  Every block and every such slot is written by exactly one cell.  The
+// records lie in the CDF buffer, free between the sort and the resampling.
+struct BirthBlock
+{
+    int cell;
+    int s, e;  // the cell's slots [s, e)
+    int nu_A;
+};
+
+__device__ __forceinline__ BirthBlock* birth_blocks(const VehDesc& d)
+{
+    return reinterpret_cast<BirthBlock*>(d.cdf);
+}
+
+// full: the slots' cells as the birth cells of a full step left them; otherwise (a stage-by-stage call, or masses
+// whose prefixes need not be monotone) searched in the particle-order ends.
 __global__ __launch_bounds__(BLOCK) void k_birth_particles(const VehDesc* __restrict__ descs,
-                                                           const uint32_t* __restrict__ tab)
+                                                           const uint32_t* __restrict__ tab,
+                                                           const DevScalars* __restrict__ scs, int full)
 {
     const TileRef tr = tile_ref(tab, 1, blockIdx.x);
     const VehDesc& d = descs[tr.v];
@@ -1086,14 +1112,29 @@ __global__ __launch_bounds__(BLOCK) void k_birth_particles(const VehDesc* __rest
     if (k0 >= B)
         return;  // wave-uniform
     const int k = k0 + lane;
-    const int* pend = d.pend;
-    const int j = wave_slot_cells(pend, d.C, k0, min(k0 + WAVE - 1, B - 1), k, lane);
-    if (k >= B)
-        return;
-    const int s = j > 0 ? pend[j - 1] : 0;
-    const int n = pend[j] - s;
-    const int nu_A = (int)roundf((float)n * d.meas[j].p_A);
-    const bool assoc = (k - s) <= nu_A;
+    int j;
+    bool assoc;
+    if (full && !scs[tr.v].born_odd)
+    {
+        if (k >= B)
+            return;
+        const int4 b = reinterpret_cast<const int4*>(birth_blocks(d))[k0 / WAVE];
+        const int w = d.birth.idx[k];
+        const bool spans = k < b.z;
+        j = spans ? b.x : word_index(w);
+        assoc = spans ? (k - b.y) <= b.w : word_assoc(w) != 0;
+    }
+    else
+    {
+        const int* pend = d.pend;
+        j = wave_slot_cells(pend, d.C, k0, min(k0 + WAVE - 1, B - 1), k, lane);
+        if (k >= B)
+            return;
+        const int s = j > 0 ? pend[j - 1] : 0;
+        const int n = pend[j] - s;
+        const int nu_A = (int)roundf((float)n * d.meas[j].p_A);
+        assoc = (k - s) <= nu_A;
+    }
     const u32x4 r = draw(d.seed, d.inst, TAG_BIRTH, d.ep_birth, (uint32_t)k);
     float n0, n1;
     box_muller(r.x, r.y, &n0, &n1);
@@ -1499,19 +1540,175 @@ void run_moments(Engine* E, int pph, bool fused_post, bool empty_done, bool birt
     launch_end(E, K_EMPTY_CELLS);
 }
 
-// The birth cells of a full step, and in the workgroups after the `tiles` cell tiles the moments of cells crossing
+// Birth cells of a full step, 256 cells (a unit) per workgroup with one cell per lane (IT = 1) or per wave with
+// four (IT = 4).  Cells without born mass have no births (equal prefixes round to equal particle orders), so
+// a unit without any converts and rounds nothing; it only stores zero w_A and w_UA where the last full update
+// left births.  The others hand their slots to the birth particles (BirthBlock), which then need no search over
+// the particle-order ends, and those are not stored.
+// Bound by the dependent chain of the few units with births (exact scan, roundings, the association
+// probability, divisions, slots): IT = 1 spreads it over four times the waves, which wins while the step leaves
+// the GPU idle (250 x 250 cells: 5.7 us against 10.4), IT = 4 has a quarter of the waves, which wins on large
+// grids and batches (BIRTH_WIDE_UNITS; 32 x 1200 x 1200 cells: 1.6% of the whole step).  The birth particles
+// went from 10.9 to 5.1 us at 2e5 slots.
+constexpr int BIRTH_WIDE_UNITS = 4096;
+
+template <int IT>
+__device__ __forceinline__ void birth_cells_unit(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab,
+                                                 int unit, const fx_t* __restrict__ tile_pre,
+                                                 const fx_t* __restrict__ unit_sums,
+                                                 const DevScalars* __restrict__ scs)
+{
+    constexpr int GROUP = WAVE / IT;  // lanes per 64 cells (one mark)
+    const TileRef tr = tile_ref(tab, 1, unit);
+    const VehDesc& d = descs[tr.v];
+    const DevScalars* sc = scs + tr.v;
+    const int C = d.C, v = d.B;
+    if (tr.base >= C)
+        return;
+    const int lane = threadIdx.x & (WAVE - 1), wid = wave_index();
+    const int w0 = tr.base + (IT == 1 ? wid * WAVE : 0);  // the wave's first cell
+    const int p0 = w0 + lane * IT;
+    const int cnt = max(0, min(IT, C - p0));
+    // Every load that does not depend on a value comes first: the chain below is what bounds the kernel.
+    float f[IT];
+    load_run<IT>(d.born, p0, cnt, f);
+    // The unit's prefix: its tile's plus the tile's earlier units (a vehicle's units start on a tile boundary).
+    fx_t before = tile_pre[unit / SCAN_Q];
+#pragma unroll
+    for (int q = 0; q < SCAN_Q - 1; ++q)
+    {
+        const fx_t x = unit_sums[unit - unit % SCAN_Q + q];
+        before += q < unit % SCAN_Q ? x : (fx_t)0;
+    }
+    const bool uniform = sc->total == 0;  // equal split over all cells
+    const bool odd = sc->born_odd != 0;
+    const bool all = uniform || odd || tr.base + UNIT >= C;  // (the last cell takes the remainder)
+    uint8_t* mark = d.bu + w0 / WAVE;
+    const uint32_t marks = w0 >= C ? 0u : IT == 1 ? *mark : *reinterpret_cast<const uint32_t*>(mark);
+    const bool had = !d.nz_valid || marks != 0;
+    fx_t run = 0;
+    int e[IT], s[IT], nu_A[IT];
+    float a[IT], u[IT];
+    bool any = false, mass = false;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+    {
+        e[i] = s[i] = nu_A[i] = 0;
+        a[i] = u[i] = 0.0f;
+        mass |= f[i] != 0.0f;
+    }
+    // With one cell per lane a wave's prefix needs the unit's other waves, so the unit decides together.
+    const bool active = (IT == 1 ? __syncthreads_or(mass) : __ballot(mass) != 0) || all;
+    if (active)
+    {
+        // Loaded beside the scan, not in the branch of a cell with births, behind it.
+        float pA[IT];
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+            pA[i] = i < cnt && (f[i] != 0.0f || all) ? d.meas[p0 + i].p_A : 0.0f;
+        fx_t own[IT], sum = 0;
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+        {
+            own[i] = fx_from_f32(f[i]);
+            sum += own[i];
+        }
+        const fx_t incl = wave_inclusive_scan_fx(sum);
+        if constexpr (IT == 1)
+        {
+            __shared__ fx_t s_wave[BLOCK / WAVE];
+            if (lane == WAVE - 1)
+                s_wave[wid] = incl;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < BLOCK / WAVE - 1; ++w)
+                before += w < wid ? s_wave[w] : (fx_t)0;
+        }
+        run = before + incl - sum;
+        // P_{j-1} of the lane's first cell, then P_j cell by cell.
+        int prev = p0 == 0 || cnt == 0 ? 0 : order_end_at(p0 - 1, run, sc, C, v);
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+        {
+            const int j = p0 + i;
+            run += own[i];
+            s[i] = e[i] = prev;
+            if (i < cnt)
+            {
+                if (f[i] != 0.0f || all)
+                    e[i] = order_end_at(j, run, sc, C, v);
+                const int n = e[i] - prev;
+                if (n > 0)  // cells without birth slots keep w_A = w_UA = 0
+                {
+                    nu_A[i] = (int)roundf((float)n * pA[i]);
+                    const int nu_UA = n - nu_A[i];
+                    a[i] = nu_A[i] > 0 ? (pA[i] * f[i]) / (float)nu_A[i] : 0.0f;
+                    u[i] = nu_UA > 0 ? ((1.0f - pA[i]) * f[i]) / (float)nu_UA : 0.0f;
+                    any = true;
+                }
+                prev = e[i];
+            }
+        }
+    }
+    const uint64_t births = __ballot(any);
+    if (had || births)
+    {
+        store_run<IT>(d.f[GF_W_A], p0, cnt, a);
+        store_run<IT>(d.f[GF_W_UA], p0, cnt, u);
+        if (cnt > 0 && lane % GROUP == 0)
+            mark[lane / GROUP] = GROUP == WAVE ? births != 0 : ((births >> lane) & ((1ull << (GROUP & 63)) - 1)) != 0;
+    }
+    if (odd)
+    {
+        store_run<IT>(d.pend, p0, cnt, e);  // the birth particles search
+        return;
+    }
+    if (!births)
+        return;
+    // The slots [s, e) of a cell: those before the first block boundary one by one, then one record per block.
+    int* words = d.birth.idx;
+    BirthBlock* blocks = birth_blocks(d);
+    const auto put = [&](int cell, int s0, int e0, int nu, int first, int step) {
+        const int q0 = (s0 + WAVE - 1) / WAVE;
+        for (int k = s0 + first; k < min(e0, q0 * WAVE); k += step)
+            words[k] = (int)((unsigned)cell | ((k - s0) <= nu ? WORD_ASSOC : 0u));
+        for (int q = q0 + first; q * WAVE < e0; q += step)
+            blocks[q] = BirthBlock{cell, s0, e0, nu};
+    };
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+    {
+        const bool many = e[i] - s[i] > 8;
+        if (e[i] > s[i] && !many)
+            put(p0 + i, s[i], e[i], nu_A[i], 0, 1);
+        // Cells with many slots by the whole wave, one after the other.
+        uint64_t todo = __ballot(many);
+        while (todo)
+        {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            put(w0 + l * IT + i, __shfl(s[i], l, WAVE), __shfl(e[i], l, WAVE), __shfl(nu_A[i], l, WAVE), lane, WAVE);
+        }
+    }
+}
+
+// The birth cells of a full step, and in the workgroups after the `cell_groups` the moments of cells crossing
 // chunks (both wait for the moments' launch only; as a launch of its own the latter took 4 to 5 us).
+template <int IT>
 __global__ __launch_bounds__(BLOCK) void k_birth_cells(const VehDesc* __restrict__ descs,
-                                                       const uint32_t* __restrict__ tab_c, int tiles,
+                                                       const uint32_t* __restrict__ tab_c, int cell_groups,
                                                        const fx_t* __restrict__ tile_pre,
+                                                       const fx_t* __restrict__ unit_sums,
                                                        const DevScalars* __restrict__ scs,
                                                        const uint32_t* __restrict__ tab_p, int units, int pph,
                                                        SegCarry carry)
 {
-    if ((int)blockIdx.x < tiles)
-        scan_apply_body(SrcBorn{0}, SinkBirth{}, descs, tab_c, blockIdx.x, tile_pre, scs);
+    const int group = blockIdx.x;
+    if (group < cell_groups)
+        birth_cells_unit<IT>(descs, tab_c, IT == 1 ? group : group * (BLOCK / WAVE) + wave_index(), tile_pre,
+                             unit_sums, scs);
     else
-        moments_fix_chunk(descs, tab_p, ((int)blockIdx.x - tiles) * BLOCK + (int)threadIdx.x, units, pph, carry);
+        moments_fix_chunk(descs, tab_p, (group - cell_groups) * BLOCK + (int)threadIdx.x, units, pph, carry);
 }
 
 void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
@@ -1520,10 +1717,18 @@ void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
     // stage still consumes its RNG epoch, so the stream of later stages does not depend on B.
     if (moments_first)
     {
-        const int tiles = E->tiles(SP_C, SCAN_Q), units = (int)E->units[SP_P];
+        const int cell_units = E->tiles(SP_C, 1), units = (int)E->units[SP_P], fix = div_up(units, BLOCK);
+        const bool wide = cell_units > BIRTH_WIDE_UNITS;
+        const int groups = wide ? cell_units / (BLOCK / WAVE) : cell_units;
         launch_begin(E, K_BIRTH_CELLS);
-        hipLaunchKernelGGL(k_birth_cells, dim3(tiles + div_up(units, BLOCK)), dim3(BLOCK), 0, E->stream, E->d_desc,
-                           E->tab(SP_C), tiles, E->scan_tile_pre, E->scalars, E->tab(SP_P), units, pph, E->seg);
+        if (wide)
+            hipLaunchKernelGGL(k_birth_cells<4>, dim3(groups + fix), dim3(BLOCK), 0, E->stream, E->d_desc,
+                               E->tab(SP_C), groups, E->scan_tile_pre, born_unit_sums(E), E->scalars, E->tab(SP_P),
+                               units, pph, E->seg);
+        else
+            hipLaunchKernelGGL(k_birth_cells<1>, dim3(groups + fix), dim3(BLOCK), 0, E->stream, E->d_desc,
+                               E->tab(SP_C), groups, E->scan_tile_pre, born_unit_sums(E), E->scalars, E->tab(SP_P),
+                               units, pph, E->seg);
         launch_end(E, K_BIRTH_CELLS);
     }
     else
@@ -1535,7 +1740,8 @@ void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
     if (blocks <= 0)
         return;
     launch_begin(E, K_BIRTH_PARTICLES);
-    hipLaunchKernelGGL(k_birth_particles, dim3(blocks), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_B));
+    hipLaunchKernelGGL(k_birth_particles, dim3(blocks), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_B), E->scalars,
+                       moments_first ? 1 : 0);
     launch_end(E, K_BIRTH_PARTICLES);
 }
 
