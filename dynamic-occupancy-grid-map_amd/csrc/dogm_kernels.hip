@@ -1258,10 +1258,11 @@ struct BirthTop
 
 // CELLS: the vehicles with per-cell weights (their records hold the posterior weights, so no prior or
 // likelihood weights are read: 16 N instead of 24 N); else the others.  Bound by the latency of the cell
-// records and of the f64 scans: 19.5 us at 2e6 particles with six waves per SIMD and no spills, 20.6 with seven
-// (2 registers spilled), 25.5 with eight (10 spilled).
+// records and of the f64 scans.  With the unit's index as a scalar (wave_index) the descriptor and its pointers take
+// no vector registers and no vector loads: 19.5 -> 16.3 us at 2e6 particles, 66 registers for seven waves per
+// SIMD; eight (4 registers spilled) take 17.9.
 template <int WAVES_PER_WG, bool CELLS>
-__global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per_eu(CELLS ? 6 : 7)))
+__global__ __launch_bounds__(WAVES_PER_WG* WAVE) __attribute__((amdgpu_waves_per_eu(7)))
 void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab, int pph, int post,
                SegCarry carry, int top, BirthTop births)
 {
@@ -1273,8 +1274,7 @@ void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ t
         return;
     }
     const int lane = threadIdx.x & (WAVE - 1);
-    const int unit =
-        xcd_tile((int)blockIdx.x - top, (int)gridDim.x - top) * WAVES_PER_WG + (int)threadIdx.x / WAVE;
+    const int unit = xcd_tile((int)blockIdx.x - top, (int)gridDim.x - top) * WAVES_PER_WG + wave_index();
     const TileRef tr = tile_ref(tab, 1, unit);
     const VehDesc& d = descs[tr.v];
     if (CELLS != (d.wcell != 0))
