@@ -49,6 +49,23 @@ enum GridField
     GF_COUNT
 };
 
+// A pointer to device memory as the step descriptors hold it.  The kernels load their array pointers from
+// the descriptors; the address space in the type tells the compiler that what they point to is global memory, so
+// accesses are global loads and stores and not flat ones, which also count as LDS operations: a wait for an LDS
+// value then waits for every flat load in flight.
+template <class T>
+struct GlobalPtr
+{
+    T __attribute__((address_space(1))) * p;
+    __host__ __device__ GlobalPtr& operator=(T* q)
+    {
+        p = (T __attribute__((address_space(1)))*)q;
+        return *this;
+    }
+    __host__ __device__ T* get() const { return (T*)p; }
+    __host__ __device__ operator T*() const { return get(); }
+};
+
 // pos and vel share one allocation of 16 bytes per particle (pos first); read-backs pack them into
 // the reference's (x, y, vx, vy) records.
 struct DevParticles
@@ -58,6 +75,24 @@ struct DevParticles
     int* idx;       // grid cell index
     float* weight;
     uint8_t* assoc;
+};
+
+// The same arrays in a step descriptor.
+struct DescParticles
+{
+    GlobalPtr<float2> pos, vel;
+    GlobalPtr<int> idx;
+    GlobalPtr<float> weight;
+    GlobalPtr<uint8_t> assoc;
+    DescParticles& operator=(const DevParticles& q)
+    {
+        pos = q.pos;
+        vel = q.vel;
+        idx = q.idx;
+        weight = q.weight;
+        assoc = q.assoc;
+        return *this;
+    }
 };
 
 struct DevGrid
@@ -127,40 +162,40 @@ struct VehDesc
     int draw_mode;           // resampling draws (dogm_num::DrawMode)
     int u0[SP_COUNT];        // first table unit of this vehicle per space
     int nu[SP_COUNT];        // its units per space (multiple of UNIT_ALIGN)
-    DevParticles part[2];
-    DevParticles birth;
-    int* start;
-    int* end;
-    float* f[GF_COUNT];      // f[GF_FREE] is not used by step kernels: see free[]
-    float* free[2];
-    dogm_measurement_cell* meas;
+    DescParticles part[2];
+    DescParticles birth;
+    GlobalPtr<int> start;
+    GlobalPtr<int> end;
+    GlobalPtr<float> f[GF_COUNT];      // f[GF_FREE] is not used by step kernels: see free[]
+    GlobalPtr<float> free[2];
+    GlobalPtr<dogm_measurement_cell> meas;
     // A device measurement grid of this step not yet copied into meas: the occupancy update reads it
     // from here and writes the copy (dogm.cu:205-215) as it goes, instead of a separate copy.
-    const dogm_measurement_cell* meas_in;
-    float* weight_array;
-    float4* cellrec;  // Vehicle::cellrec
-    float2* cellin;   // Vehicle::cellin
-    float* born;
-    float* m_raw;
-    int* pend;
-    int* ancestors;
-    int* sort_keys[2];
-    int* sort_vals[2];
-    fx_t* cdf;
+    GlobalPtr<const dogm_measurement_cell> meas_in;
+    GlobalPtr<float> weight_array;
+    GlobalPtr<float4> cellrec;  // Vehicle::cellrec
+    GlobalPtr<float2> cellin;   // Vehicle::cellin
+    GlobalPtr<float> born;
+    GlobalPtr<float> m_raw;
+    GlobalPtr<int> pend;
+    GlobalPtr<int> ancestors;
+    GlobalPtr<int> sort_keys[2];
+    GlobalPtr<int> sort_vals[2];
+    GlobalPtr<fx_t> cdf;
     // result extraction (allocated on first use)
-    float* x_occ;                 // [C] pignistic occupancy
-    uint8_t* x_img;               // [C] 8-bit occupancy image
-    unsigned long long* x_mask;   // [4 per unit] velocity-test ballots of the unit's waves
-    int* x_cnt;                   // [units] passing cells per unit
-    int* x_off;                   // [units + 1] their exclusive prefix; x_off[units] = total
-    int* x_idx;                   // [C] passing cells, row-major
+    GlobalPtr<float> x_occ;                 // [C] pignistic occupancy
+    GlobalPtr<uint8_t> x_img;               // [C] 8-bit occupancy image
+    GlobalPtr<unsigned long long> x_mask;   // [4 per unit] velocity-test ballots of the unit's waves
+    GlobalPtr<int> x_cnt;                   // [units] passing cells per unit
+    GlobalPtr<int> x_off;                   // [units + 1] their exclusive prefix; x_off[units] = total
+    GlobalPtr<int> x_idx;                   // [C] passing cells, row-major
     // Occupancy bits of the last full update (bit c % 64 of nz[c / 64]: cell c had particles) and
     // whether they describe the grid in memory (see Vehicle::nz_valid).
-    unsigned long long* nz;
+    GlobalPtr<unsigned long long> nz;
     int nz_valid;
     // Per 64 cells: one of them had birth slots at the last full update (so w_A or w_UA may be non-zero);
     // describes the grid in memory while nz_valid holds.
-    uint8_t* bu;
+    GlobalPtr<uint8_t> bu;
 };
 
 // Scalars produced and consumed on the device within one step, one per vehicle.

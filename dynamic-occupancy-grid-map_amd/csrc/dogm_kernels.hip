@@ -234,7 +234,7 @@ __device__ __forceinline__ bool border_cell(int c, int gs)
 }
 __device__ __forceinline__ int* border_out(const VehDesc& d)
 {
-    return reinterpret_cast<int*>(d.m_raw);
+    return reinterpret_cast<int*>(d.m_raw.get());
 }
 
 // start = end = -1 for the cells of work-table group `group` (THREADS x 4 cells), four cells per
@@ -313,9 +313,9 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
             (&s_h[0][0])[i] = 0u;
         __syncthreads();
     }
-    const DevParticles P = d.part[pph];
-    const DevParticles Q = d.part[pph ^ 1];  // sources of a deferred resampled set
-    const DevParticles Bq = d.birth;
+    const DescParticles P = d.part[pph];
+    const DescParticles Q = d.part[pph ^ 1];  // sources of a deferred resampled set
+    const DescParticles Bq = d.birth;
     const int gs = d.gs;
     const float dt = d.dt;
     const float zero = 0.0f, one = 1.0f;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
             int word = cell;
             if (aos)
             {
-                stream_store(reinterpret_cast<float4*>(d.cdf) + i, o);
+                stream_store(reinterpret_cast<float4*>(d.cdf.get()) + i, o);
                 word = (int)((unsigned)cell | (assoc ? WORD_ASSOC : 0u) |
                              (d.wcell && outside_grid(d, o) ? WORD_OUT : 0u));
             }
@@ -456,8 +456,8 @@ __global__ __launch_bounds__(BLOCK) void k_sort_gather(const VehDesc* __restrict
     const int n = d.N;
     if (k >= n)
         return;
-    const DevParticles src = d.part[pph];
-    const DevParticles dst = d.part[pph ^ 1];
+    const DescParticles src = d.part[pph];
+    const DescParticles dst = d.part[pph ^ 1];
     const int* skeys = d.sort_keys[fin];
     const int sv = d.sort_vals[fin][k];
     const int o = word_index(sv);
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(BLOCK) void k_normalize(const VehDesc* __restrict__
     const int i = tr.base + threadIdx.x;
     if (i >= d.N)
         return;
-    const DevParticles P = d.part[pph];
+    const DescParticles P = d.part[pph];
     const float m = d.m_raw[P.idx[i]];
     if (m > 1.0f)
     {
@@ -889,7 +889,7 @@ struct PersOp
             lw[i] = i < cnt ? lik[i] * w[i] : 0.0f;
             v[i][0] = lw[i];
         }
-        store_run<ITEMS>(d.weight_array, p0, cnt, lw);
+        store_run<ITEMS>(d.weight_array.get(), p0, cnt, lw);
     }
     __device__ void finalize(const VehDesc& d, int key, const fx_t (&s)[1]) const
     {
@@ -931,7 +931,7 @@ __global__ __launch_bounds__(BLOCK) void k_post_weights(const VehDesc* __restric
     const int i = tr.base + threadIdx.x;
     if (i >= d.N)
         return;
-    const DevParticles P = d.part[pph];
+    const DescParticles P = d.part[pph];
     const int c = P.idx[i];
     const float pA = d.meas[c].p_A;
     d.weight_array[i] = pA * d.f[GF_MU_A][c] * d.weight_array[i] + (1.0f - pA) * d.f[GF_MU_UA][c] * P.weight[i];
@@ -989,7 +989,7 @@ struct SinkOrders
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             e[i] = i < cnt ? order_end_at(p0 + i, pre[i], sc, d.C, d.N) : 0;
-        store_run<4>(d.pend, p0, cnt, e);
+        store_run<4>(d.pend.get(), p0, cnt, e);
     }
 };
 
@@ -1027,9 +1027,9 @@ struct SinkBirth
                 }
             }
         }
-        store_run<4>(d.pend, p0, cnt, e);
-        store_run<4>(d.f[GF_W_A], p0, cnt, a);
-        store_run<4>(d.f[GF_W_UA], p0, cnt, u);
+        store_run<4>(d.pend.get(), p0, cnt, e);
+        store_run<4>(d.f[GF_W_A].get(), p0, cnt, a);
+        store_run<4>(d.f[GF_W_UA].get(), p0, cnt, u);
     }
 };
 
@@ -1095,7 +1095,7 @@ struct BirthBlock
 
 __device__ __forceinline__ BirthBlock* birth_blocks(const VehDesc& d)
 {
-    return reinterpret_cast<BirthBlock*>(d.cdf);
+    return reinterpret_cast<BirthBlock*>(d.cdf.get());
 }
 
 // full: the slots' cells as the birth cells of a full step left them; otherwise (a stage-by-stage call, or masses
@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(BLOCK) void k_init_particles(const VehDesc* __restr
     const int j = upper_bound_i32(d.pend, d.C, k);
     const u32x4 r = draw(d.seed, d.inst, TAG_INIT_PARTICLES, d.ep_init, (uint32_t)k);
     const float v = d.vmax;
-    const DevParticles P = d.part[0];
+    const DescParticles P = d.part[0];
     P.pos[k] = make_float2((float)(j % gs) + 0.5f, (float)(j / gs) + 0.5f);
     P.vel[k] = make_float2(-v + (v - -v) * uniform01(r.x), -v + (v - -v) * uniform01(r.y));
     P.idx[k] = j;
@@ -1336,7 +1336,7 @@ void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ t
             }
             w[i] = word_out(word[i]) ? out : in;
         }
-        store_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
+        store_run<MOM_ITEMS>(d.weight_array.get(), p0, cnt, w);
     }
     else
     {
@@ -1356,7 +1356,7 @@ void k_moments(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ t
             for (int i = 0; i < MOM_ITEMS; ++i)
                 if (i < cnt)
                     w[i] = cf[i].x * w[i] + cf[i].y * wp[i];  // (p_A mu_A) w + ((1 - p_A) mu_UA) w_prior
-            store_run<MOM_ITEMS>(d.weight_array, p0, cnt, w);
+            store_run<MOM_ITEMS>(d.weight_array.get(), p0, cnt, w);
         }
     }
     float vx[MOM_ITEMS], vy[MOM_ITEMS];
@@ -1653,14 +1653,14 @@ __device__ __forceinline__ void birth_cells_unit(const VehDesc* __restrict__ des
     const uint64_t births = __ballot(any);
     if (had || births)
     {
-        store_run<IT>(d.f[GF_W_A], p0, cnt, a);
-        store_run<IT>(d.f[GF_W_UA], p0, cnt, u);
+        store_run<IT>(d.f[GF_W_A].get(), p0, cnt, a);
+        store_run<IT>(d.f[GF_W_UA].get(), p0, cnt, u);
         if (cnt > 0 && lane % GROUP == 0)
             mark[lane / GROUP] = GROUP == WAVE ? births != 0 : ((births >> lane) & ((1ull << (GROUP & 63)) - 1)) != 0;
     }
     if (odd)
     {
-        store_run<IT>(d.pend, p0, cnt, e);  // the birth particles search
+        store_run<IT>(d.pend.get(), p0, cnt, e);  // the birth particles search
         return;
     }
     if (!births)

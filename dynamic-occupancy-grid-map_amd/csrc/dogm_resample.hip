@@ -284,7 +284,7 @@ __global__ __launch_bounds__(BLOCK) void k_cdff_apply(const VehDesc* __restrict_
 #pragma unroll
     for (int w = 0; w < BLOCK / WAVE; ++w)
         tmax = s_m[w] > tmax ? s_m[w] : tmax;
-    double* cdf = reinterpret_cast<double*>(d.cdf);
+    double* cdf = reinterpret_cast<double*>(d.cdf.get());
 #pragma unroll
     for (int i = 0; i < 4; ++i)
     {
@@ -374,7 +374,7 @@ struct CdfFloatTr
     }
     __device__ static V value(const VehDesc& d, const void* ci, int t0, int j)
     {
-        const double c = reinterpret_cast<const double*>(d.cdf)[j];
+        const double c = reinterpret_cast<const double*>(d.cdf.get())[j];
         const double b = static_cast<const double*>(ci)[ENV_STRIDE * (size_t)(t0 + j / SCAN_TILE) + 1];
         return c > b ? c : b;
     }

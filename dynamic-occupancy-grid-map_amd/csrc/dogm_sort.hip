@@ -18,15 +18,10 @@ namespace dogm_hip
 
 constexpr int SORT_WAVES = BLOCK / WAVE;
 
-// Lanes of the wave holding the same digit (among `active` lanes).  Nearly sorted keys usually
-// give one digit per wave: that case costs one ballot.
+// Lanes of the wave holding the same digit (among `active` lanes).  No test for waves of one digit: the branch
+// cost more than it saved (7.0 against 7.6 us per scatter pass of 3e5 keys, 11.8 against 12.7 of 2e6).
 __device__ __forceinline__ uint64_t match_digit(unsigned d, uint64_t active)
 {
-    if (active == 0)
-        return 0;
-    const unsigned first = __shfl(d, (int)__builtin_ctzll(active), WAVE);
-    if ((__ballot(d == first) & active) == active)
-        return active;
     // Bit-sliced match on 32-bit halves: per bit, the lane's bit spread to 0 / all ones (e), the
     // wave's mask m of lanes with the bit set, and peers &= ~(m ^ e) (m where the bit is set, its
     // complement where not).
@@ -83,27 +78,120 @@ __device__ __forceinline__ const int* sort_keys_in(const VehDesc& d, int pph, in
     return ps == 0 ? d.part[pph].idx : d.sort_keys[(ps - 1) & 1];
 }
 
-// Key and value of element p of a pass.  Pass 0 (no values yet) takes the identity values with the
-// particles' flags: from the words predict left in the same step (packed), else from the association bytes.
-__device__ __forceinline__ void load_key(const VehDesc& d, int pph, const int* __restrict__ keys_in,
-                                         const int* __restrict__ vals_in, int p, bool valid, bool packed, int& key,
-                                         int& val)
+// Clears the waves' digit counters, four per 8-byte store.
+__device__ __forceinline__ void clear_counts(uint16_t* s_wcnt)
 {
-    const int k = valid ? keys_in[p] : 0;
+    static_assert(SORT_WAVES * RADIX == 4 * BLOCK, "one store per thread");
+    reinterpret_cast<uint64_t*>(s_wcnt)[threadIdx.x] = 0;
+}
+
+// Keys and values of a thread's elements p0, p0 + 64, ... of a pass (past n: the last element again; the callers
+// mask them).  Pass 0 (no values yet) takes the identity values with the particles' flags: from the words predict
+// left in the same step (packed), else from the association bytes.  The loads are unconditional and the case
+// is decided outside the loops, so all of a thread's loads are in flight together; a load per
+// element in its own branch was waited for before the next one (scatter pass 11.5 -> 7.0 us at 3e5 keys, 15.0 ->
+// 11.8 at 2e6; gathering pass 16.2 -> 13.5 at 3e5).
+__device__ __forceinline__ void load_keys(const VehDesc& d, int pph, const int* __restrict__ keys_in,
+                                          const int* __restrict__ vals_in, int p0, int n, bool packed,
+                                          int (&key)[SORT_ITEMS], int (&val)[SORT_ITEMS])
+{
+#pragma unroll
+    for (int j = 0; j < SORT_ITEMS; ++j)
+        key[j] = keys_in[min(p0 + j * WAVE, n - 1)];
     if (vals_in)
     {
-        key = k;
-        val = valid ? vals_in[p] : 0;
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; ++j)
+            val[j] = vals_in[min(p0 + j * WAVE, n - 1)];
     }
     else if (packed)
     {
-        key = word_index(k);
-        val = (int)((unsigned)p | ((unsigned)k & WORD_FLAGS));
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; ++j)
+        {
+            val[j] = (int)((unsigned)(p0 + j * WAVE) | ((unsigned)key[j] & WORD_FLAGS));
+            key[j] = word_index(key[j]);
+        }
     }
     else
     {
-        key = k;
-        val = valid ? sort_value(p, d.part[pph].assoc[p]) : 0;
+        const uint8_t* assoc = d.part[pph].assoc;
+        uint8_t a[SORT_ITEMS];
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; ++j)
+            a[j] = assoc[min(p0 + j * WAVE, n - 1)];
+#pragma unroll
+        for (int j = 0; j < SORT_ITEMS; ++j)
+            val[j] = sort_value(p0 + j * WAVE, a[j]);
+    }
+}
+
+// The gathering pass's loads and stores of a thread's sorted elements (keys kk, values vv, destinations gg; the elements
+// past the tile's cnt repeat the last one and are not stored).  The particles' states are read at random, so
+// GATHER_AHEAD of them are in flight before the first is stored (8 take 108 registers and gain nothing).
+constexpr int GATHER_AHEAD = 4;
+
+template <int GB>
+__device__ __forceinline__ void gather_particles(const VehDesc& dv, int pph, int gflags, const int (&kk)[GB],
+                                                 const int (&vv)[GB], const unsigned (&gg)[GB], int cnt)
+{
+    const DescParticles src = dv.part[pph];
+    const DescParticles dst = dv.part[pph ^ 1];
+    const bool aos = (gflags & GATHER_AOS) != 0;
+    // Uniform weights: every particle's prior weight is weight[0], which predict left in place.
+    const float w_prior = aos && dv.wuni ? src.weight[0] : 0.0f;
+    static_assert(GB % GATHER_AHEAD == 0, "whole batches");
+#pragma unroll
+    for (int b0 = 0; b0 < GB; b0 += GATHER_AHEAD)
+    {
+        float4 st[GATHER_AHEAD];
+        float w[GATHER_AHEAD];
+        if (aos)
+        {
+            const float4* rec = reinterpret_cast<const float4*>(dv.cdf.get());
+#pragma unroll
+            for (int k = 0; k < GATHER_AHEAD; ++k)
+                st[k] = rec[word_index(vv[b0 + k])];
+        }
+        else
+        {
+#pragma unroll
+            for (int k = 0; k < GATHER_AHEAD; ++k)
+            {
+                const int o = word_index(vv[b0 + k]);
+                const float2 p = src.pos[o], v = src.vel[o];
+                st[k] = make_float4(p.x, p.y, v.x, v.y);
+            }
+        }
+        if (!(aos && dv.wuni))
+        {
+#pragma unroll
+            for (int k = 0; k < GATHER_AHEAD; ++k)
+                w[k] = src.weight[word_index(vv[b0 + k])];
+        }
+        else
+        {
+#pragma unroll
+            for (int k = 0; k < GATHER_AHEAD; ++k)
+                w[k] = predicted_weight(dv, w_prior, st[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < GATHER_AHEAD; ++k)
+        {
+            const int b = b0 + k;
+            if ((int)threadIdx.x + b * BLOCK >= cnt)
+                continue;
+            const unsigned g = gg[b];
+            dst.pos[g] = make_float2(st[k].x, st[k].y);
+            dst.vel[g] = make_float2(st[k].z, st[k].w);
+            dst.assoc[g] = word_assoc(vv[b]);
+            dst.idx[g] = (int)((unsigned)kk[b] | ((unsigned)vv[b] & WORD_OUT));
+            if (dv.wcell)
+                continue;  // the occupancy update forms the weights per cell
+            dst.weight[g] = w[k];
+            if (gflags & GATHER_WA)
+                dv.weight_array[g] = w[k];
+        }
     }
 }
 
@@ -121,6 +209,12 @@ __global__ __launch_bounds__(BLOCK) void k_sort_upsweep(const VehDesc* __restric
     const int n = dv.N;
     const int shift = ps * RADIX_BITS;
     const int* keys = sort_keys_in(dv, pph, ps);
+    if (tr.base >= n)
+    {
+        for (int d = threadIdx.x; d < RADIX; d += BLOCK)
+            thist[(size_t)d * tiles + blockIdx.x] = 0u;
+        return;
+    }
     for (int i = threadIdx.x; i < RADIX; i += BLOCK)
         s_h[i] = 0u;
     __syncthreads();
@@ -130,8 +224,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_upsweep(const VehDesc* __restric
 #pragma unroll
     for (int i = 0; i < SORT_ITEMS; ++i)
     {
-        const int p = tr.base + i * BLOCK + threadIdx.x;
-        kd[i] = p < n ? (unsigned)keys[p] : 0xffffffffu;
+        kd[i] = (unsigned)keys[min(tr.base + i * BLOCK + (int)threadIdx.x, n - 1)];
     }
 #pragma unroll
     for (int i = 0; i < SORT_ITEMS; ++i)
@@ -233,7 +326,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
                                                           const unsigned* __restrict__ goff, int passes,
                                                           unsigned* __restrict__ ghist, int gflags)
 {
-    __shared__ uint16_t s_wcnt[SORT_WAVES][RADIX];  // counts <= SORT_TILE; 16 bits keep 8 workgroups per CU
+    __shared__ __attribute__((aligned(8))) uint16_t s_wcnt[SORT_WAVES][RADIX];  // counts <= SORT_TILE; 16 bits keep 8 workgroups per CU
     __shared__ unsigned s_digoff[RADIX];
     __shared__ int s_keys[SORT_TILE];
     __shared__ int s_vals[SORT_TILE];
@@ -262,30 +355,23 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
 
     const int lane = threadIdx.x & (WAVE - 1);
     const int wid = threadIdx.x / WAVE;
-    for (int i = threadIdx.x; i < SORT_WAVES * RADIX; i += BLOCK)
-        (&s_wcnt[0][0])[i] = 0;
-    __syncthreads();
-
     int key[SORT_ITEMS], val[SORT_ITEMS];
     unsigned rank[SORT_ITEMS];
     const uint64_t lt = lanemask_lt();
+    load_keys(dv, pph, keys_in, vals_in, tbase + wid * SORT_ITEMS * WAVE + lane, n, packed, key, val);
+    clear_counts(&s_wcnt[0][0]);
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < SORT_ITEMS; ++j)
     {
         const int p = tbase + (wid * SORT_ITEMS + j) * WAVE + lane;
         const bool valid = p < n;
-        load_key(dv, pph, keys_in, vals_in, p, valid, packed, key[j], val[j]);
         const unsigned d = ((unsigned)key[j] >> shift) & (RADIX - 1);
         const uint64_t peers = match_digit(d, __ballot(valid));
-        unsigned r = 0;
-        if (valid)
-        {
-            const unsigned before = s_wcnt[wid][d];
-            r = before + (unsigned)__popcll(peers & lt);
-            if ((peers & lt) == 0)
-                s_wcnt[wid][d] = (uint16_t)(before + (unsigned)__popcll(peers));
-        }
-        rank[j] = r;
+        const unsigned before = s_wcnt[wid][d];
+        rank[j] = before + (unsigned)__popcll(peers & lt);
+        if (valid && (peers & lt) == 0)
+            s_wcnt[wid][d] = (uint16_t)(before + (unsigned)__popcll(peers));
     }
     __syncthreads();
 
@@ -355,45 +441,20 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
         const unsigned d = ((unsigned)kk[b] >> shift) & (RADIX - 1);
         gg[b] = s_digoff[d] + (unsigned)s;
     }
-    // Uniform weights: every particle's prior weight is weight[0], which predict left in place.
-    const float w_prior = GATHER && (gflags & GATHER_AOS) && dv.wuni ? dv.part[pph].weight[0] : 0.0f;
-#pragma unroll
-    for (int b = 0; b < GB; ++b)
+    if constexpr (GATHER)
     {
-        if ((int)threadIdx.x + b * BLOCK >= cnt)
-            break;
-        const unsigned g = gg[b];
-        if constexpr (GATHER)
+        gather_particles(dv, pph, gflags, kk, vv, gg, cnt);
+    }
+    else
+    {
+#pragma unroll
+        for (int b = 0; b < GB; ++b)
         {
-            const DevParticles src = dv.part[pph];
-            const DevParticles dst = dv.part[pph ^ 1];
-            const int o = word_index(vv[b]);
-            dst.assoc[g] = word_assoc(vv[b]);
-            dst.idx[g] = (int)((unsigned)kk[b] | ((unsigned)vv[b] & WORD_OUT));
-            float w;
-            if (gflags & GATHER_AOS)
+            if ((int)threadIdx.x + b * BLOCK < cnt)
             {
-                const float4 st = reinterpret_cast<const float4*>(dv.cdf)[o];
-                dst.pos[g] = make_float2(st.x, st.y);
-                dst.vel[g] = make_float2(st.z, st.w);
-                if (dv.wcell)
-                    continue;  // the occupancy update forms the weights per cell
-                w = dv.wuni ? predicted_weight(dv, w_prior, st) : src.weight[o];
+                keys_out[gg[b]] = kk[b];
+                vals_out[gg[b]] = vv[b];
             }
-            else
-            {
-                w = src.weight[o];
-                dst.pos[g] = src.pos[o];
-                dst.vel[g] = src.vel[o];
-            }
-            dst.weight[g] = w;
-            if (gflags & GATHER_WA)
-                dv.weight_array[g] = w;
-        }
-        else
-        {
-            keys_out[g] = kk[b];
-            vals_out[g] = vv[b];
         }
     }
 }
@@ -469,7 +530,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
                                                          unsigned* __restrict__ tickets, unsigned epoch,
                                                          int spin_limit, unsigned* __restrict__ err, int gflags)
 {
-    __shared__ uint16_t s_wcnt[SORT_WAVES][RADIX];  // counts <= SORT_TILE; 16 bits keep 8 workgroups per CU
+    __shared__ __attribute__((aligned(8))) uint16_t s_wcnt[SORT_WAVES][RADIX];  // counts <= SORT_TILE; 16 bits keep 8 workgroups per CU
     __shared__ unsigned s_digoff[RADIX];
     __shared__ unsigned s_gbase[RADIX];
     __shared__ int s_keys[SORT_TILE];
@@ -479,8 +540,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
 
     if (threadIdx.x == 0)
         s_tile = (int)atomicAdd(&tickets[ps], 1u);
-    for (int i = threadIdx.x; i < SORT_WAVES * RADIX; i += BLOCK)
-        (&s_wcnt[0][0])[i] = 0;
+    clear_counts(&s_wcnt[0][0]);
     __syncthreads();
     const int tile = s_tile;
     const TileRef tr = tile_ref(tab, SORT_Q, tile);
@@ -502,23 +562,18 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
     int key[SORT_ITEMS], val[SORT_ITEMS];
     unsigned rank[SORT_ITEMS];
     const uint64_t lt = lanemask_lt();
+    load_keys(dv, pph, keys_in, vals_in, tbase + wid * SORT_ITEMS * WAVE + lane, n, packed, key, val);
 #pragma unroll
     for (int j = 0; j < SORT_ITEMS; ++j)
     {
         const int p = tbase + (wid * SORT_ITEMS + j) * WAVE + lane;
         const bool valid = p < n;
-        load_key(dv, pph, keys_in, vals_in, p, valid, packed, key[j], val[j]);
         const unsigned d = ((unsigned)key[j] >> shift) & (RADIX - 1);
         const uint64_t peers = match_digit(d, __ballot(valid));
-        unsigned r = 0;
-        if (valid)
-        {
-            const unsigned before = s_wcnt[wid][d];
-            r = before + (unsigned)__popcll(peers & lt);
-            if ((peers & lt) == 0)
-                s_wcnt[wid][d] = (uint16_t)(before + (unsigned)__popcll(peers));
-        }
-        rank[j] = r;
+        const unsigned before = s_wcnt[wid][d];
+        rank[j] = before + (unsigned)__popcll(peers & lt);
+        if (valid && (peers & lt) == 0)
+            s_wcnt[wid][d] = (uint16_t)(before + (unsigned)__popcll(peers));
     }
     __syncthreads();
 
@@ -670,45 +725,20 @@ __global__ __launch_bounds__(BLOCK) void k_sort_onesweep(const VehDesc* __restri
         const unsigned db = ((unsigned)kk[b] >> shift) & (RADIX - 1);
         gg[b] = s_gbase[db] + ((unsigned)s - s_digoff[db]);
     }
-    // Uniform weights: every particle's prior weight is weight[0], which predict left in place.
-    const float w_prior = GATHER && (gflags & GATHER_AOS) && dv.wuni ? dv.part[pph].weight[0] : 0.0f;
-#pragma unroll
-    for (int b = 0; b < GB; ++b)
+    if constexpr (GATHER)
     {
-        if ((int)threadIdx.x + b * BLOCK >= cnt)
-            break;
-        const unsigned g = gg[b];
-        if constexpr (GATHER)
+        gather_particles(dv, pph, gflags, kk, vv, gg, cnt);
+    }
+    else
+    {
+#pragma unroll
+        for (int b = 0; b < GB; ++b)
         {
-            const DevParticles src = dv.part[pph];
-            const DevParticles dst = dv.part[pph ^ 1];
-            const int o = word_index(vv[b]);
-            dst.assoc[g] = word_assoc(vv[b]);
-            dst.idx[g] = (int)((unsigned)kk[b] | ((unsigned)vv[b] & WORD_OUT));
-            float w;
-            if (gflags & GATHER_AOS)
+            if ((int)threadIdx.x + b * BLOCK < cnt)
             {
-                const float4 st = reinterpret_cast<const float4*>(dv.cdf)[o];
-                dst.pos[g] = make_float2(st.x, st.y);
-                dst.vel[g] = make_float2(st.z, st.w);
-                if (dv.wcell)
-                    continue;  // the occupancy update forms the weights per cell
-                w = dv.wuni ? predicted_weight(dv, w_prior, st) : src.weight[o];
+                keys_out[gg[b]] = kk[b];
+                vals_out[gg[b]] = vv[b];
             }
-            else
-            {
-                w = src.weight[o];
-                dst.pos[g] = src.pos[o];
-                dst.vel[g] = src.vel[o];
-            }
-            dst.weight[g] = w;
-            if (gflags & GATHER_WA)
-                dv.weight_array[g] = w;
-        }
-        else
-        {
-            keys_out[g] = kk[b];
-            vals_out[g] = vv[b];
         }
     }
 }
