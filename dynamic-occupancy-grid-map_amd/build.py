@@ -77,7 +77,8 @@ def build_oracle() -> Path:
 
 
 def build_cpp_tests() -> list[Path]:
-    """C++ drop-in tests: include/dogm/dogm.h linked against libdogm_hip.so with g++."""
+    """C++ drop-in tests (include/dogm/dogm.h linked against libdogm_hip.so with g++) and device-only tests of the
+    headers (hipcc, the library's flags)."""
     outs = []
     tdir = REPO / "tests" / "cpp"
     for src in sorted(tdir.glob("*.cpp")):
@@ -87,6 +88,10 @@ def build_cpp_tests() -> list[Path]:
             f"-I{REPO / 'include'}", str(src), "-o", str(exe),
             f"-L{LIB}", "-ldogm_hip", f"-Wl,-rpath,{LIB}",
         ])
+        outs.append(exe)
+    for src in sorted(tdir.glob("*.hip")):
+        exe = tdir / src.stem
+        _run([HIPCC, *HIP_FLAGS, str(src), "-o", str(exe)])
         outs.append(exe)
     return outs
 

@@ -154,6 +154,40 @@ DOGM_HD float uniform_range(uint32_t x, float lo, float hi)
 // ---------------------------------------------------------------------------------------------
 // Elementary functions for Box-Muller
 // ---------------------------------------------------------------------------------------------
+// Correctly rounded f / d of the logarithm below, |f| < 0.42 and 1.7 < d < 2.42 (f = 0 included): a quotient by a
+// refined reciprocal and one remainder step (Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", 1990).  The general division also scales its operands and repairs special
+// results, which this range does not need.  Equal to f / d for all 2^24 arguments the draws take.
+DOGM_HD float log_quotient(float f, float d)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    const float q = f * r;
+    return fmaf(fmaf(-d, q, f), r, q);
+#else
+    return f / d;
+#endif
+}
+
+// Correctly rounded square root of 0 (either sign, returned as it is) or 1e-7 < x < 40, by Goldschmidt iteration on
+// a reciprocal square root and one remainder step (Markstein, same paper); equal to sqrtf for all 2^24
+// arguments of Box-Muller.
+DOGM_HD float box_muller_sqrt(float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y = __builtin_amdgcn_rsqf(x);
+    float g = x * y, h = 0.5f * y;
+    const float r = fmaf(-h, g, 0.5f);
+    g = fmaf(g, r, g);
+    h = fmaf(h, r, h);
+    g = fmaf(fmaf(-g, g, x), h, g);
+    return x == 0.0f ? x : g;
+#else
+    return sqrtf(x);
+#endif
+}
+
 // Natural logarithm of a positive normal float.
 // x = m * 2^e with m in [sqrt(1/2), sqrt(2)); ln m = 2 atanh(s), s = (m - 1) / (m + 1),
 // |s| <= 0.1716, atanh series to s^11 (truncation < 2e-10 relative).
@@ -168,7 +202,7 @@ DOGM_HD float log_f32(float x)
         e = e + 1;
     }
     const float f = m - 1.0f;  // exact (Sterbenz)
-    const float s = f / (m + 1.0f);
+    const float s = log_quotient(f, m + 1.0f);
     const float s2 = s * s;
     float p = fmaf(s2, 0.0909090936f, 0.111111112f);  // 1/11, 1/9
     p = fmaf(s2, p, 0.142857149f);                    // 1/7
@@ -181,16 +215,11 @@ DOGM_HD float log_f32(float x)
     return fmaf(fe, 0.693145752f, fmaf(fe, 1.42860677e-06f, lnm));
 }
 
-// sin(2 pi t), cos(2 pi t) for t in [0, 1).
-// t * 4 = q + f (q quadrant, f in [0, 1)); angle = q pi/2 + pi/4 + x with x = (f - 1/2) pi/2,
-// |x| <= pi/4; Taylor polynomials to x^9 / x^10 (truncation < 2e-9).
-DOGM_HD void sincos_2pi_f32(float t, float* s_out, float* c_out)
+// sin(2 pi t), cos(2 pi t) for t in [0, 1), t * 4 = q + f (q quadrant, f in [0, 1)):
+// angle = q pi/2 + pi/4 + x with x = (f - 1/2) pi/2, |x| <= pi/4; Taylor polynomials to x^9 / x^10
+// (truncation < 2e-9).
+DOGM_HD void sincos_quadrant_f32(uint32_t q, float f, float* s_out, float* c_out)
 {
-    const float t4 = t * 4.0f;  // exact
-    int q = (int)t4;
-    if (q > 3)
-        q = 3;
-    const float f = t4 - (float)q;  // exact
     const float x = (f - 0.5f) * 1.57079637f;
     const float x2 = x * x;
     float ps = fmaf(x2, 2.75573188e-06f, -1.98412701e-04f);  // 1/9!, -1/7!
@@ -204,39 +233,31 @@ DOGM_HD void sincos_2pi_f32(float t, float* s_out, float* c_out)
     const float cx = fmaf(x2, pc, 1.0f);
     const float sp = (sx + cx) * 0.707106769f;  // sin(pi/4 + x)
     const float cp = (cx - sx) * 0.707106769f;  // cos(pi/4 + x)
-    float s, c;
-    if (q == 0)
-    {
-        s = sp;
-        c = cp;
-    }
-    else if (q == 1)
-    {
-        s = cp;
-        c = -sp;
-    }
-    else if (q == 2)
-    {
-        s = -sp;
-        c = -cp;
-    }
-    else
-    {
-        s = -cp;
-        c = sp;
-    }
-    *s_out = s;
-    *c_out = c;
+    // (s, c) = (sp, cp), (cp, -sp), (-sp, -cp), (-cp, sp) for q = 0 .. 3.
+    const bool swap = (q & 1u) != 0u;
+    *s_out = f32_from_bits(f32_bits(swap ? cp : sp) ^ ((q & 2u) << 30));
+    *c_out = f32_from_bits(f32_bits(swap ? sp : cp) ^ (((q + 1u) & 2u) << 30));
+}
+
+DOGM_HD void sincos_2pi_f32(float t, float* s_out, float* c_out)
+{
+    const float t4 = t * 4.0f;  // exact
+    int q = (int)t4;
+    if (q > 3)
+        q = 3;
+    sincos_quadrant_f32((uint32_t)q, t4 - (float)q, s_out, c_out);  // the difference is exact
 }
 
 // Two standard normals from two 32-bit words (Box-Muller).
 DOGM_HD void box_muller(uint32_t a, uint32_t b, float* z0, float* z1)
 {
     const float u1 = uniform01_oc(a);
-    const float t = uniform01(b);
-    const float r = sqrtf(-2.0f * log_f32(u1));
+    const float r = box_muller_sqrt(-2.0f * log_f32(u1));
+    // t = uniform01(b) has 24 bits: the top two are the quadrant, the other 22 the fraction (exact, as in
+    // sincos_2pi_f32).
+    const float f = (float)((b >> 8) & 0x3fffffu) * 0x1p-22f;
     float s, c;
-    sincos_2pi_f32(t, &s, &c);
+    sincos_quadrant_f32(b >> 30, f, &s, &c);
     *z0 = r * c;
     *z1 = r * s;
 }
