@@ -430,7 +430,7 @@ int engine_reserve(Engine* E, int m, std::string* why)
         int st;
         if ((st = dalloc(&E->d_desc, cap, "step descriptors", why)) ||
             (st = dalloc(&E->d_upre, (size_t)SP_COUNT * (cap + 1), "step tables", why)) ||
-            (st = dalloc(&E->sort_ghist, (size_t)cap * 4 * 256 + 64, "sort histograms", why)) ||
+            (st = dalloc(&E->sort_ghist, (size_t)cap * 5 * 256 + 64, "sort histograms", why)) ||
             (st = dalloc(&E->scalars, cap, "step scalars", why)))
             return st;
         // Cleared on the engine's own stream and waited for: hipMemset runs on the null stream, which
@@ -441,6 +441,7 @@ int engine_reserve(Engine* E, int m, std::string* why)
             hipStreamSynchronize(E->stream) != hipSuccess)
             return set_err(why, DOGM_ERR_HIP, "clearing step scalars");
         E->sort_tickets = E->sort_ghist + (size_t)cap * 4 * 256;
+        E->sort_totals = E->sort_tickets + 64;
         E->ghist_clean = true;
         E->m_cap = cap;
     }

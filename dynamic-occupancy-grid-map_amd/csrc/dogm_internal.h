@@ -465,7 +465,8 @@ struct Engine
     long long status_plan = -1;       // plan whose tiles sort_status holds lookback words for
     int lookback_spin = 1 << 20;      // polls before a lookback wait gives up (DOGM_ERR_DEVICE_CHECK)
     unsigned* sort_tickets = nullptr; // [4] tile tickets of the passes (after sort_ghist's histograms)
-    // sort_ghist is all zero: every sort clears the histograms it consumed in its last pass, so the
+    unsigned* sort_totals = nullptr;  // [m * 256] digit totals of a reduce-then-scan pass (after the tickets)
+    // sort_ghist is all zero: every onesweep sort clears the histograms it consumed in its last pass, so the
     // next step's predict can count into them without a fill (false after a step that stopped early).
     bool ghist_clean = false;
     int ghist_cap = 0;

@@ -207,12 +207,15 @@ __device__ __forceinline__ int clamp_cell(float x, int gs)
 
 // A workgroup covers one sort tile: PB threads of SORT_TILE / PB particles each (strided by PB).
 // 512 x 4 (the built-in choice) gives a single 2e6-particle grid about 8 waves per SIMD to hide the
-// Philox / Box-Muller latency; 256 x 8 is the other choice of the tuning.  The item loop loads ahead and stays
-// rolled (3e5 particles 13.6 -> 11.2 us, with the shorter quotient and root of the normal draws).
-
-// With passes > 0 the workgroup also counts the radix digits of the new cell indices for every
-// sort pass into ghist[(vehicle * 4 + pass) * 256 + digit] (the sort's one-time histogram) and
-// clears the sort passes' tile tickets (the passes run after predict on the same stream); with
+// Philox / Box-Muller latency; 256 x 8 is the other choice of the tuning.  Bound by memory where many vehicles
+// share a launch (41 bytes a particle; 16 x 2e6: 329 us) and by latency below: with the item loop loading ahead,
+// without its digit counts' global atomics and with the shorter quotient and root, 2e6 particles went from 35.5 to
+// 23.8 us and 3e5 from 13.6 to 9.6; the item loop stays rolled (unrolled: 23.5 and 11.0).
+//
+// With passes > 0 the workgroup also counts the radix digits of the new cell indices (of every sort pass for the
+// onesweep form, of the first for reduce-then-scan: `passes`).  Without thist the counts go to
+// ghist[(vehicle * 4 + pass) * 256 + digit] (onesweep's one-time histogram; the sort passes' tile tickets are
+// cleared too); with
 // thist set (reduce-then-scan sort) it stores the first pass's digit counts of its tile as
 // thist[digit * tiles + tile]: a workgroup covers exactly one sort tile, so the sort skips that
 // upsweep.  With aos (the sort's gathering pass follows in the same step) the new state goes to the
@@ -416,6 +419,12 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
     if (passes > 0)
     {
         __syncthreads();
+        if (thist)
+        {
+            for (int i = threadIdx.x; i < RADIX; i += PRED_BLOCK)
+                thist[(size_t)i * tiles + blockIdx.x] = s_h[0][i];
+            return;
+        }
         unsigned* gh = ghist + (size_t)tr.v * 4 * RADIX;
         for (int i = threadIdx.x; i < passes * RADIX; i += PRED_BLOCK)
         {
@@ -423,9 +432,6 @@ __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restric
             if (v)
                 atomicAdd(&gh[i], v);
         }
-        if (thist)
-            for (int i = threadIdx.x; i < RADIX; i += PRED_BLOCK)
-                thist[(size_t)i * tiles + blockIdx.x] = s_h[0][i];
     }
 }
 
@@ -434,11 +440,15 @@ void run_predict(Engine* E, int pph, bool hist, bool aos)
     const int blocks = E->tiles(SP_P, SORT_Q);
     if (blocks <= 0)
         return;
-    if (hist && !E->ghist_clean)
-        run_fill_u32(E, E->sort_ghist, 0u, (long long)E->m * 4 * RADIX);
-    E->ghist_clean = false;  // until the sort of this step has cleared them again
-    unsigned* thist = E->tune.sort == SORT_REDUCE_SCAN ? E->sort_status : nullptr;
-    const int passes = hist ? E->passes : 0;
+    const bool onesweep = E->tune.sort == SORT_ONESWEEP;
+    if (hist && onesweep)
+    {
+        if (!E->ghist_clean)
+            run_fill_u32(E, E->sort_ghist, 0u, (long long)E->m * 4 * RADIX);
+        E->ghist_clean = false;  // until the sort of this step has cleared them again
+    }
+    unsigned* thist = onesweep ? nullptr : E->sort_status;
+    const int passes = hist ? (onesweep ? E->passes : 1) : 0;
     // With the assignment in the same step (hist), its bounds reset runs in extra workgroups.
     const int pb = E->tune.pred_block == 256 ? 256 : 512;
     const int resets = hist ? E->tiles(SP_C, pb * 4 / UNIT) : 0;

@@ -2,12 +2,12 @@
 // dogm/src/dogm.cu:270-276).
 //
 // Keys are cell indices < grid_size^2, so only ceil(log2(C)) bits are sorted, 8 bits per pass.
-// One histogram of every pass's digits is counted once (by predict when it runs in the same step).
 // Two forms of a pass, chosen per step by the engine's tuning:
 //  * reduce-then-scan: tile digit counts (predict stores the first pass's) -> per-vehicle,
-//    per-digit exclusive scan over the vehicle's tiles plus the digit's base -> ranking and scatter,
-//    tiles taken in an XCD-aware order;
-//  * onesweep: a single launch per pass; a tile ranks its keys, obtains every digit's offset from
+//    per-digit exclusive scan over the vehicle's tiles, and the digit's total -> ranking and scatter (each tile scans
+//    the digits' totals for their bases), tiles taken in an XCD-aware order;
+//  * onesweep: a histogram of every pass's digits, counted once (by predict when it runs in the same step), then
+//    a single launch per pass; a tile ranks its keys, obtains every digit's offset from
 //    the earlier tiles of its vehicle by a decoupled lookback, and scatters.
 // Both rank and scatter identically, so their results are identical.  Every vehicle of a step is
 // sorted independently into its own buffers; all use the step's pass count.
@@ -234,33 +234,16 @@ __global__ __launch_bounds__(BLOCK) void k_sort_upsweep(const VehDesc* __restric
         thist[(size_t)d * tiles + blockIdx.x] = s_h[d];
 }
 
-// One workgroup per (digit, vehicle): exclusive scan over the vehicle's tiles plus the digit's
-// base inside the vehicle.  Each thread scans a contiguous chunk of the row.
+// One workgroup per (digit, vehicle): exclusive scan over the vehicle's tiles, and the digit's total.  Each
+// thread scans a contiguous chunk of the row.
 __global__ __launch_bounds__(BLOCK) void k_sort_scan(const VehDesc* __restrict__ descs, unsigned* __restrict__ thist,
-                                                     int tiles, const unsigned* __restrict__ ghist, int ps)
+                                                     int tiles, unsigned* __restrict__ totals)
 {
     __shared__ unsigned s_w[SORT_WAVES];
-    __shared__ unsigned s_base;
     const int d = blockIdx.x;
     const int v = blockIdx.y;
     const VehDesc& dv = descs[v];
-    const unsigned* ghist_pass = ghist + ((size_t)v * 4 + ps) * RADIX;
     const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
-    if (threadIdx.x < WAVE)
-    {
-        unsigned b = 0;
-#pragma unroll
-        for (int k = 0; k < RADIX / WAVE; ++k)  // independent loads
-        {
-            const int e = lane + k * WAVE;
-            b += e < d ? ghist_pass[e] : 0u;
-        }
-#pragma unroll
-        for (int s = WAVE / 2; s > 0; s >>= 1)
-            b += __shfl_xor(b, s, WAVE);
-        if (lane == 0)
-            s_base = b;
-    }
     const int t0 = dv.u0[SP_P] / SORT_Q;
     const int nt = dv.nu[SP_P] / SORT_Q;
     unsigned* row = thist + (size_t)d * tiles + t0;
@@ -290,11 +273,13 @@ __global__ __launch_bounds__(BLOCK) void k_sort_scan(const VehDesc* __restrict__
     if (lane == WAVE - 1)
         s_w[wid] = incl;
     __syncthreads();
-    unsigned run = s_base + incl - sum;
+    unsigned run = incl - sum;
 #pragma unroll
     for (int w = 0; w < SORT_WAVES; ++w)
         if (w < wid)
             run += s_w[w];
+    if (threadIdx.x == BLOCK - 1)
+        totals[(size_t)v * RADIX + d] = run + sum;
     for (int tc = b0; tc < b1; tc += 8)
     {
         unsigned x[8];
@@ -320,17 +305,22 @@ __global__ __launch_bounds__(BLOCK) void k_sort_scan(const VehDesc* __restrict__
 // With GATHER_AOS the state is read from the 16-byte records predict left in the CDF buffer, and
 // for vehicles with uniform weights the predicted weight is formed here (predicted_weight), or not at all where
 // the occupancy update forms the weights per cell (VehDesc::wcell).
+//
+// Every tile scans the digits' totals itself: counted ahead by predict, they took 977 x 768 atomics on the same
+// 768 words (predict of 2e6 particles 35.5 us, 23.8 without), and a scatter with the scan costs 126 us for 16 x 2e6
+// keys against 119.  Seven waves per SIMD are asked for because the scatter would take 78 registers, six waves,
+// 131 us; eight waves spill (171 us).
 template <bool GATHER>
-__global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restrict__ descs,
+__global__ __launch_bounds__(BLOCK, GATHER ? 6 : 7) void k_sort_downsweep(const VehDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ tab, int pph, int ps, int tiles,
-                                                          const unsigned* __restrict__ goff, int passes,
-                                                          unsigned* __restrict__ ghist, int gflags)
+                                                          const unsigned* __restrict__ goff,
+                                                          const unsigned* __restrict__ totals, int gflags)
 {
     __shared__ __attribute__((aligned(8))) uint16_t s_wcnt[SORT_WAVES][RADIX];  // counts <= SORT_TILE; 16 bits keep 8 workgroups per CU
     __shared__ unsigned s_digoff[RADIX];
     __shared__ int s_keys[SORT_TILE];
     __shared__ int s_vals[SORT_TILE];
-    __shared__ unsigned s_scan[SORT_WAVES];
+    __shared__ uint2 s_scan[SORT_WAVES];
 
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const TileRef tr = tile_ref(tab, SORT_Q, tile);
@@ -341,13 +331,6 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
         return;
     const int shift = ps * RADIX_BITS;
     const bool packed = (gflags & GATHER_AOS) != 0;
-    if (ps == passes - 1 && tbase == 0)
-    {
-        // The digit scans of every pass have run: clear this vehicle's histograms for the next sort.
-        unsigned* gh = ghist + (size_t)tr.v * 4 * RADIX;
-        for (int i = threadIdx.x; i < 4 * RADIX; i += BLOCK)
-            gh[i] = 0u;
-    }
     const int* keys_in = sort_keys_in(dv, pph, ps);
     const int* vals_in = ps == 0 ? nullptr : dv.sort_vals[(ps - 1) & 1];
     int* keys_out = dv.sort_keys[ps & 1];
@@ -375,7 +358,12 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
     }
     __syncthreads();
 
-    // Per digit: tile total, offsets of the waves inside the digit, tile-local digit offsets.
+    // Per digit: tile total, offsets of the waves inside the digit, tile-local digit offsets, and the digit's base
+    // in the vehicle (two exclusive scans over the digits, one digit per thread), from the digit's keys in the
+    // vehicle's earlier tiles and in all.
+    const unsigned before = goff[(size_t)threadIdx.x * tiles + tile];
+    const unsigned total = totals[(size_t)tr.v * RADIX + threadIdx.x];
+    unsigned gbase;
     {
         const int d = threadIdx.x;  // BLOCK == RADIX
         unsigned run = 0;
@@ -386,26 +374,31 @@ __global__ __launch_bounds__(BLOCK) void k_sort_downsweep(const VehDesc* __restr
             s_wcnt[w][d] = (uint16_t)run;
             run += c;
         }
-        unsigned incl = run;
+        unsigned incl = run, base = total;
 #pragma unroll
         for (int s = 1; s < WAVE; s <<= 1)
         {
-            const unsigned u = __shfl_up(incl, s, WAVE);
+            const unsigned u = __shfl_up(incl, s, WAVE), v = __shfl_up(base, s, WAVE);
             if (lane >= s)
+            {
                 incl += u;
+                base += v;
+            }
         }
         if (lane == WAVE - 1)
-            s_scan[wid] = incl;
+            s_scan[wid] = make_uint2(incl, base);
         __syncthreads();
-        unsigned wc = 0;
+        unsigned wc = 0, wb = 0;
 #pragma unroll
         for (int w = 0; w < SORT_WAVES; ++w)
-            if (w < wid)
-                wc += s_scan[w];
+        {
+            const uint2 x = s_scan[w];
+            wc += w < wid ? x.x : 0u;
+            wb += w < wid ? x.y : 0u;
+        }
         s_digoff[d] = wc + incl - run;
+        gbase = before + wb + base - total;  // the digit's destination base for this tile
     }
-    // The digit's destination base for this tile: one load per digit instead of one per key.
-    const unsigned gbase = goff[(size_t)threadIdx.x * tiles + tile];
     __syncthreads();
 
 #pragma unroll
@@ -763,7 +756,7 @@ void run_sort(Engine* E, int pph, bool hist_done, bool gather, bool write_wa)
     }
     if (!onesweep)
         E->status_plan = -1;  // the buffer now holds tile counts
-    if (!hist_done)
+    if (onesweep && !hist_done)
     {
         if (!E->ghist_clean)
             run_fill_u32(E, E->sort_ghist, 0u, (long long)E->m * 4 * RADIX);
@@ -803,18 +796,19 @@ void run_sort(Engine* E, int pph, bool hist_done, bool gather, bool write_wa)
         }
         launch_begin(E, K_SORT_SCAN);
         hipLaunchKernelGGL(k_sort_scan, dim3(RADIX, E->m), dim3(BLOCK), 0, E->stream, E->d_desc, E->sort_status, tiles,
-                           E->sort_ghist, ps);
+                           E->sort_totals);
         launch_end(E, K_SORT_SCAN);
         launch_begin(E, g ? K_SORT_GATHER : K_SORT_DOWNSWEEP);
         if (g)
             hipLaunchKernelGGL(k_sort_downsweep<true>, dim3(tiles), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_P),
-                               pph, ps, tiles, E->sort_status, passes, E->sort_ghist, gflags);
+                               pph, ps, tiles, E->sort_status, E->sort_totals, gflags);
         else
             hipLaunchKernelGGL(k_sort_downsweep<false>, dim3(tiles), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, ps, tiles, E->sort_status, passes, E->sort_ghist, gflags);
+                               E->tab(SP_P), pph, ps, tiles, E->sort_status, E->sort_totals, gflags);
         launch_end(E, g ? K_SORT_GATHER : K_SORT_DOWNSWEEP);
     }
-    E->ghist_clean = true;  // the last pass cleared the histograms
+    if (onesweep)
+        E->ghist_clean = true;  // the last pass cleared the histograms
 }
 
 }  // namespace dogm_hip
