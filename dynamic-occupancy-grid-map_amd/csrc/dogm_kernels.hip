@@ -583,12 +583,33 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
     const float* free_src = d.free[0];
     const float one = 1.0f;
     float m_occ_pred = 0.0f;
-    const bool occupied = d.start[c] != -1;
+    // Everything a cell reads is loaded before the first branch on it or store (75% of the wave cycles were
+    // waits, for one load after the other).
+    const int start = d.start[c], end = d.end[c];
+    const unsigned long long was = zero_empty == 3 && d.nz_valid ? d.nz[c >> 6] : ~0ull;
+    const float prior = d.wcell ? d.part[pph ^ 1].weight[0] : 0.0f;
+    const dogm_measurement_cell mc = d.meas_in ? d.meas_in[c] : d.meas[c];
+    float fprev;
+    if (d.shifted)
+    {
+        const int x = c % gs, y = c / gs;
+        const int sx = x + d.gx, sy = y + d.gy;
+        fprev = (sx > 0 && sx < gs && sy > 0 && sy < gs) ? free_src[sx + gs * sy] : 0.0f;
+    }
+    else if (d.xform_g)
+    {
+        const int sc = ego_source_cell(c, gs, d.xt);
+        fprev = sc >= 0 ? free_src[sc] : 0.0f;
+    }
+    else
+    {
+        fprev = free_src[c];
+    }
+    const bool occupied = start != -1;
     bool zero_fields = !occupied && zero_empty;
     if (zero_empty == 3)
     {
         // Work-table units are 256 cells, so each wave covers one aligned 64-cell word.
-        const unsigned long long was = d.nz_valid ? d.nz[c >> 6] : ~0ull;
         zero_fields = zero_fields && ((was >> (c & 63)) & 1ull);
         const unsigned long long now = __ballot(occupied);
         if ((c & 63) == 0)
@@ -598,9 +619,9 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
     int n_in = 0, n_out = 0;
     if (occupied && d.wcell)
     {
-        w_in = d.ps * d.part[pph ^ 1].weight[0];
+        w_in = d.ps * prior;
         n_out = border_cell(c, gs) ? border_out(d)[c] : 0;
-        n_in = d.end[c] - d.start[c] + 1 - n_out;
+        n_in = end - start + 1 - n_out;
         m_occ_pred = fx_to_f32(fx_from_f32(w_in) * n_in);
     }
     else if (occupied)
@@ -609,7 +630,7 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
         m_occ_pred = d.m_raw[c];
         if (m_occ_pred != m_occ_pred)  // marked: the cell crosses reduction tiles
         {
-            const int ts = d.start[c] / OT, te = d.end[c] / OT;
+            const int ts = start / OT, te = end / OT;
             const int t0 = d.u0[SP_P] / (OT / UNIT);
             fx_t sum = carry.tail_partial[t0 + ts];
             for (int t = ts + 1; t < te; ++t)
@@ -633,25 +654,8 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
     const float m_raw_c = m_occ_pred;  // Σw of the cell before the clamp
     if (m_occ_pred > one)
         m_occ_pred = one;
-    float fprev;
-    if (d.shifted)
-    {
-        const int x = c % gs, y = c / gs;
-        const int sx = x + d.gx, sy = y + d.gy;
-        fprev = (sx > 0 && sx < gs && sy > 0 && sy < gs) ? free_src[sx + gs * sy] : 0.0f;
-    }
-    else if (d.xform_g)
-    {
-        const int sc = ego_source_cell(c, gs, d.xt);
-        fprev = sc >= 0 ? free_src[sc] : 0.0f;
-    }
-    else
-    {
-        fprev = free_src[c];
-    }
     // The step's measurement grid, copied into the vehicle's buffer on the way when it comes from
     // the caller's device buffer (dogm.cu:205-215).
-    const dogm_measurement_cell mc = d.meas_in ? d.meas_in[c] : d.meas[c];
     if (d.meas_in)
         stream_store(&d.meas[c], mc);
     if ((zero_empty & 1) && occupied && !d.wcell)
