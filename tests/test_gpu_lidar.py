@@ -131,3 +131,49 @@ def test_server_scan_frames_match_plain_handles():
                 assert_grid_equal(f"frame {f} vehicle {k}", srv.get_grid_cells(ids[k]), plains[k].get_grid_cells())
     for lid in lidars.values():
         lid.close()
+
+
+@pytest.mark.parametrize("gs,n_beams", [(1187, 700), (1217, 1100)])
+def test_generate_many_beyond_the_cache(gs, n_beams):
+    """Calls of more than 256 MB take the tiles (ragged last tiles; more beams than a workgroup's threads): equal to
+    grids generated one by one, bit for bit, also for directions and ranges that no scanner gives; two of
+    them against the checker."""
+    res, max_range = 0.1, 70.0
+    count = (256 << 20) // (gs * gs * 16) + 1
+    rng = np.random.default_rng(gs)
+    ang = 2.0 * np.pi * np.arange(n_beams) / n_beams
+    cs, sn = np.cos(ang), np.sin(ang)
+    cs[::50], sn[::50] = 0.0, 0.0
+    cs[1::50] *= 37.0
+    cs[2::50], sn[2::50] = np.nan, 1e300
+    cs[3::50], sn[3::50] = 1e-310, -1.0
+    cs[4::50], sn[4::50] = 1.0, 0.0
+    ranges = rng.uniform(-5.0, 90.0, (count, n_beams))
+    ranges[:, ::7] = np.nan
+    ranges[:, 1::7] = np.inf
+    ranges[:, 2::7] = 0.0
+    ranges[:, 3::7] = -np.inf
+    ranges[:, 4::7] = np.round(ranges[:, 4::7] / res) * res
+    cells = gs * gs
+    with Lidar(grid_size=gs, beam_count=n_beams, resolution=res, max_range=max_range, occ_mass=0.7, free_mass=0.4,
+               beam_cos=cs, beam_sin=sn) as lidar:
+        bufs = [DeviceBuffer(cells * 16) for _ in range(count)]
+        one = DeviceBuffer(cells * 16)
+        _say(f"lidar generate_many {count} x {gs}")
+        lidar.generate_many(ranges, [b.ptr for b in bufs])
+        for i in range(count):
+            got = _download(bufs[i], cells)
+            lidar.generate(ranges[i], one.ptr)
+            assert got.tobytes() == _download(one, cells).tobytes(), f"grid {i}"
+            if i in (0, count - 1):
+                want = oc.lidar_grid(gs, res, max_range, 0.7, 0.4, cs, sn, ranges[i])
+                assert got.tobytes() == want.tobytes(), f"grid {i}"
+        # The same buffer twice: marks of both scans, as in a small call.
+        _say("lidar generate_many, one buffer twice")
+        lidar.generate_many(ranges, [bufs[0].ptr] * 2 + [b.ptr for b in bufs[2:]])
+        twice = _download(bufs[0], cells)
+        lidar.generate_many(ranges[:2], [one.ptr] * 2)
+        assert twice.tobytes() == _download(one, cells).tobytes()
+        for b in bufs:
+            b.free()
+        one.free()
