@@ -47,20 +47,19 @@ def kernel_bytes(name: str, N: int, B: int, C: int, passes: int) -> float | None
     """Algorithmic bytes one launch must move per vehicle (read once what it consumes, write once what
     it hands on); gathers through cell indices count their payload once."""
     table = {
-        # ancestor index, its 16 B state and association in; state, idx and association out (the
-        # resampling leaves the new set as ancestors, read here; the prior weights are equal after every
-        # resampling, so predict leaves them in place and the gathering pass forms the predicted weights)
-        "predict": 42 * N,
+        # ancestor index, its 16 B state and association in; state and cell word (with the association) out
+        # (the resampling leaves the new set as ancestors, read here; the prior weights are equal after
+        # every resampling, so the occupancy update forms the weights per cell)
+        "predict": 41 * N,
         "sort_downsweep": 16 * N,                # a pass before the last: keys + values in and out
-        # the last pass: keys + values in, the 16 B state gathered, sorted particles (25 B) out (the
-        # weight copy is skipped: the persistent update of the same step rewrites it)
-        "sort_gather": (8 + 16 + 25) * N,
-        "seg_occ": 8 * N,                        # keys + weights
-        # start, free, meas occ/free in; 6 fields out; the step's measurement grid copied from the
+        # the last pass: keys + values in, the 16 B state gathered, sorted particles without their weights
+        # (21 B) out
+        "sort_gather": (8 + 16 + 21) * N,
+        "cell_bounds": 4 * N + 8 * C,            # cell words in, first and last particle of a cell out
+        # start, end, free, meas occ/free in; 6 fields out; the step's measurement grid copied from the
         # caller's device buffer on the way (16 B in, 16 B out per cell)
-        "mass_update": 72 * C,
-        "seg_pers": 12 * N,                      # keys + weights in, likelihood-weighted weights out
-        "seg_moments": 24 * N,                   # keys, lik-weighted and prior weights, vx, vy in; posterior out
+        "mass_update": 76 * C,
+        "seg_moments": 16 * N,                   # cell words, vx, vy in; posterior weights out
         "rs_merge": 8 * N + 4 * B,               # joint weights in; ancestor indices out
         "birth_particles": 25 * B,
         "birth_cells": 20 * C,
@@ -72,9 +71,9 @@ def kernel_bytes(name: str, N: int, B: int, C: int, passes: int) -> float | None
 
 # Profiled kernel names (rocprofv3) of the per-kernel timers.
 PROFILED_NAME = {
-    "predict": "k_predict", "seg_occ": "k_segreduce<OccOp>", "seg_pers": "k_segreduce<PersOp>",
-    "seg_moments": "k_moments<4>", "mass_update": "k_mass_update", "rs_merge": "k_rs_merge_exact",
-    "birth_cells": "k_scan_apply<SrcBorn,SinkBirth>",
+    "predict": "k_predict", "cell_bounds": "k_cell_bounds", "seg_moments": "k_moments",
+    "mass_update": "k_mass_update", "rs_merge": "k_rs_merge_exact", "birth_cells": "k_birth_cells",
+    "birth_particles": "k_birth_particles",
 }
 # The scatter and gathering passes of the radix sort, by the pass form the tuning gives the step.
 SORT_PROFILED_NAME = {
