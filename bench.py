@@ -424,7 +424,7 @@ def run_generation(args, b, ids, sc, total):
     return {"grids_per_s": round(grids / el, 1), "us_per_call": round(el / reps * 1e6, 2), "grids_per_call": len(ids),
             "algorithmic_bytes_per_grid": int(per_grid),
             "achieved_GBs_wall": round(per_grid * grids / el / 1e9, 1),
-            "note": "wall time of blocking calls (ranges upload, three launches, stream wait)"}
+            "note": "wall time of blocking calls (ranges upload, launches, stream wait)"}
 
 
 def run_extraction(args, b, ids, p, step, first_frame):
