@@ -225,8 +225,8 @@ __device__ __forceinline__ int clamp_cell(float x, int gs)
 // flags (WORD_FLAGS), so the sort's first pass reads one word per particle and no association byte.
 // Border cells: the cells whose coordinate predict clamps to, so the only ones that can hold out-of-grid
 // particles (weight 0) beside in-grid ones.  For vehicles with per-cell weights their out-of-grid particles
-// are counted in m_raw (as ints), which such vehicles do not use otherwise: zeroed beside predict, counted
-// by k_cell_bounds, read by the occupancy update.
+// are counted in the born masses (as ints), which the occupancy update rewrites cell by cell after it has read
+// the cell's count: zeroed beside predict, counted by k_cell_bounds.
 __device__ __forceinline__ bool border_cell(int c, int gs)
 {
     const int y = c / gs, x = c - y * gs;
@@ -234,7 +234,7 @@ __device__ __forceinline__ bool border_cell(int c, int gs)
 }
 __device__ __forceinline__ int* border_out(const VehDesc& d)
 {
-    return reinterpret_cast<int*>(d.m_raw.get());
+    return reinterpret_cast<int*>(d.born.get());
 }
 
 // start = end = -1 for the cells of work-table group `group` (THREADS x 4 cells), four cells per
@@ -688,6 +688,9 @@ __device__ __forceinline__ float mass_update_cell(const VehDesc& d, int c, int z
         d.f[GF_MU_A][c] = mu_A;
         d.f[GF_MU_UA][c] = mu_UA;
         d.cellrec[c] = make_float4(a * lwi + b * wi, a * lwo + b * wo, rho_p, 0.0f);
+        // As the general path leaves it: an occupancy update on its own, after the resampling moved the particles,
+        // reads it for cells that hold none now.
+        stream_store(&d.m_raw[c], m_raw_c);
     }
     stream_store(&d.born[c], rho_b);
     stream_store(&d.f[GF_PERS][c], rho_p);

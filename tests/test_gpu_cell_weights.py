@@ -97,6 +97,33 @@ def test_stage_calls_after_full_updates():
         orc.close()
 
 
+@pytest.mark.parametrize("gs,n", [(1, 63), (5, 257), (33, 1000), (64, 700)])
+def test_single_stages_after_full_updates(gs, n):
+    """An occupancy update on its own, straight after full updates, reads the sums that both paths leave per cell: the
+    cells the resampling emptied have no particles to sum.  Without births the resampled sets stay sorted, and in one
+    reduction tile no cell's particles are cut, so what the stage sums does not depend on the bounds of the last sort."""
+    p = small_params(gs=gs, res=0.5, n=n, b=0)
+    rng = np.random.default_rng(gs)
+    with DOGM(p, seed=SEED) as cells, DOGM(p, seed=SEED) as general:
+        for f in range(5):
+            m = _grid(gs, rng)
+            m["likelihood"] = rng.choice([0.05, 5.0], gs * gs)  # cells lose all their particles
+            if f:
+                general.set_particles(weight=general.get_particles()["weight"])
+            for g in (cells, general):
+                g.update_grid(m, 0.4 * f, 3.0 * gs if f == 3 else 0.0, 0.0, 0.1)
+                if f % 2:
+                    continue
+                if f == 4:
+                    g.update_pose(0.4 * f + 1.1, 0.0, 0.0)  # moves the cells' particle ranges as well
+                g.grid_cell_occupancy_update(0.1)
+                g.resampling()
+            assert_vehicle_equal(f"frame {f}", cells.get_particles(), general.get_particles(),
+                                 cells.get_grid_cells(), general.get_grid_cells())
+            a, c = cells.get_born_masses().view(np.uint32), general.get_born_masses().view(np.uint32)
+            np.testing.assert_array_equal(a, c)
+
+
 def test_batch_mixes_both_paths():
     """A vehicle whose weights are not uniform beside one whose weights are, in the same launches."""
     ps = [small_params(gs=g, res=0.5, n=n, b=n // 10) for g, n in ((40, 9000), (24, 5000), (64, 20000))]
