@@ -769,6 +769,7 @@ constexpr int SCAN_Q = SCAN_TILE / UNIT;  // units per scan tile
 //   __device__ bool active(const VehDesc& d) const;                   // vehicle takes part
 //   __device__ int len(const VehDesc& d) const;                       // elements of the vehicle
 //   __device__ void load4(const VehDesc& d, int p0, int cnt, float (&v)[4]) const;
+//   __device__ void seen(int vehicle, const float (&v)[4], fx_t incl) const;  // four values, prefix in the tile
 // A CDF segment is one wave's share of a scan tile.  With seg_end set, the tile-local inclusive end
 // of every segment is written at seg_end[CDF_SEGS_PER_TILE * tile + segment]; with the tile's prefix added (the
 // merge does that as it reads them) these are the vehicle's inclusive segment ends: the resampling CDF index.
@@ -838,6 +839,7 @@ __device__ __forceinline__ void scan_tile_body(const Src& src, const VehDesc* __
             s += Src::kNonNeg ? fx_from_f32_nonneg(v[i]) : fx_from_f32(v[i]);
     fx_t total;
     const fx_t ex = block_exclusive_scan_fx(s, &total);
+    src.seen(tr.v, v, ex + s);
     if (threadIdx.x == 0)
         tile_sum[tile] = total;
     if (seg_end && (threadIdx.x & (WAVE - 1)) == WAVE - 1)
@@ -898,12 +900,13 @@ __device__ __forceinline__ fx_t scan_tile_total(const fx_t* __restrict__ tile_su
 
 // Exclusive prefix of the ntiles tile totals from t0 on, by NT threads (thread `tid` of the group, s_wave its LDS);
 // tile_pre may be tile_sum.  Every thread of the workgroup takes part, in `rounds` rounds of
-// TOP_ITEMS consecutive tiles per thread (enough for the longest group).  Returns the total.
+// TOP_ITEMS consecutive tiles per thread (enough for the longest group).  Returns the total; seen() gets the
+// inclusive prefixes.
 constexpr int TOP_ITEMS = 4;
 
-template <int NT>
+template <int NT, class Seen>
 __device__ __forceinline__ fx_t scan_tile_prefixes(const fx_t* tile_sum, fx_t* tile_pre, int t0, int ntiles, int parts,
-                                                   int tid, int rounds, fx_t* s_wave)
+                                                   int tid, int rounds, fx_t* s_wave, const Seen& seen)
 {
     fx_t carry = 0;
     for (int r = 0; r < rounds; ++r)
@@ -925,6 +928,7 @@ __device__ __forceinline__ fx_t scan_tile_prefixes(const fx_t* tile_sum, fx_t* t
             if (b + k < ntiles)
                 tile_pre[t0 + b + k] = run;
             run += x[k];
+            seen(run);
         }
         carry += total;
     }
@@ -949,7 +953,7 @@ __device__ __forceinline__ void scan_top_orders(const VehDesc* __restrict__ desc
         return;  // uniform over the workgroup
     const int ntiles = d.nu[SP_C] / SCAN_Q;
     const fx_t total = scan_tile_prefixes<NT>(tile_sum, tile_pre, d.u0[SP_C] / SCAN_Q, ntiles, parts, threadIdx.x,
-                                              top_rounds(ntiles, NT), s_wave);
+                                              top_rounds(ntiles, NT), s_wave, [](fx_t) {});
     if (threadIdx.x == 0)
     {
         const int n = mode == SCAN_ORDERS_N ? d.N : d.B;

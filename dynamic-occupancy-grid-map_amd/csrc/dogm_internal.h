@@ -207,6 +207,8 @@ struct DevScalars
     double scale;      // particle-order scale v / total
     double ftotal;     // resampling, float CDF modes: the CDF total (envelope maximum)
     float new_weight;  // resampling: f32 of the CDF total over N
+    int beyond_tiles;  // resampling: a weight or tile is beyond the merge's keys (cleared by the top-level scan)
+    int beyond_keys;   // resampling: one is, or the CDF
     int born_odd;      // a born mass of this step is negative, NaN or above BORN_MAX (k_mass_update)
 };
 

@@ -1000,6 +1000,7 @@ struct SrcBorn
     __device__ bool active(const VehDesc& d) const { return !init_only || d.init; }
     __device__ int len(const VehDesc& d) const { return d.C; }
     __device__ void load4(const VehDesc& d, int p0, int cnt, float (&v)[4]) const { load_run<4>(d.born, p0, cnt, v); }
+    __device__ void seen(int, const float (&)[4], fx_t) const {}
 };
 
 __device__ __forceinline__ int order_end_at(int j, fx_t prefix, const DevScalars* sc, int C, int v)

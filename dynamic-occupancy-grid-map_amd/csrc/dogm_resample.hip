@@ -40,9 +40,25 @@ constexpr int FSUM_STRIDE = sizeof(fx_t) / sizeof(double);
 
 static_assert(RS_TILE == SCAN_TILE, "draw tiles and CDF tiles share the exact-scan tile size");
 
+// What the merge's window keys cover: joint weights below 2^37 and a CDF below 2^38.  Four such weights (a thread's) sum
+// to less than 2^39, so the first prefix outside the range shows as one at or above 2^38 or, wrapped, below 0.
+constexpr float KEY_WEIGHT_MAX = 0x1p37f;
+
+__device__ __forceinline__ bool beyond_keys(fx_t prefix)
+{
+    return (prefix >> (38 + FX_FRAC)) != 0;
+}
+
 struct SrcJointPos
 {
     static constexpr bool kNonNeg = true;  // cdf_weight: +0 or positive
+    DevScalars* scs;                       // null where the weights are only read again
+    // Marks a vehicle beyond the keys (k_scan_top_resample clears the mark).
+    __device__ void seen(int vehicle, const float (&v)[4], fx_t incl) const
+    {
+        if (fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])) >= KEY_WEIGHT_MAX || beyond_keys(incl))
+            scs[vehicle].beyond_tiles = 1;
+    }
     __device__ bool active(const VehDesc& d) const { return d.cdf_mode == CDF_EXACT; }
     __device__ int len(const VehDesc& d) const { return d.N + d.B; }
     __device__ void load4(const VehDesc& d, int p0, int cnt, float (&v)[4]) const
@@ -137,7 +153,7 @@ __device__ __forceinline__ void tile_float_scan(const VehDesc& d, int p0, int cn
     __shared__ T s_w[BLOCK / WAVE];
     float f[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (cnt > 0)
-        SrcJointPos{}.load4(d, p0, cnt, f);
+        SrcJointPos{nullptr}.load4(d, p0, cnt, f);
     T run = (T)0;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -581,7 +597,7 @@ __device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const SegEn
     const int cnt = max(0, min(SCAN_ITEMS, J - q0));
     float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (cnt > 0)
-        SrcJointPos{}.load4(d, q0, cnt, f);
+        SrcJointPos{nullptr}.load4(d, q0, cnt, f);
     fx_t v[SCAN_ITEMS];
     fx_t sum = 0;
 #pragma unroll
@@ -601,6 +617,176 @@ __device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const SegEn
     return s * CDF_SEG + below;
 }
 
+// The merge of a vehicle whose CDF is beyond the window keys (infinite weights count 2^38).  The 128-bit entries of
+// `segs` segments (a window: 4 or 8) are rebuilt and searched, four segments at a time in the workgroup's 16 KB; a
+// draw is resolved in the first window whose last entry is >= its value, by a branch-free binary search over
+// the window padded to a power of two.  While the CDF is non-decreasing that is its lower bound.  Past the
+// fixed-point range the sums wrap and the answer depends on the probes, so their order is fixed: the whole coarse
+// index first, windows of a given length, halved from the front.
+// 2.2e5 joint weights, one of them infinite: 12.4 us (one by one, with wave_exact_ancestor, 457).
+__device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevScalars* sc, const SegEnds& seg_end,
+                                                  int pph, int base, int n, int J,
+                                                  const fx_t* __restrict__ exp_tile_pre, int segs, uint64_t* s_mem)
+{
+    constexpr int NWAVE = BLOCK / WAVE;
+    constexpr int HALF = NWAVE * CDF_SEG;  // entries staged at once, a segment per wave
+    static_assert(HALF == RS_TILE, "the entries' bytes also stage the draws");
+    __shared__ fx_t s_rb[2], s_wr[NWAVE];
+    __shared__ int s_wmin[NWAVE];
+    int64_t* s_hi64 = reinterpret_cast<int64_t*>(s_mem);
+    uint64_t* s_lo64 = s_mem + HALF;
+    const int lane = threadIdx.x & (WAVE - 1), wid = wave_index();
+    const auto put = [=](int i, fx_t x) {
+        s_hi64[i] = (int64_t)(x >> 64);
+        s_lo64[i] = (uint64_t)x;
+    };
+    const auto get = [=](int i) { return (fx_t)(((ufx_t)(uint64_t)s_hi64[i] << 64) | (ufx_t)s_lo64[i]); };
+    const Spacing sp = sc->spacing;
+    fx_t r[RS_ITEMS];
+    if (d.draw_mode == DRAW_SYSTEMATIC)
+    {
+        const uint32_t u = systematic_u32(d.seed, d.inst, d.ep_rs);
+#pragma unroll
+        for (int i = 0; i < RS_ITEMS; ++i)
+            r[i] = spacing_draw_nonneg(systematic_s(base + (int)threadIdx.x + i * BLOCK, u), sp);
+    }
+    else
+    {
+        spacing_prefixes(d, base, n, exp_tile_pre,
+                         [&](int i, fx_t s_k) { put(threadIdx.x * RS_ITEMS + i, spacing_draw_nonneg(s_k, sp)); });
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < RS_ITEMS; ++i)
+            r[i] = get(threadIdx.x + i * BLOCK);
+    }
+    const int last = min(base + RS_TILE, n) - 1;
+    int anc[RS_ITEMS];
+#pragma unroll
+    for (int i = 0; i < RS_ITEMS; ++i)
+    {
+        const int k = base + (int)threadIdx.x + i * BLOCK;
+        anc[i] = -1;
+        if (k == base)
+            s_rb[0] = r[i];
+        if (k == last)
+            s_rb[1] = r[i];
+    }
+    __syncthreads();
+    int s_lo, s_hi;
+    wave_find2<fx_t>(seg_end, seg_end.segs, s_rb[0], s_rb[1], &s_lo, &s_hi);
+    for (int s0 = s_lo; s0 <= s_hi;)
+    {
+        const int s1 = min(s0 + segs, s_hi + 1);  // window: segments [s0, s1)
+        const int c0 = s0 * CDF_SEG;
+        const int clen = min(J, s1 * CDF_SEG) - c0;
+        const fx_t cmax = seg_end(s1 - 1), next_max = seg_end(min(s1 - 1 + segs, s_hi));
+        const bool two = clen > HALF;
+        const fx_t mid = two ? seg_end(s0 + NWAVE - 1) : (fx_t)0;  // entry HALF - 1: the first probe
+        const int span = clen > 1 ? 1 << (32 - __clz(clen - 1)) : 1;
+        // The weights and prefixes of both halves are in flight together.
+        float f[2][SCAN_ITEMS];
+        fx_t before[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            const int s = s0 + h * NWAVE + wid;
+            const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
+#pragma unroll
+            for (int i = 0; i < SCAN_ITEMS; ++i)
+                f[h][i] = 0.0f;
+            if (s < s1 && q0 < J)
+                SrcJointPos{nullptr}.load4(d, q0, min(SCAN_ITEMS, J - q0), f[h]);
+            before[h] = s < s1 && s > 0 ? seg_end(s - 1) : (fx_t)0;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            if (h == 1 && !two)
+                break;
+            __syncthreads();  // the searches (and the draws' staging) before are done
+            fx_t v[SCAN_ITEMS];
+            fx_t sum = 0;
+#pragma unroll
+            for (int i = 0; i < SCAN_ITEMS; ++i)
+            {
+                v[i] = fx_from_f32_nonneg(f[h][i]);  // cdf_weight: sign bit clear; 0 past the entries
+                sum += v[i];
+            }
+            fx_t run = wave_inclusive_scan_fx(sum) - sum + before[h];
+#pragma unroll
+            for (int i = 0; i < SCAN_ITEMS; ++i)
+            {
+                run += v[i];
+                put(wid * CDF_SEG + lane * SCAN_ITEMS + i, run);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < RS_ITEMS; ++i)
+            {
+                const bool upper = two && mid < r[i];
+                if (anc[i] >= 0 || base + (int)threadIdx.x + i * BLOCK > last || cmax < r[i] || upper != (h != 0))
+                    continue;
+                // lo counts the entries below the draw; past the window the last entry stands for the ones missing.
+                int lo = h * HALF;
+                for (int step = two ? HALF / 2 : span >> 1; step > 0; step >>= 1)
+                    if (get(min(lo + step, clen) - 1 - h * HALF) < r[i])
+                        lo += step;
+                anc[i] = c0 + lo;
+            }
+        }
+        if (s1 > s_hi)
+            break;
+        // The smallest unresolved draw: each wave's minimum (draw indices are distinct, so one lane holds it) with its
+        // value, then the minimum over the waves.
+        int mine = n;
+        fx_t rmine = 0;
+#pragma unroll
+        for (int i = RS_ITEMS - 1; i >= 0; --i)
+        {
+            const int k = base + (int)threadIdx.x + i * BLOCK;
+            if (anc[i] < 0 && k <= last)
+            {
+                mine = k;
+                rmine = r[i];
+            }
+        }
+        int wmin = mine;
+#pragma unroll
+        for (int o = WAVE / 2; o > 0; o >>= 1)
+            wmin = min(wmin, __shfl_xor(wmin, o, WAVE));
+        if (wmin < n && mine == wmin)
+            s_wr[wid] = rmine;
+        if (lane == 0)
+            s_wmin[wid] = wmin;
+        __syncthreads();
+        int kmin = n, kw = 0;
+#pragma unroll
+        for (int w = 0; w < NWAVE; ++w)
+        {
+            const int x = s_wmin[w];
+            if (x < kmin)
+            {
+                kmin = x;
+                kw = w;
+            }
+        }
+        if (kmin >= n)
+            break;
+        const fx_t rmin = s_wr[kw];
+        if (!(next_max < rmin))
+        {
+            s0 = s1;
+        }
+        else
+        {
+            int c, unused;
+            wave_find2<fx_t>(seg_end, seg_end.segs, rmin, rmin, &c, &unused);
+            s0 = max(s1, c);
+        }
+    }
+    merge_write(d, sc, pph, base, n, J, anc);
+}
+
 // Exact-CDF merge.  The workgroup's ancestors lie in the CDF segments [s_lo, s_hi] holding its first and
 // last draw; they are staged WSEG segments at a time (a window).  The answer is the exact lower bound in the 128-bit
 // CDF, but nearly every comparison is decided by far fewer bits: a window stages one 31-bit key per entry,
@@ -613,8 +799,10 @@ __device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const SegEn
 //     keys are exact.
 //   - A draw within 1 of an entry's key (about 3e-6 of them: a window holds at most 2048 of 2^30 keys, and draws
 //     fall in proportion to the CDF) is resolved by wave_exact_ancestor.
-//   - A window whose sums could leave the fixed-point range (a weight of 2^27 or more, or a wrapped CDF), or
-//     whose total is below 2^-66 of the CDF before it, sends all remaining draws there.
+//   - A window whose total is below 2^-66 of a CDF above 2^107 raw units before it sends the draws that land in it
+//     there (a draw lands in a window in proportion to its total).
+//   - A vehicle with a weight of 2^37 or more, or with a CDF of 2^38 or more, may have sums that leave the fixed-point
+//     range, which these bounds do not cover: merge_beyond_keys.
 // Draws are sorted, so the resolved ones are a prefix: the next window starts at the segment of the first draw left.
 // Bound by the vector ALU (Philox and logarithms of the draws, searches).  Before, windows held 128-bit
 // entries (four 128-bit conversions and adds per lane and segment, 128-bit scans and two-word probes).
@@ -625,15 +813,18 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
                                                           const fx_t* __restrict__ exp_tile_pre,
                                                           const fx_t* __restrict__ seg_local,
                                                           const fx_t* __restrict__ cdf_pre,
-                                                          const DevScalars* __restrict__ scs)
+                                                          const DevScalars* __restrict__ scs, int beyond_segs)
 {
     constexpr int WLEN = WSEG * CDF_SEG;
     constexpr int NWAVE = BLOCK / WAVE;
     constexpr uint32_t PAD = 0xffffffffu;  // above every draw's key
     static_assert((WLEN & (WLEN - 1)) == 0, "the search halves the window");
-    __shared__ double s_r[RS_TILE];  // the draws in raw units
-    __shared__ __attribute__((aligned(16))) uint32_t s_key[WLEN];  // keys + margin
-    __shared__ int s_big[NWAVE], s_done[NWAVE];
+    // The draws in raw units and the window's keys + margin; merge_beyond_keys takes the same bytes.
+    constexpr int MEM = RS_TILE + WLEN / 2 > 2 * RS_TILE ? RS_TILE + WLEN / 2 : 2 * RS_TILE;
+    __shared__ __attribute__((aligned(16))) uint64_t s_mem[MEM];
+    double* s_r = reinterpret_cast<double*>(s_mem);
+    uint32_t* s_key = reinterpret_cast<uint32_t*>(s_mem + RS_TILE);
+    __shared__ int s_done[NWAVE];
 
     const TileRef tr = tile_ref(tab, RS_TILE / UNIT, blockIdx.x);
     const VehDesc& d = descs[tr.v];
@@ -643,6 +834,14 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
         return;
     const DevScalars* sc = scs + tr.v;
     const int J = n + d.B;
+    const int t0 = d.u0[SP_J] / SCAN_Q;
+    const SegEnds seg_end{seg_local + (size_t)t0 * CDF_SEGS_PER_TILE, cdf_pre + t0, sc->cdf_total,
+                          (J + SCAN_TILE - 1) / SCAN_TILE, (J + CDF_SEG - 1) / CDF_SEG};
+    if (sc->beyond_keys)
+    {
+        merge_beyond_keys(d, sc, seg_end, pph, base, n, J, exp_tile_pre, beyond_segs, s_mem);
+        return;
+    }
     const int cnt_draws = min(RS_TILE, n - base);
     const int wid = threadIdx.x / WAVE;
     const int lane = threadIdx.x & (WAVE - 1);
@@ -669,9 +868,6 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
         anc[i] = threadIdx.x + i * BLOCK < cnt_draws ? -1 : 0;
-    const int t0 = d.u0[SP_J] / SCAN_Q;
-    const SegEnds seg_end{seg_local + (size_t)t0 * CDF_SEGS_PER_TILE, cdf_pre + t0, sc->cdf_total,
-                          (J + SCAN_TILE - 1) / SCAN_TILE, (J + CDF_SEG - 1) / CDF_SEG};
     int s_lo, s_hi;
     seg_end.find2(draw_fx(s_r[0]), draw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
     for (int s0 = s_lo;;)
@@ -684,12 +880,11 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
         const int m = W > 0 ? 127 - clz128((ufx_t)W) : 0;
         const int mb = B0 > 0 ? 127 - clz128((ufx_t)B0) : 0;
         // Two doubles hold B0 exactly up to 107 bits, and to 2^-40 W while m >= mb - 66.
-        const bool odd = B0 < 0 || W < 0 || (mb > 106 && m < mb - 66);
+        const bool exact = mb > 106 && m < mb - 66;
         const double g = ldexp(1.0, 30 - m);
         const uint32_t margin = m <= 30 ? 0u : 1u;
-        const double b_hi = odd ? 0.0 : fx_raw_f64(B0);
-        const double b_lo = odd ? 0.0 : fx_raw_f64(B0 - draw_fx(b_hi));
-        bool big = odd;
+        const double b_hi = exact ? 0.0 : fx_raw_f64(B0);
+        const double b_lo = exact ? 0.0 : fx_raw_f64(B0 - draw_fx(b_hi));
 #pragma unroll
         for (int q = 0; q < WSEG / NWAVE; ++q)
         {
@@ -701,14 +896,13 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
                 const int cnt = max(0, min(SCAN_ITEMS, J - q0));
                 float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
                 if (cnt > 0)
-                    SrcJointPos{}.load4(d, q0, cnt, f);
+                    SrcJointPos{nullptr}.load4(d, q0, cnt, f);
                 double v[SCAN_ITEMS];
                 raw_weights(f, v);
                 double sum = v[0];
 #pragma unroll
                 for (int i = 1; i < SCAN_ITEMS; ++i)
                     sum += v[i];
-                big |= fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])) >= 0x1p27f;
                 const fx_t before = s > s0 ? seg_end(s - 1) - B0 : (fx_t)0;
                 double run = wave_inclusive_scan_val(sum) - sum + fx_raw_f64(before);
 #pragma unroll
@@ -722,14 +916,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             *reinterpret_cast<uint4*>(&s_key[(q * NWAVE + wid) * CDF_SEG + lane * SCAN_ITEMS]) =
                 make_uint4(key[0], key[1], key[2], key[3]);
         }
-        const bool any_big = __ballot(big) != 0;
-        if (lane == 0)
-            s_big[wid] = any_big;
         __syncthreads();
-        bool exact = false;
-#pragma unroll
-        for (int w = 0; w < NWAVE; ++w)
-            exact |= s_big[w] != 0;
         // Keys below rk - margin (staged: below rk) are below the draw, keys from rk + 2 margin on are not.  The
         // thread's searches go step by step together (four LDS reads in flight).
         uint32_t rk[RS_ITEMS];
@@ -928,14 +1115,21 @@ __global__ __launch_bounds__(TOP_BLOCK) void k_scan_top_resample(const VehDesc* 
     constexpr int HALF = TOP_BLOCK / 2;
     __shared__ fx_t s_wave[2][HALF / WAVE];
     __shared__ fx_t s_total[2];
+    __shared__ int s_beyond;
     const VehDesc& d = descs[blockIdx.x];
+    if (threadIdx.x == 0)
+        s_beyond = 0;
     const int half = threadIdx.x / HALF, tid = threadIdx.x % HALF;
     const int nj = d.cdf_mode == CDF_EXACT ? d.nu[SP_J] / SCAN_Q : 0;
     const int ne = d.draw_mode == DRAW_MULTINOMIAL ? d.nu[SP_E] / SCAN_Q : 0;
     const int rounds = max(top_rounds(nj, HALF), top_rounds(ne, HALF));
+    bool beyond = false;
     const fx_t total = scan_tile_prefixes<HALF>(half ? exp_sum : cdf_sum, half ? exp_pre : cdf_sum,
                                                 half ? d.u0[SP_E] / SCAN_Q : d.u0[SP_J] / SCAN_Q, half ? ne : nj, 1, tid,
-                                                rounds, s_wave[half]);
+                                                rounds, s_wave[half],
+                                                [&](fx_t prefix) { beyond |= beyond_keys(prefix); });
+    if (beyond && half == 0)
+        s_beyond = 1;
     if (tid == 0)
         s_total[half] = total;
     __syncthreads();
@@ -946,6 +1140,8 @@ __global__ __launch_bounds__(TOP_BLOCK) void k_scan_top_resample(const VehDesc* 
         // Systematic draws do not use the exponentials: S_N = N * 2^32 (dogm_numerics.h).
         sc->spacing = spacing_setup(ne ? s_total[1] : systematic_s(d.N, 0u), cdf_total);
         sc->cdf_total = cdf_total;
+        sc->beyond_keys = sc->beyond_tiles | s_beyond;
+        sc->beyond_tiles = 0;
         if (nj)
         {
             const float jm = fx_to_f32(cdf_total);
@@ -964,7 +1160,7 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
     // then both top-level scans in one launch.
     launch_begin(E, K_SCAN_TILES);
     hipLaunchKernelGGL(k_scan_tiles_exp<SrcJointPos>, dim3(jtiles + etiles), dim3(BLOCK), 0, E->stream,
-                       SrcJointPos{}, E->tab(SP_J), jtiles, E->scan_tile_sum, E->cdf_tile_incl, E->tab(SP_E),
+                       SrcJointPos{E->scalars}, E->tab(SP_J), jtiles, E->scan_tile_sum, E->cdf_tile_incl, E->tab(SP_E),
                        E->exp_tile_sum, E->d_desc);
     launch_end(E, K_SCAN_TILES);
     launch_begin(E, K_SCAN_TOP);
@@ -996,15 +1192,19 @@ void run_resampling(Engine* E, int pph, int modes, bool exp_done)
 
     const int mt = E->tiles(SP_P, RS_TILE / UNIT);
     const bool wide = E->tune.merge_slice != 1;
+    // Windows of merge_beyond_keys: 8 segments for launches of up to 4096 workgroups, 4 for larger ones.
+    const int beyond_segs = (E->tune.merge_slice == 0 ? mt <= 4096 : wide) ? RS_WINDOW_WIDE : RS_WINDOW_NARROW;
     launch_begin(E, K_RS_MERGE);
     if (exact)
     {
         if (wide)
             hipLaunchKernelGGL(k_rs_merge_exact<RS_WINDOW_WIDE>, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars);
+                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars,
+                               beyond_segs);
         else
             hipLaunchKernelGGL(k_rs_merge_exact<RS_WINDOW_NARROW>, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc,
-                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars);
+                               E->tab(SP_P), pph, E->scan_tile_pre, E->cdf_tile_incl, E->scan_tile_sum, E->scalars,
+                               beyond_segs);
     }
     if (modes & ~(1 << CDF_EXACT))
         hipLaunchKernelGGL(k_rs_merge_float, dim3(mt), dim3(BLOCK), 0, E->stream, E->d_desc, E->tab(SP_P), pph,

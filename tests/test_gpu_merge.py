@@ -1,5 +1,7 @@
 """Ancestor search of the exact resampling on weights that reach every way a window is decided: keys that decide, keys
-that tie (exact resolution), totals small enough for exact keys, and weights beyond the keys' range."""
+that tie (exact resolution), totals small enough for exact keys, and weights and totals beyond the keys' range."""
+import hashlib
+
 import numpy as np
 import pytest
 
@@ -37,6 +39,14 @@ def _weights(kind, n, rng):
         return w
     if kind == "large":
         return np.where(rng.random(n) < 0.01, 2.0 ** 27, 1.0)
+    if kind == "key_limit":  # the largest weights that have keys
+        w = rng.random(n)
+        w[n // 2] = np.nextafter(np.float32(2.0 ** 37), np.float32(0))
+        return w
+    if kind == "total_beyond":  # a CDF between the keys' range (2^38) and the fixed-point range (2^39)
+        w = rng.random(n)
+        w[[n // 3, n // 2, 2 * n // 3]] = 2.0 ** 36.9
+        return w
     assert kind == "infinite"
     w = rng.random(n)
     w[n // 3] = np.inf
@@ -45,7 +55,7 @@ def _weights(kind, n, rng):
 
 @pytest.mark.parametrize("wide", [1, 2])
 @pytest.mark.parametrize("kind", ["uniform", "dominant", "decades", "raw_units", "below_units", "zero", "sparse",
-                                  "mixed_scales", "large", "infinite"])
+                                  "mixed_scales", "large", "key_limit", "total_beyond", "infinite"])
 @pytest.mark.parametrize("n,b", [(1, 0), (1023, 1), (1025, 300), (200_003, 20_001)])
 def test_ancestors(kind, n, b, wide):
     rng = np.random.default_rng(n)
@@ -71,3 +81,63 @@ def test_ancestors(kind, n, b, wide):
             orc.close()
     finally:
         tuning_override(None)
+
+
+# Ancestors of CDFs whose sums wrap (beyond 2^39) as first released: they depend on which entries the search probes.
+WRAPPED = {
+    ("infinite_two", 1025, 300): ("ef29790038c9", "ef29790038c9"),
+    ("infinite_two", 200_003, 20_001): ("762fa33b085f", "762fa33b085f"),
+    ("infinite_1%", 6000, 0): ("3e8b915fb856", "3e8b915fb856"),
+    ("infinite_1%", 200_003, 20_001): ("068ab73d0702", "068ab73d0702"),
+    ("infinite_1%", 5_000_000, 1000): ("251b9f0bf3e7", "a79b5bfba33a"),
+    ("huge", 200_003, 20_001): ("02ae56276f00", "f1957805289b"),
+}
+
+
+@pytest.mark.parametrize("kind,n,b", WRAPPED)
+def test_wrapped_sums(kind, n, b):
+    w = _wrapped_weights(kind, n + b, np.random.default_rng(n))
+    got = []
+    with DOGM(small_params(gs=16, res=0.5, n=n, b=b), seed=SEED) as gpu:
+        gpu.update_measurement_grid(small_scene(gs=16, res=0.5).measurement(0))
+        for draws in ("multinomial", "systematic"):
+            gpu.set_resampling_mode(draws)
+            gpu.set_weight_array(w[:n])
+            if b:
+                gpu.set_birth_particles(weight=w[n:])
+            gpu.resampling()
+            got.append(hashlib.sha1(gpu.get_resampled_indices().tobytes()).hexdigest()[:12])
+    assert tuple(got) == WRAPPED[kind, n, b]
+
+
+def _wrapped_weights(kind, n, rng):
+    w = rng.random(n).astype(np.float32)
+    if kind == "infinite_two":
+        w[[n // 3, 2 * n // 3]] = np.inf
+    elif kind == "infinite_1%":
+        w[rng.random(n) < 0.01] = np.inf
+    else:
+        w = (w + 1) * np.float32(2.0 ** 30)
+    return w
+
+
+@pytest.mark.parametrize("kind", ["large", "infinite"])
+def test_weights_beyond_the_keys_are_not_slow(kind):
+    """A window search, not one search per draw: measured at 1.5 times the time of ordinary weights and below; the bound
+    leaves room for a slow box, one search per draw takes 35 times as long."""
+    n, b = 200_003, 20_001
+    took = {}
+    with DOGM(small_params(gs=16, res=0.5, n=n, b=b), seed=SEED) as gpu:
+        gpu.update_measurement_grid(small_scene(gs=16, res=0.5).measurement(0))
+        gpu.set_kernel_timing("rs_merge")
+        for k in ("uniform", kind):
+            w = _weights(k, n + b, np.random.default_rng(n)).astype(np.float32)
+            ms = []
+            for _ in range(5):
+                gpu.set_weight_array(w[:n])
+                gpu.set_birth_particles(weight=w[n:])
+                gpu.reset_kernel_timing()
+                gpu.resampling()
+                ms.append(gpu.kernel_timing("rs_merge")[0])
+            took[k] = min(ms)
+    assert took[kind] < 8 * took["uniform"], took
