@@ -14,11 +14,12 @@
 //
 // Large calls take one launch (blockIdx.y = grid), a workgroup per square tile of cells: the beams that can cross the tile
 // are found, their samples inside it marked in LDS, and every cell is then written once.
-// Calls that this does not suit (lidar_tiled) take three launches, each over every grid of the call:
+// Calls that this does not suit (lidar_form) take three launches, each over every grid of the call:
 //   clear  16-byte stores of (0, 0, 1, 1) over the cells;
 //   free   one thread per (beam, step) sample: an idempotent 4-byte store of free_mass;
 //   occ    one thread per beam: occ_mass and free 0 at the return's cell (after every free store).
 #include "dogm_internal.h"
+#include "dogm_lidar_form.h"
 
 #include <algorithm>
 #include <cmath>
@@ -132,16 +133,18 @@ __global__ __launch_bounds__(BLOCK) void k_lidar_occ(dogm_measurement_cell* cons
 // left, and its return; then the waves take the queued beams in turn, a lane per sample.  The samples' positions
 // and cells are computed as in k_lidar_free; marks are plain byte stores, free and occupied apart, so
 // their order does not matter.
-// Writes the grids once (737 MB in 230 us), where the three launches write every cell and then 4-byte pieces of most
-// cache lines again; side 64 and 512 threads: 32 x 1200 x 1200 cells from 1080 beams 262 us, side 32 384, side 16 1118,
-// 1024 threads 292 (three launches 464).
+// Writes the grids once, where the three launches write every cell and then 4-byte pieces of most cache lines again.
+// Side 64 and 512 threads: 32 x 1200 x 1200 cells (737 MB) from 1080 beams 262 us, side 32 384, side 16 1118, 1024
+// threads 292 (three launches 464).  The tiles around the sensor walk every beam: a call of these grids from scans
+// of a scene takes 194 us with them first and 238 grid after grid, where the last grid's are still at it when all
+// is written (three launches 413).
 constexpr int LIDAR_TILE = 64;
 constexpr int LIDAR_THREADS = 512;
 
 __global__ __launch_bounds__(LIDAR_THREADS) void k_lidar_tiles(dogm_measurement_cell* const* __restrict__ outs,
                                                                const double* __restrict__ ranges,
                                                                const double* __restrict__ dir, LidarArgs a,
-                                                               int stride)
+                                                               int side, int count, int centre_first)
 {
     constexpr int T = LIDAR_TILE, THREADS = LIDAR_THREADS;
     __shared__ __attribute__((aligned(16))) uint8_t s_free[T * T];
@@ -150,9 +153,30 @@ __global__ __launch_bounds__(LIDAR_THREADS) void k_lidar_tiles(dogm_measurement_
     __shared__ int2 s_k[THREADS];
     __shared__ int s_n;
     const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
-    const int x0 = (int)(blockIdx.x % (unsigned)stride) * T, y0 = (int)(blockIdx.x / (unsigned)stride) * T;
-    if (x0 >= a.gs || y0 >= a.gs)
-        return;
+    const int id = (int)blockIdx.x;
+    int grid, tx, ty;
+    if (centre_first)
+    {
+        // Rows and columns of tiles outwards from the sensor's, all grids at each.
+        const int rank = id / count, mid = a.gs / 2 / T;
+        const auto outwards = [=](int r) { return (mid + ((r & 1) ? (r + 1) / 2 : side - r / 2)) % side; };
+        grid = id % count;
+        tx = outwards(rank % side);
+        ty = outwards(rank / side);
+    }
+    else
+    {
+        // Workgroups go to the 8 XCDs in turn.  An odd count along both sides spreads the busy middle tiles of every row
+        // and grid over them; at a multiple of 8 they fall to two (24 x 1024 x 1024 cells 348 us, 219 with the odd
+        // counts).
+        const int stride = side | 1, t = id % (stride * stride);
+        grid = id / (stride * stride);
+        tx = t % stride;
+        ty = t / stride;
+        if (tx >= side || ty >= side)
+            return;
+    }
+    const int x0 = tx * T, y0 = ty * T;
     for (int i = threadIdx.x; i < T * T / 4; i += THREADS)
     {
         reinterpret_cast<uint32_t*>(s_free)[i] = 0u;
@@ -178,7 +202,7 @@ __global__ __launch_bounds__(LIDAR_THREADS) void k_lidar_tiles(dogm_measurement_
         {
             const double dx = dir[b], dy = dir[a.beams + b];
             const double ix = dir[2 * (size_t)a.beams + b], iy = dir[3 * (size_t)a.beams + b];
-            const double r = ranges[(size_t)blockIdx.y * a.beams + b];
+            const double r = ranges[(size_t)grid * a.beams + b];
             const double lim = lidar_limit(r, a.max_range);
             // Distances at which the beam is inside (a direction of 0 gives infinite ones, empty if outside).
             const double xl = xa * ix, xh = xb * ix, yl = ya * iy, yh = yb * iy;
@@ -212,7 +236,7 @@ __global__ __launch_bounds__(LIDAR_THREADS) void k_lidar_tiles(dogm_measurement_
         }
         __syncthreads();
     }
-    dogm_measurement_cell* out = outs[blockIdx.y];
+    dogm_measurement_cell* out = outs[grid];
     for (int i = threadIdx.x; i < T * T; i += THREADS)
     {
         const int x = i % T, y = i / T;
@@ -291,34 +315,25 @@ int lidar_reserve(dogm_lidar* l, int count)
     return DOGM_OK;
 }
 
-// Whether a call takes the tiles.
-//  * The grids exceed the last-level cache (256 MB).  Below, the second write of the three launches finds the cells
-//    there: 4 x 1200 x 1200 cells 75 us against 117 with tiles (a workgroup in the middle clips and walks
-//    every beam, 70 us); above, 20 grids 215 against 192, 32 grids 464 against 260.
-//  * Beams reach 0.4 of a side: with fewer cells to mark, the three launches write little twice (at 0.25, 16 x 1200 x
-//    1200 cells 153 us against 165 with tiles, 32 grids 274 against 241; at 0.5, 177 to 193 against 177 and 461
-//    against 260, 16 x 2048 x 2048 534 against 394, 48 x 600 x 600 255 against 202).
-//  * No two grids overlap (a cell may then get marks of several scans), and the resolution leaves the clipping's
-//    margins far above rounding.
-bool lidar_tiled(const dogm_lidar* l, int count, dogm_measurement_cell* const* outs)
+// The form of a call (lidar_form); the launches also where two grids overlap (a cell may then get marks of several
+// scans) and where the resolution does not leave the tiles' clipping margins far above rounding.
+LidarForm lidar_call_form(const dogm_lidar* l, int count, const double* ranges, dogm_measurement_cell* const* outs)
 {
+    const LidarForm form =
+        lidar_form(l->p.grid_size, l->p.resolution, l->p.max_range, l->p.beam_count, count, ranges);
+    if (form == LIDAR_LAUNCHES || !(l->p.resolution > 1e-100 && l->p.resolution < 1e100))
+        return LIDAR_LAUNCHES;
     const uintptr_t bytes = sizeof(dogm_measurement_cell) * (uintptr_t)l->p.grid_size * (uintptr_t)l->p.grid_size;
-    if (bytes * (uintptr_t)count <= ((uintptr_t)256 << 20))
-        return false;
-    if (!(l->p.max_range >= 0.4 * l->p.grid_size * l->p.resolution))
-        return false;
-    if (!(l->p.resolution > 1e-100 && l->p.resolution < 1e100))
-        return false;
     const std::unique_ptr<uintptr_t[]> at(new (std::nothrow) uintptr_t[count]);
     if (!at)
-        return false;
+        return LIDAR_LAUNCHES;
     for (int i = 0; i < count; ++i)
         at[i] = reinterpret_cast<uintptr_t>(outs[i]);
     std::sort(at.get(), at.get() + count);
     for (int i = 1; i < count; ++i)
         if (at[i] - at[i - 1] < bytes)
-            return false;
-    return true;
+            return LIDAR_LAUNCHES;
+    return form;
 }
 
 }  // namespace
@@ -425,14 +440,13 @@ int dogm_lidar_generate_many(dogm_lidar* l, int count, const double* ranges, dog
                       1.0 / l->step, l->p.occ_mass,
                       l->p.free_mass};
     const int cells = gs * gs;
-    if (lidar_tiled(l, count, device_out))
+    const LidarForm form = lidar_call_form(l, count, ranges, device_out);
+    if (form != LIDAR_LAUNCHES)
     {
-        // Workgroups go to the 8 XCDs in turn.  An odd count along both sides spreads the busy middle tiles of every
-        // row and grid over them; at a multiple of 8 they fall to two (24 x 1024 x 1024 cells 348 us, 219 with the
-        // odd count).
-        const int tx = div_up(gs, LIDAR_TILE) | 1;
-        hipLaunchKernelGGL(k_lidar_tiles, dim3(tx * tx, count), dim3(LIDAR_THREADS), 0, l->stream, l->d_out,
-                           l->d_ranges, l->d_dir, a, tx);
+        const int side = div_up(gs, LIDAR_TILE), centre_first = form == LIDAR_TILES_CENTRE;
+        const int stride = centre_first ? side : side | 1;
+        hipLaunchKernelGGL(k_lidar_tiles, dim3(stride * stride * count), dim3(LIDAR_THREADS), 0, l->stream, l->d_out,
+                           l->d_ranges, l->d_dir, a, side, count, centre_first);
     }
     else
     {

@@ -133,7 +133,8 @@ def test_server_scan_frames_match_plain_handles():
         lid.close()
 
 
-@pytest.mark.parametrize("gs,n_beams", [(1187, 700), (1217, 1100)])
+# Tiles from the centre outwards (one side even, one odd in tiles), and grid after grid.
+@pytest.mark.parametrize("gs,n_beams", [(1187, 700), (1217, 1100), (195, 700), (331, 150), (449, 180)])
 def test_generate_many_beyond_the_cache(gs, n_beams):
     """Calls of more than 256 MB take the tiles (ragged last tiles; more beams than a workgroup's threads): equal to
     grids generated one by one, bit for bit, also for directions and ranges that no scanner gives; two of
