@@ -605,7 +605,6 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         d.x_idx = v->x_idx;
         d.nz = v->nz;
         d.nz_valid = v->nz_valid ? 1 : 0;
-        d.bu = v->bu;
     }
     E->any_wcell = E->any_general = false;
     for (int i = 0; i < m; ++i)
@@ -1175,10 +1174,10 @@ size_t vehicle_footprint(const dogm_params* p)
     const long long part = 16 + 4 + 4 + 1;
     // particles x2 + births, 16 grid fields + free_alt + field_tmp + meas(16) + born + m_raw + pend,
     // weights + ancestors + sort (16 B), CDF (16 B per joint entry), cell factors (16 B) and inputs
-    // (8 B), occupancy bits and birth groups.
+    // (8 B), occupancy bits.
     const long long pad = 8 * (2 * (N & 1) + (B & 1));  // the velocity arrays start 16-byte aligned
     return (size_t)(2 * N * part + B * part + pad + C * 4 * (GF_COUNT + 2 + 2) + C * 16 + C * 12 + N * 8 +
-                    N * 16 + (N + B) * 16 + C * 24 + (C + 63) / 64 * 8 + (C + UNIT - 1) / UNIT * 4);
+                    N * 16 + (N + B) * 16 + C * 24 + (C + 63) / 64 * 8);
 }
 
 int vehicle_alloc(Vehicle* v, const dogm_params* params, uint64_t seed, uint32_t instance, std::string* why)
@@ -1214,8 +1213,7 @@ int vehicle_alloc(Vehicle* v, const dogm_params* params, uint64_t seed, uint32_t
         (st = dalloc(&v->sort_vals[0], N, "sort", why, by)) || (st = dalloc(&v->sort_vals[1], N, "sort", why, by)) ||
         (st = dalloc(&v->cdf, (size_t)N + B, "cdf", why, by)) || (st = dalloc(&v->cellrec, C, "cell factors", why, by)) ||
         (st = dalloc(&v->cellin, C, "cell inputs", why, by)) ||
-        (st = dalloc(&v->nz, ((size_t)C + 63) / 64, "occupancy bits", why, by)) ||
-        (st = dalloc(&v->bu, ((size_t)C + UNIT - 1) / UNIT * (UNIT / WAVE), "birth groups", why, by)))
+        (st = dalloc(&v->nz, ((size_t)C + 63) / 64, "occupancy bits", why, by)))
         return st;
 
     // initGridCellsKernel (init.cu:69-84): start = end = -1, masses 0, measurement (0, 0, 1, 1);
@@ -1262,8 +1260,7 @@ void vehicle_free(Vehicle* v)
                     v->m_raw,    v->pend,         v->ancestors,    v->sort_keys[0], v->sort_keys[1],
                     v->sort_vals[0], v->sort_vals[1], v->cdf,      v->aos_tmp,      v->state_tmp,
                     v->x_occ,    v->x_img,        v->x_mask,       v->x_cnt,        v->x_off,
-                    v->x_idx,    v->x_rec,        v->nz,           v->cellrec,      v->cellin,
-                    v->bu};
+                    v->x_idx,    v->x_rec,        v->nz,           v->cellrec,      v->cellin};
     for (void* b : bufs)
         (void)hipFree(b);
     *v = Vehicle{};

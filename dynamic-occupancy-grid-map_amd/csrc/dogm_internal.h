@@ -193,9 +193,6 @@ struct VehDesc
     // whether they describe the grid in memory (see Vehicle::nz_valid).
     GlobalPtr<unsigned long long> nz;
     int nz_valid;
-    // Per 64 cells: one of them had birth slots at the last full update (so w_A or w_UA may be non-zero);
-    // describes the grid in memory while nz_valid holds.
-    GlobalPtr<uint8_t> bu;
 };
 
 // Scalars produced and consumed on the device within one step, one per vehicle.
@@ -325,7 +322,10 @@ struct Vehicle
     float* weight_array = nullptr;
     float* born = nullptr;
     float* m_raw = nullptr;  // per-cell predicted occupancy before the >1 clamp
-    int* pend = nullptr;     // particle-order ends P_j (birth / initial placement)
+    // Particle-order ends P_j (birth / initial placement in their own stages).  Between full updates its first bytes hold
+    // a mark per 64 cells: one of them had birth slots at the last one (so w_A or w_UA may be non-zero); they
+    // describe the grid in memory while nz_valid holds.
+    int* pend = nullptr;
     int* ancestors = nullptr;
     int* sort_keys[2] = {nullptr, nullptr};
     int* sort_vals[2] = {nullptr, nullptr};
@@ -340,7 +340,6 @@ struct Vehicle
     // those fields (stage-by-stage steps, eager shifts and rotations, grid-cell injection) clears
     // nz_valid, and the next full update rewrites every cell.
     unsigned long long* nz = nullptr;
-    uint8_t* bu = nullptr;  // 64-cell groups with birth slots at the last full update (see VehDesc::bu)
     bool nz_valid = false;
     size_t bytes = 0;                   // device bytes held
 

@@ -1131,6 +1131,19 @@ __device__ __forceinline__ BirthBlock* birth_blocks(const VehDesc& d)
     return reinterpret_cast<BirthBlock*>(d.cdf.get());
 }
 
+// Marks of the 64-cell groups with birth slots (Vehicle::pend), four per unit.
+__device__ __forceinline__ uint8_t* birth_marks(const VehDesc& d)
+{
+    return reinterpret_cast<uint8_t*>(d.pend.get());
+}
+
+// Particle-order ends of a full step whose born masses are out of range: in the cell inputs, which the persistent update
+// has read by then (pend holds the marks).
+__device__ __forceinline__ int* odd_ends(const VehDesc& d)
+{
+    return reinterpret_cast<int*>(d.cellin.get());
+}
+
 // full: the slots' cells as the birth cells of a full step left them; otherwise (a stage-by-stage call, or masses
 // whose prefixes need not be monotone) searched in the particle-order ends.
 __global__ __launch_bounds__(BLOCK) void k_birth_particles(const VehDesc* __restrict__ descs,
@@ -1159,7 +1172,7 @@ __global__ __launch_bounds__(BLOCK) void k_birth_particles(const VehDesc* __rest
     }
     else
     {
-        const int* pend = d.pend;
+        const int* pend = full ? odd_ends(d) : d.pend.get();
         j = wave_slot_cells(pend, d.C, k0, min(k0 + WAVE - 1, B - 1), k, lane);
         if (k >= B)
             return;
@@ -1616,9 +1629,9 @@ __device__ __forceinline__ void birth_cells_unit(const VehDesc* __restrict__ des
     const bool uniform = sc->total == 0;  // equal split over all cells
     const bool odd = sc->born_odd != 0;
     const bool all = uniform || odd || tr.base + UNIT >= C;  // (the last cell takes the remainder)
-    uint8_t* mark = d.bu + w0 / WAVE;
+    uint8_t* mark = birth_marks(d) + w0 / WAVE;
     const uint32_t marks = w0 >= C ? 0u : IT == 1 ? *mark : *reinterpret_cast<const uint32_t*>(mark);
-    const bool had = !d.nz_valid || marks != 0;
+    const bool had = !d.nz_valid || d.init || marks != 0;  // (an initialisation in the step writes its ends over the marks)
     fx_t run = 0;
     int e[IT], s[IT], nu_A[IT];
     float a[IT], u[IT];
@@ -1693,7 +1706,7 @@ __device__ __forceinline__ void birth_cells_unit(const VehDesc* __restrict__ des
     }
     if (odd)
     {
-        store_run<IT>(d.pend.get(), p0, cnt, e);  // the birth particles search
+        store_run<IT>(odd_ends(d), p0, cnt, e);  // the birth particles search
         return;
     }
     if (!births)

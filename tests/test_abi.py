@@ -41,3 +41,14 @@ def test_null_handle_calls_are_rejected():
     assert lib.dogm_update_grid(None, None, 0.0, 0.0, 0.0, 0.1, 0) == 1
     assert lib.dogm_get_grid_size(None) == 0
     assert lib.dogm_last_error(None) == b"null handle"
+
+
+def test_vehicle_footprints():
+    """Budgets given in bytes keep admitting the vehicles they were made for."""
+    for gs, n, b, want in ((1, 1, 0, 238), (17, 1025, 63, 130_733), (250, 300_000, 30_000, 35_987_816),
+                           (1200, 2_000_000, 200_000, 366_940_000), (2048, 8_000_000, 800_000, 1_273_417_984)):
+        p = dogm_ctypes.Params(size=(gs + 0.25) * 0.5, resolution=0.5, particle_count=n, new_born_particle_count=b,
+                               persistence_prob=0.99, stddev_process_noise_position=0.1,
+                               stddev_process_noise_velocity=2.0, birth_prob=0.02, stddev_velocity=30.0,
+                               init_max_velocity=15.0, freespace_discount=0.01)
+        assert dogm_ctypes.vehicle_footprint(p) == want, gs
