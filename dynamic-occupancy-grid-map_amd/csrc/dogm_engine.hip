@@ -605,6 +605,7 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         d.x_idx = v->x_idx;
         d.nz = v->nz;
         d.nz_valid = v->nz_valid ? 1 : 0;
+        d.marks_valid = v->nz_valid && !d.init ? 1 : 0;
     }
     E->any_wcell = E->any_general = false;
     for (int i = 0; i < m; ++i)

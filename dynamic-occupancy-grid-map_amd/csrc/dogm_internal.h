@@ -193,6 +193,7 @@ struct VehDesc
     // whether they describe the grid in memory (see Vehicle::nz_valid).
     GlobalPtr<unsigned long long> nz;
     int nz_valid;
+    int marks_valid;  // nz_valid, and no initialisation in this step writes its particle orders over the birth marks
 };
 
 // Scalars produced and consumed on the device within one step, one per vehicle.

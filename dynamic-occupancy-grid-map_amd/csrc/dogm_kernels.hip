@@ -1631,7 +1631,7 @@ __device__ __forceinline__ void birth_cells_unit(const VehDesc* __restrict__ des
     const bool all = uniform || odd || tr.base + UNIT >= C;  // (the last cell takes the remainder)
     uint8_t* mark = birth_marks(d) + w0 / WAVE;
     const uint32_t marks = w0 >= C ? 0u : IT == 1 ? *mark : *reinterpret_cast<const uint32_t*>(mark);
-    const bool had = !d.nz_valid || d.init || marks != 0;  // (an initialisation in the step writes its ends over the marks)
+    const bool had = !d.marks_valid || marks != 0;
     fx_t run = 0;
     int e[IT], s[IT], nu_A[IT];
     float a[IT], u[IT];

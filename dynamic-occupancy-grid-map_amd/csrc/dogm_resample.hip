@@ -837,11 +837,6 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     const int t0 = d.u0[SP_J] / SCAN_Q;
     const SegEnds seg_end{seg_local + (size_t)t0 * CDF_SEGS_PER_TILE, cdf_pre + t0, sc->cdf_total,
                           (J + SCAN_TILE - 1) / SCAN_TILE, (J + CDF_SEG - 1) / CDF_SEG};
-    if (sc->beyond_keys)
-    {
-        merge_beyond_keys(d, sc, seg_end, pph, base, n, J, exp_tile_pre, beyond_segs, s_mem);
-        return;
-    }
     const int cnt_draws = min(RS_TILE, n - base);
     const int wid = threadIdx.x / WAVE;
     const int lane = threadIdx.x & (WAVE - 1);
@@ -862,6 +857,11 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
                          [&](int i, fx_t s_k) { s_r[threadIdx.x * RS_ITEMS + i] = raw_draw(s_k); });
     }
     __syncthreads();
+    if (sc->beyond_keys)
+    {
+        merge_beyond_keys(d, sc, seg_end, pph, base, n, J, exp_tile_pre, beyond_segs, s_mem);
+        return;
+    }
     // Item i of a thread is draw base + threadIdx.x + i * BLOCK, so at every item a wave searches 64 consecutive draws,
     // whose probes read neighbouring keys, and the ancestors come out wave-contiguous.
     int anc[RS_ITEMS];
