@@ -543,7 +543,8 @@ int engine_plan(Engine* E, Vehicle* const* veh, int m, int stages)
         d.init = (stages & ST_INIT) && v->init_pending ? 1 : 0;
         d.wuni = v->w_uniform || d.init ? 1 : 0;  // initialisation sets every weight to 1 / N
         // In a full update from uniform weights every in-grid particle carries the same predicted weight
-        // and every other one 0, so the per-cell sums need counts only.
+        // and every other one 0, so the per-cell sums need counts only.  Weights differ only after stage calls or
+        // writes of a single handle: steps of several vehicles have per-cell weights throughout.
         d.wcell = d.wuni && (stages & ST_ALL) == ST_ALL ? 1 : 0;
         d.rs_gather = v->rs_pending && !d.init && full_predict ? 1 : 0;
         d.ep_init = e;

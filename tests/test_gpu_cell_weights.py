@@ -124,8 +124,9 @@ def test_single_stages_after_full_updates(gs, n):
             np.testing.assert_array_equal(a, c)
 
 
-def test_batch_mixes_both_paths():
-    """A vehicle whose weights are not uniform beside one whose weights are, in the same launches."""
+def test_batch_with_a_late_vehicle():
+    """A vehicle that initialises its particles beside vehicles that read resampled sets, in the same launches.  Batches
+    run full updates only and nothing writes their weights, so every vehicle of a batched step has per-cell weights."""
     ps = [small_params(gs=g, res=0.5, n=n, b=n // 10) for g, n in ((40, 9000), (24, 5000), (64, 20000))]
     rng = np.random.default_rng(5)
     with Batch() as batch:
