@@ -967,9 +967,9 @@ constexpr int TOP_BLOCK = 1024;
 template <int Unused = 0>
 __global__ __launch_bounds__(TOP_BLOCK) void k_scan_top(const VehDesc* __restrict__ descs,
                                                         const fx_t* __restrict__ tile_sum, fx_t* __restrict__ tile_pre,
-                                                        DevScalars* __restrict__ scs, int mode, int only, int parts)
+                                                        DevScalars* __restrict__ scs, int mode, int only)
 {
-    scan_top_orders<TOP_BLOCK>(descs, blockIdx.x, tile_sum, tile_pre, scs, mode, only, parts);
+    scan_top_orders<TOP_BLOCK>(descs, blockIdx.x, tile_sum, tile_pre, scs, mode, only, 1);
 }
 
 // Sink interface:
@@ -1023,27 +1023,20 @@ __global__ __launch_bounds__(BLOCK) void k_scan_apply(Src src, Sink sink, const 
     scan_apply_body(src, sink, descs, tab, blockIdx.x, tile_pre, scs);
 }
 
-// Exact scan over the cells: tile totals, their prefixes and the order scale, the sink.  unit_sums: the sources' exact
-// sums per 256-cell unit were left there by an earlier kernel of the step (SCAN_Q per tile), so the tile
-// pass is skipped.
+// Exact scan over the cells: tile totals, their prefixes and the order scale, the sink.
 template <class Src, class Sink>
-inline void run_exact_scan(Engine* E, const Src& src, const Sink& sink, int mode, int kid_apply, int only,
-                           const fx_t* unit_sums = nullptr)
+inline void run_exact_scan(Engine* E, const Src& src, const Sink& sink, int mode, int kid_apply, int only)
 {
     const int tiles = E->tiles(SP_C, SCAN_Q);
     if (tiles <= 0)
         return;
-    if (!unit_sums)
-    {
-        launch_begin(E, K_SCAN_TILES);
-        hipLaunchKernelGGL(k_scan_tiles<Src>, dim3(tiles), dim3(BLOCK), 0, E->stream, src, E->d_desc, E->tab(SP_C),
-                           E->scan_tile_sum, (fx_t*)nullptr);
-        launch_end(E, K_SCAN_TILES);
-    }
+    launch_begin(E, K_SCAN_TILES);
+    hipLaunchKernelGGL(k_scan_tiles<Src>, dim3(tiles), dim3(BLOCK), 0, E->stream, src, E->d_desc, E->tab(SP_C),
+                       E->scan_tile_sum, (fx_t*)nullptr);
+    launch_end(E, K_SCAN_TILES);
     launch_begin(E, K_SCAN_TOP);
-    hipLaunchKernelGGL(k_scan_top<0>, dim3(E->m), dim3(TOP_BLOCK), 0, E->stream, E->d_desc,
-                       unit_sums ? unit_sums : E->scan_tile_sum, E->scan_tile_pre, E->scalars, mode, only,
-                       unit_sums ? SCAN_Q : 1);
+    hipLaunchKernelGGL(k_scan_top<0>, dim3(E->m), dim3(TOP_BLOCK), 0, E->stream, E->d_desc, E->scan_tile_sum,
+                       E->scan_tile_pre, E->scalars, mode, only);
     launch_end(E, K_SCAN_TOP);
     launch_begin(E, kid_apply);
     hipLaunchKernelGGL((k_scan_apply<Src, Sink>), dim3(tiles), dim3(BLOCK), 0, E->stream, src, sink, E->d_desc,

@@ -775,7 +775,7 @@ int engine_run(Engine* E, Vehicle* const* veh, int m, int stages)
         if (stages & ST_BIRTH)
         {
             StageRange r("initializeNewParticles");
-            run_births(E, occ_birth, moments_first, pph);
+            run_births(E, moments_first, pph);
         }
         if ((stages & ST_MOMENTS) && !moments_first)
         {

@@ -639,7 +639,7 @@ void run_occupancy(Engine* E, int pph, int zero_empty, bool defer_normalize, boo
 void run_persistent(Engine* E, int pph, bool fused_normalize, bool empty_done, bool defer_post);
 // moments_first (full steps, after run_moments with births_top): the birth orders' top-level scan has run, and
 // the launch of the birth cells also sums the moments of cells crossing chunks.
-void run_births(Engine* E, bool born_sums, bool moments_first, int pph);
+void run_births(Engine* E, bool moments_first, int pph);
 // Unit sums of the born masses between the occupancy update and the births of a step: the CDF index
 // buffer (SCAN_Q units per scan tile fit its CDF_SEGS_PER_TILE entries per tile), unused until the
 // resampling.

@@ -205,24 +205,6 @@ __device__ __forceinline__ int clamp_cell(float x, int gs)
     return (int)fminf(fmaxf(x, 0.0f), (float)(gs - 1));  // NaN gives cell 0
 }
 
-// A workgroup covers one sort tile: PB threads of SORT_TILE / PB particles each (strided by PB).
-// 512 x 4 (the built-in choice) gives a single 2e6-particle grid about 8 waves per SIMD to hide the
-// Philox / Box-Muller latency; 256 x 8 is the other choice of the tuning.  Bound by memory where many vehicles
-// share a launch (41 bytes a particle; 16 x 2e6: 329 us) and by latency below: with the item loop loading ahead,
-// without its digit counts' global atomics and with the shorter quotient and root, 2e6 particles went from 35.5 to
-// 23.8 us and 3e5 from 13.6 to 9.6; the item loop stays rolled (unrolled: 23.5 and 11.0).
-//
-// With passes > 0 the workgroup also counts the radix digits of the new cell indices (of every sort pass for the
-// onesweep form, of the first for reduce-then-scan: `passes`).  Without thist the counts go to
-// ghist[(vehicle * 4 + pass) * 256 + digit] (onesweep's one-time histogram; the sort passes' tile tickets are
-// cleared too); with
-// thist set (reduce-then-scan sort) it stores the first pass's digit counts of its tile as
-// thist[digit * tiles + tile]: a workgroup covers exactly one sort tile, so the sort skips that
-// upsweep.  With aos (the sort's gathering pass follows in the same step) the new state goes to the
-// vehicle's CDF buffer, free until the resampling, as 16-byte (x, y, vx, vy) records, so that the
-// gather reads one 16-byte record per particle at random instead of two 8-byte ones from two arrays;
-// nothing else reads the positions or velocities in between.  The cell indices then carry the particles'
-// flags (WORD_FLAGS), so the sort's first pass reads one word per particle and no association byte.
 // Border cells: the cells whose coordinate predict clamps to, so the only ones that can hold out-of-grid
 // particles (weight 0) beside in-grid ones.  For vehicles with per-cell weights their out-of-grid particles
 // are counted in the born masses (as ints), which the occupancy update rewrites cell by cell after it has read
@@ -276,6 +258,24 @@ __device__ __forceinline__ void reset_bounds_cells(const VehDesc* __restrict__ d
     }
 }
 
+// A workgroup covers one sort tile: PB threads of SORT_TILE / PB particles each (strided by PB).
+// 512 x 4 (the built-in choice) gives a single 2e6-particle grid about 8 waves per SIMD to hide the
+// Philox / Box-Muller latency; 256 x 8 is the other choice of the tuning.  Bound by memory where many vehicles
+// share a launch (41 bytes a particle; 16 x 2e6: 329 us) and by latency below: with the item loop loading ahead,
+// without its digit counts' global atomics and with the shorter quotient and root, 2e6 particles went from 35.5 to
+// 23.8 us and 3e5 from 13.6 to 9.6; the item loop stays rolled (unrolled: 23.5 and 11.0).
+//
+// With passes > 0 the workgroup also counts the radix digits of the new cell indices (of every sort pass for the
+// onesweep form, of the first for reduce-then-scan: `passes`).  Without thist the counts go to
+// ghist[(vehicle * 4 + pass) * 256 + digit] (onesweep's one-time histogram; the sort passes' tile tickets are
+// cleared too); with
+// thist set (reduce-then-scan sort) it stores the first pass's digit counts of its tile as
+// thist[digit * tiles + tile]: a workgroup covers exactly one sort tile, so the sort skips that
+// upsweep.  With aos (the sort's gathering pass follows in the same step) the new state goes to the
+// vehicle's CDF buffer, free until the resampling, as 16-byte (x, y, vx, vy) records, so that the
+// gather reads one 16-byte record per particle at random instead of two 8-byte ones from two arrays;
+// nothing else reads the positions or velocities in between.  The cell indices then carry the particles'
+// flags (WORD_FLAGS), so the sort's first pass reads one word per particle and no association byte.
 template <int PRED_BLOCK>
 __global__ __launch_bounds__(PRED_BLOCK) void k_predict(const VehDesc* __restrict__ descs, const uint32_t* __restrict__ tab,
                                                    int pph, int passes, unsigned* __restrict__ ghist,
@@ -1592,10 +1592,13 @@ void run_moments(Engine* E, int pph, bool fused_post, bool empty_done, bool birt
 // left births.  The others hand their slots to the birth particles (BirthBlock), which then need no search over
 // the particle-order ends, and those are not stored.
 // Bound by the dependent chain of the few units with births (exact scan, roundings, the association
-// probability, divisions, slots): IT = 1 spreads it over four times the waves, which wins while the step leaves
-// the GPU idle (250 x 250 cells: 5.7 us against 10.4), IT = 4 has a quarter of the waves, which wins on large
-// grids and batches (BIRTH_WIDE_UNITS; 32 x 1200 x 1200 cells: 1.6% of the whole step).  The birth particles
-// went from 10.9 to 5.1 us at 2e5 slots.
+// probability, divisions, slots): IT = 1 spreads it over four times the waves, which wins while the launch leaves
+// the GPU idle, IT = 4 has a quarter of the waves, which wins on large grids and batches.  Measured IT = 1 / IT = 4 in
+// us by cell units of the launch: 245 (250 x 250) 8.5 / 10.6, 1024 (16 x 128 x 128) 9.9 / 11.9, 1407 (600 x 600) 9.6 /
+// 11.2, 2823 (850 x 850) 11.5 / 12.0, 3907 (1000 x 1000) 12.9 / 12.3, 5000 (8 x 400 x 400) 18.6 / 16.1, 5625 (1200 x
+// 1200) 14.7 / 12.8, 16384 (2048 x 2048) 33.1 / 27.7, 32768 (32 x 512 x 512) 79.6 / 47.0.  The line lies a little above
+// where they meet (about 3000 units, 1% of the step between).  The birth particles went from 10.9 to 5.1 us at 2e5
+// slots.
 constexpr int BIRTH_WIDE_UNITS = 4096;
 
 template <int IT>
@@ -1757,7 +1760,7 @@ __global__ __launch_bounds__(BLOCK) void k_birth_cells(const VehDesc* __restrict
         moments_fix_chunk(descs, tab_p, (group - cell_groups) * BLOCK + (int)threadIdx.x, units, pph, carry);
 }
 
-void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
+void run_births(Engine* E, bool moments_first, int pph)
 {
     // With B = 0 the cell pass still runs (every cell gets n_j = 0 and w_A = w_UA = 0) and the
     // stage still consumes its RNG epoch, so the stream of later stages does not depend on B.
@@ -1779,8 +1782,7 @@ void run_births(Engine* E, bool born_sums, bool moments_first, int pph)
     }
     else
     {
-        run_exact_scan(E, SrcBorn{0}, SinkBirth{}, SCAN_ORDERS_B, K_BIRTH_CELLS, ONLY_ALL,
-                       born_sums ? born_unit_sums(E) : nullptr);
+        run_exact_scan(E, SrcBorn{0}, SinkBirth{}, SCAN_ORDERS_B, K_BIRTH_CELLS, ONLY_ALL);
     }
     const int blocks = E->tiles(SP_B, 1);
     if (blocks <= 0)

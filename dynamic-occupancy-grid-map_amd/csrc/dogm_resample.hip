@@ -793,10 +793,10 @@ __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevSca
 // key(x) = floor((x - B0) 2^(30 - m)) with B0 the CDF before the window, W its exact total and m = msb(W), and
 // the draws are compared by the same key.
 //   - Weights, draws and their differences from B0 are formed in f64 in raw units (integers).  The rebuild's sums (a
-//     wave scan of one segment from its exact index entry) are off by less than 2^-48 W, a draw's
-//     difference by less than that (B0 is subtracted in two doubles), so both keys are within 1 of the exact ones
-//     and two keys at least 2 apart decide.  With W below 2^31 every value is an integer below 2^31 and the
-//     keys are exact.
+//     wave scan of one segment from its exact index entry) are off by less than 2^-48 W.  B0 is subtracted in two
+//     doubles, which hold it to 2^(msb(B0) - 106): at the smallest W that keys are used for (below) a draw's
+//     difference is off by up to 2^-40 W, 2^-10 of a key.  Both keys are thus within 1 of the exact ones and two
+//     keys at least 2 apart decide.  With W below 2^31 every value is an integer below 2^31 and the keys are exact.
 //   - A draw within 1 of an entry's key (about 3e-6 of them: a window holds at most 2048 of 2^30 keys, and draws
 //     fall in proportion to the CDF) is resolved by wave_exact_ancestor.
 //   - A window whose total is below 2^-66 of a CDF above 2^107 raw units before it sends the draws that land in it
