@@ -548,6 +548,12 @@ __device__ __forceinline__ double fx_raw_f64(fx_t v)
     return fx_to_f64(v) * 0x1p88;
 }
 
+// A draw in raw units (an integer) as a fixed-point value.
+__device__ __forceinline__ fx_t raw_fx(double raw)
+{
+    return fx_from_f64_nonneg(raw * 0x1p-88);
+}
+
 // Four joint weights in raw fixed-point units: fx_from_f32_nonneg as doubles (a 24-bit significand truncated to an
 // integer), for weights below 2^39.
 __device__ __forceinline__ void raw_weights(const float (&f)[SCAN_ITEMS], double (&v)[SCAN_ITEMS])
@@ -622,58 +628,36 @@ __device__ __forceinline__ int wave_exact_ancestor(const VehDesc& d, const SegEn
 // draw is resolved in the first window whose last entry is >= its value, by a branch-free binary search over
 // the window padded to a power of two.  While the CDF is non-decreasing that is its lower bound.  Past the
 // fixed-point range the sums wrap and the answer depends on the probes, so their order is fixed: the whole coarse
-// index first, windows of a given length, halved from the front.
+// index first, windows of a given length, halved from the front.  s_mem holds the workgroup's draws on entry.
 // 2.2e5 joint weights, one of them infinite: 12.4 us (one by one, with wave_exact_ancestor, 457).
 __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevScalars* sc, const SegEnds& seg_end,
-                                                  int pph, int base, int n, int J,
-                                                  const fx_t* __restrict__ exp_tile_pre, int segs, uint64_t* s_mem)
+                                                  int pph, int base, int n, int J, int segs, uint64_t* s_mem)
 {
     constexpr int NWAVE = BLOCK / WAVE;
     constexpr int HALF = NWAVE * CDF_SEG;  // entries staged at once, a segment per wave
-    static_assert(HALF == RS_TILE, "the entries' bytes also stage the draws");
-    __shared__ fx_t s_rb[2], s_wr[NWAVE];
+    static_assert(HALF == RS_TILE, "the entries take the draws' bytes and as many again");
+    __shared__ fx_t s_wr[NWAVE];
     __shared__ int s_wmin[NWAVE];
     int64_t* s_hi64 = reinterpret_cast<int64_t*>(s_mem);
     uint64_t* s_lo64 = s_mem + HALF;
+    const double* s_r = reinterpret_cast<const double*>(s_mem);
     const int lane = threadIdx.x & (WAVE - 1), wid = wave_index();
     const auto put = [=](int i, fx_t x) {
         s_hi64[i] = (int64_t)(x >> 64);
         s_lo64[i] = (uint64_t)x;
     };
     const auto get = [=](int i) { return (fx_t)(((ufx_t)(uint64_t)s_hi64[i] << 64) | (ufx_t)s_lo64[i]); };
-    const Spacing sp = sc->spacing;
-    fx_t r[RS_ITEMS];
-    if (d.draw_mode == DRAW_SYSTEMATIC)
-    {
-        const uint32_t u = systematic_u32(d.seed, d.inst, d.ep_rs);
-#pragma unroll
-        for (int i = 0; i < RS_ITEMS; ++i)
-            r[i] = spacing_draw_nonneg(systematic_s(base + (int)threadIdx.x + i * BLOCK, u), sp);
-    }
-    else
-    {
-        spacing_prefixes(d, base, n, exp_tile_pre,
-                         [&](int i, fx_t s_k) { put(threadIdx.x * RS_ITEMS + i, spacing_draw_nonneg(s_k, sp)); });
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < RS_ITEMS; ++i)
-            r[i] = get(threadIdx.x + i * BLOCK);
-    }
     const int last = min(base + RS_TILE, n) - 1;
+    double r[RS_ITEMS];
     int anc[RS_ITEMS];
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
     {
-        const int k = base + (int)threadIdx.x + i * BLOCK;
+        r[i] = s_r[threadIdx.x + i * BLOCK];
         anc[i] = -1;
-        if (k == base)
-            s_rb[0] = r[i];
-        if (k == last)
-            s_rb[1] = r[i];
     }
-    __syncthreads();
     int s_lo, s_hi;
-    wave_find2<fx_t>(seg_end, seg_end.segs, s_rb[0], s_rb[1], &s_lo, &s_hi);
+    wave_find2<fx_t>(seg_end, seg_end.segs, raw_fx(s_r[0]), raw_fx(s_r[last - base]), &s_lo, &s_hi);
     for (int s0 = s_lo; s0 <= s_hi;)
     {
         const int s1 = min(s0 + segs, s_hi + 1);  // window: segments [s0, s1)
@@ -683,53 +667,40 @@ __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevSca
         const bool two = clen > HALF;
         const fx_t mid = two ? seg_end(s0 + NWAVE - 1) : (fx_t)0;  // entry HALF - 1: the first probe
         const int span = clen > 1 ? 1 << (32 - __clz(clen - 1)) : 1;
-        // The weights and prefixes of both halves are in flight together.
-        float f[2][SCAN_ITEMS];
-        fx_t before[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
+#pragma unroll 1
+        for (int h = 0; h <= (two ? 1 : 0); ++h)
         {
             const int s = s0 + h * NWAVE + wid;
             const int q0 = s * CDF_SEG + lane * SCAN_ITEMS;
-#pragma unroll
-            for (int i = 0; i < SCAN_ITEMS; ++i)
-                f[h][i] = 0.0f;
+            float f[SCAN_ITEMS] = {0.0f, 0.0f, 0.0f, 0.0f};
             if (s < s1 && q0 < J)
-                SrcJointPos{nullptr}.load4(d, q0, min(SCAN_ITEMS, J - q0), f[h]);
-            before[h] = s < s1 && s > 0 ? seg_end(s - 1) : (fx_t)0;
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-        {
-            if (h == 1 && !two)
-                break;
-            __syncthreads();  // the searches (and the draws' staging) before are done
-            fx_t v[SCAN_ITEMS];
+                SrcJointPos{nullptr}.load4(d, q0, min(SCAN_ITEMS, J - q0), f);
             fx_t sum = 0;
 #pragma unroll
             for (int i = 0; i < SCAN_ITEMS; ++i)
-            {
-                v[i] = fx_from_f32_nonneg(f[h][i]);  // cdf_weight: sign bit clear; 0 past the entries
-                sum += v[i];
-            }
-            fx_t run = wave_inclusive_scan_fx(sum) - sum + before[h];
+                sum += fx_from_f32_nonneg(f[i]);  // cdf_weight: sign bit clear; 0 past the entries
+            fx_t run = wave_inclusive_scan_fx(sum) - sum + (s < s1 && s > 0 ? seg_end(s - 1) : (fx_t)0);
+            __syncthreads();  // the searches (and the draws' staging) before are done
 #pragma unroll
             for (int i = 0; i < SCAN_ITEMS; ++i)
             {
-                run += v[i];
+                run += fx_from_f32_nonneg(f[i]);
                 put(wid * CDF_SEG + lane * SCAN_ITEMS + i, run);
             }
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < RS_ITEMS; ++i)
             {
-                const bool upper = two && mid < r[i];
-                if (anc[i] >= 0 || base + (int)threadIdx.x + i * BLOCK > last || cmax < r[i] || upper != (h != 0))
+                double raw = r[i];
+                asm volatile("" : "+v"(raw));  // converted here and not once for all windows: four registers a draw less
+                const fx_t ri = raw_fx(raw);
+                const bool upper = two && mid < ri;
+                if (anc[i] >= 0 || base + (int)threadIdx.x + i * BLOCK > last || cmax < ri || upper != (h != 0))
                     continue;
                 // lo counts the entries below the draw; past the window the last entry stands for the ones missing.
                 int lo = h * HALF;
                 for (int step = two ? HALF / 2 : span >> 1; step > 0; step >>= 1)
-                    if (get(min(lo + step, clen) - 1 - h * HALF) < r[i])
+                    if (get(min(lo + step, clen) - 1 - h * HALF) < ri)
                         lo += step;
                 anc[i] = c0 + lo;
             }
@@ -739,7 +710,7 @@ __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevSca
         // The smallest unresolved draw: each wave's minimum (draw indices are distinct, so one lane holds it) with its
         // value, then the minimum over the waves.
         int mine = n;
-        fx_t rmine = 0;
+        double rmine = 0.0;
 #pragma unroll
         for (int i = RS_ITEMS - 1; i >= 0; --i)
         {
@@ -755,7 +726,7 @@ __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevSca
         for (int o = WAVE / 2; o > 0; o >>= 1)
             wmin = min(wmin, __shfl_xor(wmin, o, WAVE));
         if (wmin < n && mine == wmin)
-            s_wr[wid] = rmine;
+            s_wr[wid] = raw_fx(rmine);
         if (lane == 0)
             s_wmin[wid] = wmin;
         __syncthreads();
@@ -807,8 +778,10 @@ __device__ __forceinline__ void merge_beyond_keys(const VehDesc& d, const DevSca
 // Bound by the vector ALU (Philox and logarithms of the draws, searches).  Before, windows held 128-bit
 // entries (four 128-bit conversions and adds per lane and segment, 128-bit scans and two-word probes).
 // 2e6 draws: 31.9 -> 22.1 us alone (3e5: 19.1 -> 15.2), 32 x 2e6 per step 3.4% off the whole step.
+// Eight waves per SIMD are asked for: 64 vector and 78 scalar registers without memory spills; left to itself the
+// compiler takes 99 scalar ones, and 16 x 2e6 draws 244 us instead of 221.
 template <int WSEG>
-__global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restrict__ descs,
+__global__ __launch_bounds__(BLOCK, 8) void k_rs_merge_exact(const VehDesc* __restrict__ descs,
                                                           const uint32_t* __restrict__ tab, int pph,
                                                           const fx_t* __restrict__ exp_tile_pre,
                                                           const fx_t* __restrict__ seg_local,
@@ -843,7 +816,6 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     const Spacing sp = sc->spacing;
     // fx(total * u_k) as a double: the product truncated to an integer number of raw units.
     const auto raw_draw = [&sp](fx_t s_k) { return trunc(sp.total * spacing_fraction(s_k, sp) * 0x1p88); };
-    const auto draw_fx = [](double raw) { return fx_from_f64_nonneg(raw * 0x1p-88); };
     if (d.draw_mode == DRAW_SYSTEMATIC)
     {
         const uint32_t u = systematic_u32(d.seed, d.inst, d.ep_rs);
@@ -859,7 +831,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     __syncthreads();
     if (sc->beyond_keys)
     {
-        merge_beyond_keys(d, sc, seg_end, pph, base, n, J, exp_tile_pre, beyond_segs, s_mem);
+        merge_beyond_keys(d, sc, seg_end, pph, base, n, J, beyond_segs, s_mem);
         return;
     }
     // Item i of a thread is draw base + threadIdx.x + i * BLOCK, so at every item a wave searches 64 consecutive draws,
@@ -869,7 +841,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
     for (int i = 0; i < RS_ITEMS; ++i)
         anc[i] = threadIdx.x + i * BLOCK < cnt_draws ? -1 : 0;
     int s_lo, s_hi;
-    seg_end.find2(draw_fx(s_r[0]), draw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
+    seg_end.find2(raw_fx(s_r[0]), raw_fx(s_r[cnt_draws - 1]), &s_lo, &s_hi);
     for (int s0 = s_lo;;)
     {
         const int s1 = min(s0 + WSEG, s_hi + 1);  // window: segments [s0, s1)
@@ -884,7 +856,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
         const double g = ldexp(1.0, 30 - m);
         const uint32_t margin = m <= 30 ? 0u : 1u;
         const double b_hi = exact ? 0.0 : fx_raw_f64(B0);
-        const double b_lo = exact ? 0.0 : fx_raw_f64(B0 - draw_fx(b_hi));
+        const double b_lo = exact ? 0.0 : fx_raw_f64(B0 - raw_fx(b_hi));
 #pragma unroll
         for (int q = 0; q < WSEG / NWAVE; ++q)
         {
@@ -957,7 +929,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             {
                 const int l = __builtin_ctzll(todo);
                 todo &= todo - 1;
-                const int a = wave_exact_ancestor(d, seg_end, J, draw_fx(s_r[wid * WAVE + l + i * BLOCK]));
+                const int a = wave_exact_ancestor(d, seg_end, J, raw_fx(s_r[wid * WAVE + l + i * BLOCK]));
                 if (lane == l)
                     anc[i] = a;
             }
@@ -977,7 +949,7 @@ __global__ __launch_bounds__(BLOCK) void k_rs_merge_exact(const VehDesc* __restr
             done += s_done[w];
         if (done >= cnt_draws)
             break;
-        const fx_t rmin = draw_fx(s_r[done]);
+        const fx_t rmin = raw_fx(s_r[done]);
         const int next_last = min(s1 - 1 + WSEG, s_hi);
         if (!(seg_end(next_last) < rmin))
         {
@@ -1118,7 +1090,7 @@ __global__ __launch_bounds__(TOP_BLOCK) void k_scan_top_resample(const VehDesc* 
     __shared__ int s_beyond;
     const VehDesc& d = descs[blockIdx.x];
     if (threadIdx.x == 0)
-        s_beyond = 0;
+        s_beyond = scs[blockIdx.x].beyond_tiles;  // beside the loads of the totals, not behind the scan
     const int half = threadIdx.x / HALF, tid = threadIdx.x % HALF;
     const int nj = d.cdf_mode == CDF_EXACT ? d.nu[SP_J] / SCAN_Q : 0;
     const int ne = d.draw_mode == DRAW_MULTINOMIAL ? d.nu[SP_E] / SCAN_Q : 0;
@@ -1140,7 +1112,7 @@ __global__ __launch_bounds__(TOP_BLOCK) void k_scan_top_resample(const VehDesc* 
         // Systematic draws do not use the exponentials: S_N = N * 2^32 (dogm_numerics.h).
         sc->spacing = spacing_setup(ne ? s_total[1] : systematic_s(d.N, 0u), cdf_total);
         sc->cdf_total = cdf_total;
-        sc->beyond_keys = sc->beyond_tiles | s_beyond;
+        sc->beyond_keys = s_beyond;
         sc->beyond_tiles = 0;
         if (nj)
         {
